@@ -7,11 +7,10 @@
 // MPO (DL,DR,d,d)) are read and written in place: no transposes or reshapes are
 // materialised between the legs of a contraction.
 //
-// Kernel structure: a workgroup owns a BM x BN tile of C and loops over K in
-// steps of BK. Tiles of A and B go global -> registers -> LDS (double buffered,
-// one barrier per K step); the next tile's global loads are in flight while the
-// waves run MFMA on the current one. Each wave owns a (BM/WM) x (BN/WN) sub-tile
-// built from 16x16 blocks:
+// The GEMMs of the contractions run in the pipelined kernels of gemm_pipe.hpp. The kernel here stages tiles through
+// registers (global -> registers -> LDS, double buffered, one barrier per K step; per-element 64-bit offsets where the
+// index maps are not separable). It serves outputs of at most 16 rows, the grouped launches, the block Jacobi steps and
+// the index maps that the pipelined kernels do not take. Each wave owns a (BM/WM) x (BN/WN) sub-tile of 16x16 blocks:
 //   FP64: v_mfma_f64_16x16x4_f64,  FP32: v_mfma_f32_16x16x4_f32.
 // Complex products use the 3-real-product (Gauss) form, 3 MFMAs per block per k-step:
 //   P1 = sum ar br, P2 = sum ai bi, P3 = sum (ar + ai)(br + bi);  re = P1 - P2, im = P3 - P1 - P2.
@@ -20,6 +19,7 @@
 // of the accumulator runs along M; it is picked when C is unit-stride in M, so
 // the epilogue stores are coalesced either way.
 #include "common.hpp"
+#include "gemm_plan.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -563,26 +563,77 @@ struct LaunchPlan {
     int     ksplit2 = 1;
 };
 
-static LaunchPlan heuristic_plan(const GemmDesc &g) {
-    const int64_t cus  = device_cu_count();
-    auto          nblk = [&](int bm, int bn) { return static_cast<int64_t>((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) * g.batch; };
-    LaunchPlan    p{TileCfg::T64x64, 1};
-    if(g.M <= 16) p.cfg = TileCfg::T16x128;
-    else if(g.M >= 48 && g.N >= 48) p.cfg = TileCfg::T64x64;
-    else p.cfg = g.M < g.N ? TileCfg::T32x64 : TileCfg::T64x32;
-    // Fewer 64x64 tiles than CUs: 32x32 tiles, four times as many.
-    if(p.cfg == TileCfg::T64x64 && nblk(64, 64) < cus) p.cfg = TileCfg::T32x32;
-    const CfgShape sh    = cfg_shape(p.cfg);
-    const int64_t  tiles = nblk(sh.BM, sh.BN);
-    // Small grids with a long K: slice K (slices of at least 128) so that about two workgroups per CU are in
-    // flight. These are the plans the tuner picks for the chi <= 256 matvec legs.
-    if(tiles < 2 * cus && g.K >= 256 && p.cfg != TileCfg::T16x128) {
-        int64_t ks = std::min<int64_t>({(2 * cus + tiles - 1) / tiles, g.K / 128, 8});
-        if(g.part && ks > 1) ks = std::min<int64_t>(ks, g.part_capacity / (static_cast<int64_t>(g.M) * g.N * g.batch));
-        else ks = 1;
-        p.ksplit = static_cast<int>(std::max<int64_t>(1, ks));
+// The orientation in which consecutive m are (if anything is) consecutive in C: the pipelined kernel's lanes run along M.
+static int      fast_score(const Idx2 &x) { return x.s0 == 1 ? static_cast<int>(std::min<uint32_t>(x.c, 1u << 20)) : 0; }
+static GemmDesc oriented(const GemmDesc &g) {
+    if(fast_score(g.cn) <= fast_score(g.cm)) return g;
+    GemmDesc t = g;
+    std::swap(t.A, t.B);
+    std::swap(t.am, t.bn);
+    std::swap(t.ak, t.bk);
+    std::swap(t.a_batch, t.b_batch);
+    std::swap(t.conjA, t.conjB);
+    std::swap(t.M, t.N);
+    std::swap(t.cm, t.cn);
+    return t;
+}
+
+// The pipelined shape that a tile configuration stands for, or N_SHAPES.
+static pipe::Shape shape_of(TileCfg c, dmrg_dtype t) {
+    pipe::Shape s = pipe::N_SHAPES;
+    switch(c) {
+        case TileCfg::T128x64: s = pipe::S128x64; break;
+        case TileCfg::T64x64: s = pipe::S64x64; break;
+        case TileCfg::T32x64:
+        case TileCfg::T64x32: s = pipe::S64x32; break;
+        case TileCfg::T32x32:
+        case TileCfg::T32x32K: s = pipe::S32x32; break;
+        default: return s;
     }
-    return p;
+    while(pipe::shape_info(t, s).BM == 0) s = static_cast<pipe::Shape>(s + 1); // the next smaller shape of the type
+    return s;
+}
+
+// Microseconds that the pipelined kernel takes for g in shape s with ks K slices: a CU's workgroups share its matrix
+// cores, so r of them advance one stage in r stage times of MFMA work, but none of them faster than its own chain of
+// barrier, LDS read and MFMA (about 170 clocks beyond its MFMAs). Within 15 % of the measured times of the matvec legs
+// of chi 24 to 1024 (e.g. FP64 402x165x825: 32x32 tiles 15.7 us, 3 slices 12.5, against 14.6 and 11.9 here).
+static double pipe_cost_us(const GemmDesc &g, pipe::Shape s, int ks) {
+    const pipe::ShapeInfo i = pipe::shape_info(g.dtype, s);
+    const bool   cplx = dtype_is_complex(g.dtype), sp = dtype_is_single(g.dtype);
+    const double clk = 2300.0, cus = device_cu_count();
+    const double stages = std::ceil((g.K + i.BK - 1) / i.BK / static_cast<double>(ks));
+    const double mfma   = i.TM * i.TN * (i.BK / 4) * (cplx ? 3 : 1) * (sp ? 32.0 : 64.0);
+    const double tiles  = static_cast<double>((g.M + i.BM - 1) / i.BM) * ((g.N + i.BN - 1) / i.BN) * g.batch * ks;
+    auto         round  = [&](double r) { return stages * std::max(r * mfma * 1.04, mfma + 170.0); };
+    const double per_cu = std::ceil(tiles / cus), full = std::floor(per_cu / i.resident), rest = per_cu - full * i.resident;
+    double       us     = 3.0 + (full * (round(i.resident) + 1500.0) + (rest > 0 ? round(rest) : 0.0)) / clk;
+    const double out    = static_cast<double>(g.M) * g.N * g.batch * static_cast<double>(dtype_size(g.dtype));
+    us += out / 4.0e6;                                     // the results at 4 TB/s
+    if(ks > 1) us += 3.5 + out * (ks + 1) / 3.0e6;         // the slices' sums
+    return us;
+}
+
+// All pipelined plans of g, the cheapest first.
+static std::vector<std::pair<double, LaunchPlan>> ranked_plans(const GemmDesc &g0) {
+    const GemmDesc g = oriented(g0);
+    std::vector<std::pair<double, LaunchPlan>> v;
+    for(TileCfg c : {TileCfg::T128x64, TileCfg::T64x64, TileCfg::T64x32, TileCfg::T32x32}) {
+        const pipe::Shape s = shape_of(c, g.dtype);
+        if((c == TileCfg::T128x64 && s != pipe::S128x64) || (c == TileCfg::T64x32 && s != pipe::S64x32)) continue;
+        const int bk = pipe::shape_info(g.dtype, s).BK;
+        for(int ks : {1, 2, 3, 4, 6, 8}) {
+            if(ks > 1 && (g.K < 4 * bk * ks || !g.part || g.part_capacity < static_cast<int64_t>(g.M) * g.N * g.batch * ks)) continue;
+            v.emplace_back(pipe_cost_us(g, s, ks), LaunchPlan{c, ks});
+        }
+    }
+    std::stable_sort(v.begin(), v.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
+    return v;
+}
+
+static LaunchPlan heuristic_plan(const GemmDesc &g) {
+    if(g.M <= 16) return LaunchPlan{TileCfg::T16x128, 1};
+    return ranked_plans(g).front().second;
 }
 
 // Tile-separable index map: offset(t0 + t) = offset(t0) + offset(t) for every tile origin t0 (a multiple
@@ -601,6 +652,8 @@ static bool small_tile_offsets(const Idx2 &r, int rt, const Idx2 &k, int bk, int
            k.s1 >= 0;
 }
 
+static void splitk_sum(const GemmDesc &g, hipStream_t s);
+
 template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN>
 static void launch_cfg(const GemmDesc &g, bool swap, hipStream_t s) {
     const int  tiles = ((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
@@ -617,35 +670,52 @@ static void launch_cfg(const GemmDesc &g, bool swap, hipStream_t s) {
         else hipLaunchKernelGGL((gemm_kernel<R, CPLX, BM, BN, BK, WM, WN, false, false>), grid, block, 0, s, g);
     }
     if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
-    if(g.ksplit > 1) {
-        const int64_t total = static_cast<int64_t>(g.M) * g.N * g.batch;
-        const dim3    rg(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 8192)));
-        hipLaunchKernelGGL((splitk_reduce<elem_t<R, CPLX>>), rg, dim3(256), 0, s, g);
+    if(g.ksplit > 1) splitk_sum(g, s);
+}
+
+static void splitk_sum(const GemmDesc &g, hipStream_t s) {
+    const int64_t total = static_cast<int64_t>(g.M) * g.N * g.batch;
+    const dim3    rg(static_cast<unsigned>(std::min<int64_t>((total + 255) / 256, 8192)));
+    switch(g.dtype) {
+        case DMRG_FP64: hipLaunchKernelGGL((splitk_reduce<double>), rg, dim3(256), 0, s, g); break;
+        case DMRG_CX64: hipLaunchKernelGGL((splitk_reduce<cpx<double>>), rg, dim3(256), 0, s, g); break;
+        case DMRG_FP32: hipLaunchKernelGGL((splitk_reduce<float>), rg, dim3(256), 0, s, g); break;
+        case DMRG_CX32: hipLaunchKernelGGL((splitk_reduce<cpx<float>>), rg, dim3(256), 0, s, g); break;
     }
+}
+
+// Launches g in a pipelined shape with up to ksplit K slices; false where the pipelined kernel does not take it.
+static bool launch_pipelined(const GemmDesc &g0, pipe::Shape shape, int ksplit, hipStream_t s) {
+    GemmDesc              g = oriented(g0);
+    const pipe::ShapeInfo i = pipe::shape_info(g.dtype, shape);
+    pipe::Launch          l;
+    if(!pipe::describe(g, i, ksplit, l)) return false;
+    const dim3 grid(static_cast<unsigned>((g.M + i.BM - 1) / i.BM) * static_cast<unsigned>((g.N + i.BN - 1) / i.BN), l.d.ksplit, g.batch);
+    switch(g.dtype) {
+        case DMRG_FP64: pipe::launch_f64(l, shape, grid, s); break;
+        case DMRG_CX64: pipe::launch_c128(l, shape, grid, s); break;
+        case DMRG_FP32: pipe::launch_f32(l, shape, grid, s); break;
+        case DMRG_CX32: pipe::launch_c64(l, shape, grid, s); break;
+    }
+    if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
+    if(l.d.ksplit > 1) {
+        g.ksplit = l.d.ksplit;
+        splitk_sum(g, s);
+    }
+    return true;
 }
 
 template <typename R, bool CPLX>
 static void launch_typed(const GemmDesc &g, TileCfg cfg, bool swap, hipStream_t s) {
-    // K depth per LDS stage, sized so both double-buffered tiles fit in 64 KiB of LDS:
-    // 16 elements for 8- and 16-byte elements, 32 for 4-byte ones; halved for the
-    // 16-byte element in the tall/wide configurations. All configurations run 4 waves.
+    // The kernels beside the pipelined ones: tall outputs of at most 16 rows, tiny K, and 64x64 tiles with 64-bit offsets
+    // per element for the index maps that the pipelined kernel does not take.
     constexpr int E  = static_cast<int>(sizeof(elem_t<R, CPLX>));
     constexpr int BK = E == 4 ? 32 : 16;
     constexpr int BH = E == 16 ? 8 : BK;
-    constexpr int BD = E == 4 ? 128 : 64; // deep K stage of T32x32K (LDS: at most 132 KiB of the 160 KiB)
+    if(cfg == TileCfg::SMALLK && (g.K > SMALLK_MAX_K || g.M > SMALLK_MAX_M)) cfg = TileCfg::T64x64;
     switch(cfg) {
-        case TileCfg::T64x64: launch_cfg<R, CPLX, 64, 64, BK, 2, 2>(g, swap, s); break;
-        case TileCfg::T32x64: launch_cfg<R, CPLX, 32, 64, BK, 2, 2>(g, swap, s); break;
-        case TileCfg::T64x32: launch_cfg<R, CPLX, 64, 32, BK, 2, 2>(g, swap, s); break;
         case TileCfg::T16x128: launch_cfg<R, CPLX, 16, 128, BH, 1, 4>(g, swap, s); break;
-        case TileCfg::T128x64: launch_cfg<R, CPLX, 128, 64, BH, 2, 2>(g, swap, s); break;
-        case TileCfg::T32x32: launch_cfg<R, CPLX, 32, 32, BK, 2, 2>(g, swap, s); break;
-        case TileCfg::T32x32K: launch_cfg<R, CPLX, 32, 32, BD, 2, 2>(g, swap, s); break;
         case TileCfg::SMALLK: {
-            if(g.K > SMALLK_MAX_K || g.M > SMALLK_MAX_M) { // outside the kernel's limits
-                launch_cfg<R, CPLX, 64, 64, BK, 2, 2>(g, swap, s);
-                break;
-            }
             const int64_t blocks = std::min<int64_t>((static_cast<int64_t>(g.N) + 255) / 256, 8192);
             const dim3    grid(static_cast<unsigned>(blocks), g.batch);
             if(g.K <= 8) hipLaunchKernelGGL((smallk_kernel<R, CPLX, 8>), grid, dim3(256), 0, s, g);
@@ -654,11 +724,16 @@ static void launch_typed(const GemmDesc &g, TileCfg cfg, bool swap, hipStream_t 
             if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
             break;
         }
-        default: throw Error(DMRG_ERR_ARG, "bad tile config");
+        case TileCfg::AUTO: throw Error(DMRG_ERR_ARG, "bad tile config");
+        default: {
+            const dim3 grid(((g.M + 63) / 64) * ((g.N + 63) / 64), g.ksplit, g.batch), block(256);
+            if(swap) hipLaunchKernelGGL((gemm_kernel<R, CPLX, 64, 64, BK, 2, 2, true, false>), grid, block, 0, s, g);
+            else hipLaunchKernelGGL((gemm_kernel<R, CPLX, 64, 64, BK, 2, 2, false, false>), grid, block, 0, s, g);
+            if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
+            if(g.ksplit > 1) splitk_sum(g, s);
+        }
     }
 }
-
-static int fast_score(const Idx2 &x) { return x.s0 == 1 ? static_cast<int>(std::min<uint32_t>(x.c, 1u << 20)) : 0; }
 
 // ---------------------------------------------------------------------------------------
 // Autotuner: times candidate (tile configuration, K slices) plans of a GEMM with HIP events on
@@ -682,9 +757,6 @@ static std::string tune_key(const GemmDesc &g) {
 }
 
 static void launch_plan_single(GemmDesc g, const LaunchPlan &p0, hipStream_t stream);
-
-// K depth of one LDS stage rounded up to 32 (every configuration's BK divides 32, except T32x32K's deep stage).
-static int deep_bk(TileCfg c, dmrg_dtype t) { return c == TileCfg::T32x32K ? (dtype_size(t) == 4 ? 128 : 64) : 32; }
 
 // Columns [n0, n0 + nn) of g as a GEMM of their own (valid when the B and C column maps are separable at n0).
 static GemmDesc column_slice(const GemmDesc &g, int n0, int nn) {
@@ -715,8 +787,13 @@ static void launch_plan_single(GemmDesc g, const LaunchPlan &p0, hipStream_t str
         const int64_t need = static_cast<int64_t>(g.M) * g.N * g.batch * p.ksplit;
         if(!g.part || g.part_capacity < need) p.ksplit = 1;
     }
-    g.ksplit = 1;
-    const int kr = deep_bk(p.cfg, g.dtype); // K extent per slice: a multiple of the configuration's BK
+    const pipe::Shape shape = shape_of(p.cfg, g.dtype);
+    if(shape != pipe::N_SHAPES && launch_pipelined(g, shape, p.ksplit, stream)) {
+        DMRG_HIP_CHECK(hipGetLastError());
+        return;
+    }
+    g.ksplit     = 1;
+    const int kr = 32; // K extent per slice: a multiple of every configuration's BK
     g.kchunk = (g.K + kr - 1) / kr * kr;
     if(p.ksplit > 1) {
         const int kc = (((g.K + p.ksplit - 1) / p.ksplit) + kr - 1) / kr * kr;
@@ -868,79 +945,27 @@ void grouped_free(std::vector<GroupedGemm> &gg) {
     gg.clear();
 }
 
-// Workgroups of configuration t that one CU holds at once (aligned, swapped variant as the representative).
-template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN>
-static int occupancy_of() {
-    int nb = 0;
-    if(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, gemm_kernel<R, CPLX, BM, BN, BK, WM, WN, true, true>, 64 * WM * WN, 0) != hipSuccess)
-        return 0;
-    return nb;
-}
-template <typename R, bool CPLX>
-static int occupancy_typed(TileCfg t) {
-    constexpr int E  = static_cast<int>(sizeof(elem_t<R, CPLX>));
-    constexpr int BK = E == 4 ? 32 : 16;
-    switch(t) {
-        case TileCfg::T64x64: return occupancy_of<R, CPLX, 64, 64, BK, 2, 2>();
-        case TileCfg::T32x64: return occupancy_of<R, CPLX, 32, 64, BK, 2, 2>();
-        case TileCfg::T64x32: return occupancy_of<R, CPLX, 64, 32, BK, 2, 2>();
-        default: return 0;
-    }
-}
-static int resident_blocks(dmrg_dtype dt, TileCfg t) {
-    static std::mutex mu;
-    static std::map<std::pair<int, int>, int> cache;
-    std::lock_guard<std::mutex> lock(mu);
-    const auto key = std::make_pair(static_cast<int>(dt), static_cast<int>(t));
-    auto       it  = cache.find(key);
-    if(it != cache.end()) return it->second;
-    int v = 0;
-    switch(dt) {
-        case DMRG_FP64: v = occupancy_typed<double, false>(t); break;
-        case DMRG_CX64: v = occupancy_typed<double, true>(t); break;
-        case DMRG_FP32: v = occupancy_typed<float, false>(t); break;
-        case DMRG_CX32: v = occupancy_typed<float, true>(t); break;
-    }
-    cache[key] = v;
-    return v;
-}
-
 static std::vector<LaunchPlan> candidates(const GemmDesc &g) {
     std::vector<LaunchPlan> c;
-    const TileCfg cfgs[] = {TileCfg::T64x64, TileCfg::T32x64, TileCfg::T64x32, TileCfg::T32x32, TileCfg::T128x64, TileCfg::T16x128};
     if(g.K <= SMALLK_MAX_K && g.M <= SMALLK_MAX_M) c.push_back({TileCfg::SMALLK, 1});
-    // Hybrid plans: whole waves of tiles without K slicing, the remaining tile columns sliced over K.
+    if(g.M <= 32) c.push_back({TileCfg::T16x128, 1});
+    // The pipelined plans within a third of the cheapest.
+    const auto ranked = ranked_plans(g);
+    for(const auto &r : ranked)
+        if(r.first <= 1.34 * ranked.front().first) c.push_back(r.second);
+    // Hybrid plans: as many tile columns as occupy every CU equally without K slicing, the remaining ones sliced over K.
     if(g.part && g.batch == 1 && g.K >= 128) {
-        const TileCfg hcfgs[] = {TileCfg::T64x64, TileCfg::T32x64, TileCfg::T64x32};
-        for(TileCfg t : hcfgs) {
-            const CfgShape sh    = cfg_shape(t);
-            const int      tm    = (g.M + sh.BM - 1) / sh.BM, tn = (g.N + sh.BN - 1) / sh.BN;
-            const int64_t  slots = static_cast<int64_t>(device_cu_count()) * resident_blocks(g.dtype, t);
-            if(slots <= 0 || static_cast<int64_t>(tm) * tn <= slots) continue;
-            const int64_t full_cols = (static_cast<int64_t>(tm) * tn / slots) * slots / tm; // tile columns in whole waves
-            if(full_cols <= 0 || full_cols >= tn) continue;
-            const int nsplit = static_cast<int>(full_cols * sh.BN);
+        for(TileCfg t : {TileCfg::T64x64, TileCfg::T64x32}) {
+            if(shape_of(t, g.dtype) != (t == TileCfg::T64x64 ? pipe::S64x64 : pipe::S64x32)) continue;
+            const CfgShape sh = cfg_shape(t);
+            const int      tm = (g.M + sh.BM - 1) / sh.BM, tn = (g.N + sh.BN - 1) / sh.BN;
+            const int64_t  cus = device_cu_count(), whole = static_cast<int64_t>(tm) * tn / cus * cus / tm;
+            if(whole <= 0 || whole >= tn) continue;
+            const int nsplit = static_cast<int>(whole * sh.BN);
             for(int ks2 : {2, 3, 4, 8}) {
                 if(g.K < 64 * ks2 || g.part_capacity < static_cast<int64_t>(g.M) * (g.N - nsplit) * ks2) continue;
                 c.push_back({t, 1, nsplit, ks2});
             }
-        }
-    }
-    for(TileCfg t : cfgs) {
-        if(t == TileCfg::T16x128 && g.M > 32) continue;
-        if(t == TileCfg::T128x64 && g.M < 128) continue;
-        for(int ks : {1, 2, 3, 4, 8}) {
-            if(ks > 1 && (g.K < 256 * ks || !g.part || g.part_capacity < static_cast<int64_t>(g.M) * g.N * g.batch * ks)) continue;
-            c.push_back({t, ks});
-        }
-    }
-    // Deep-K 32x32 tiles for grids that fill at most two workgroups per CU; K slices down to one stage each.
-    const int64_t tiles32 = static_cast<int64_t>((g.M + 31) / 32) * ((g.N + 31) / 32) * g.batch;
-    if(tiles32 <= 2 * device_cu_count()) {
-        const int bd = deep_bk(TileCfg::T32x32K, g.dtype);
-        for(int ks : {1, 2, 4, 8}) {
-            if(ks > 1 && (g.K < bd * ks || !g.part || g.part_capacity < static_cast<int64_t>(g.M) * g.N * g.batch * ks)) continue;
-            c.push_back({TileCfg::T32x32K, ks});
         }
     }
     return c;

@@ -1,0 +1,17 @@
+// Pipelined GEMM kernels, complex double (the shapes of shape_info).
+#include "gemm_plan.hpp"
+
+namespace dmrg {
+namespace pipe {
+
+void launch_c128(const Launch &l, Shape s, dim3 grid, hipStream_t st) {
+    switch(s) {
+        case S64x64: launch_shape<double, true, 64, 64, 8, 2, 2, 4>(l, grid, st); break;
+        case S64x32: launch_shape<double, true, 64, 32, 16, 2, 2, 3>(l, grid, st); break;
+        case S32x32: launch_shape<double, true, 32, 32, 8, 2, 2, 4>(l, grid, st); break;
+        default: throw Error(DMRG_ERR_ARG, "no such tile shape");
+    }
+}
+
+} // namespace pipe
+} // namespace dmrg

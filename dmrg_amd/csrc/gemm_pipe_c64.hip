@@ -1,0 +1,17 @@
+// Pipelined GEMM kernels, complex float (the shapes of shape_info).
+#include "gemm_plan.hpp"
+
+namespace dmrg {
+namespace pipe {
+
+void launch_c64(const Launch &l, Shape s, dim3 grid, hipStream_t st) {
+    switch(s) {
+        case S64x64: launch_shape<float, true, 64, 64, 16, 2, 2, 4>(l, grid, st); break;
+        case S64x32: launch_shape<float, true, 64, 32, 16, 2, 2, 4>(l, grid, st); break;
+        case S32x32: launch_shape<float, true, 32, 32, 16, 2, 2, 4>(l, grid, st); break;
+        default: throw Error(DMRG_ERR_ARG, "no such tile shape");
+    }
+}
+
+} // namespace pipe
+} // namespace dmrg

@@ -1,0 +1,18 @@
+// Pipelined GEMM kernels, real double (the shapes of shape_info).
+#include "gemm_plan.hpp"
+
+namespace dmrg {
+namespace pipe {
+
+void launch_f64(const Launch &l, Shape s, dim3 grid, hipStream_t st) {
+    switch(s) {
+        case S128x64: launch_shape<double, false, 128, 64, 16, 2, 2, 3>(l, grid, st); break;
+        case S64x64: launch_shape<double, false, 64, 64, 16, 2, 2, 4>(l, grid, st); break;
+        case S64x32: launch_shape<double, false, 64, 32, 16, 2, 2, 4>(l, grid, st); break;
+        case S32x32: launch_shape<double, false, 32, 32, 16, 2, 2, 4>(l, grid, st); break;
+        default: throw Error(DMRG_ERR_ARG, "no such tile shape");
+    }
+}
+
+} // namespace pipe
+} // namespace dmrg
