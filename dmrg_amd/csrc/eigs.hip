@@ -344,8 +344,7 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
             host[SB_Y + 2 * i]     = Z[i + static_cast<size_t>(m_) * col_in_H].real();
             host[SB_Y + 2 * i + 1] = Z[i + static_cast<size_t>(m_) * col_in_H].imag();
         }
-        DMRG_HIP_CHECK(hipMemcpyAsync(sm + SB_Y, host + SB_Y, 2 * m_ * sizeof(double), hipMemcpyHostToDevice, s));
-        ritz_residual<T>(n, m_, Vp, Wp, n, sm + SB_Y, w[col_in_H], xout, r, sm + SB_RITZ, scratch.as<double>(), s);
+        ritz_residual<T>(n, m_, Vp, Wp, n, host + SB_Y, sm + SB_Y, w[col_in_H], xout, r, sm + SB_RITZ, scratch.as<double>(), s);
     };
     auto ritz_norm = [&]() { // |r| / |x| from the host copy of SB_RITZ
         return std::sqrt(std::max(0.0, host[SB_RITZ])) / std::sqrt(std::max(1e-300, host[SB_RITZ + 1]));

@@ -56,12 +56,16 @@ static int grid_for(int64_t n) {
 }
 
 // ------------------------------------------------------------------------------------------- fused folds
-// A reduction over few workgroups folds its partial sums in its last workgroup instead of a second launch:
-// every workgroup publishes its partials (release fence) and counts itself in; the one that counts last
-// reads all partials past the non-coherent L1 and sums them in workgroup order (the order of the separate
-// fold kernel's operands, so the result stays deterministic), then resets the counter for the next use.
-constexpr int FUSE_MAX_BLOCKS = 128; // more partials than this per value are folded by a separate launch
+// A reduction over few workgroups folds its partial sums in its last workgroup instead of a second launch: every
+// workgroup stores its partials at device scope (past the XCD's own L2, so that no cache write-back is needed), waits for
+// them and counts itself in; the one that counts last reads all partials past the non-coherent caches and sums them in
+// workgroup order (deterministic), then resets the counter for the next use.
+// Up to 128 workgroups: every one of them counts itself in at one address, which takes about 10 ns each (n = 122880: 480
+// workgroups, update and norm 6.9 us, against 3.3 + 2.6 for the update and a fold of its own).
+constexpr int FUSE_MAX_BLOCKS = 128;
 constexpr int FUSE_MAX_VALUES = VT_THREADS;
+
+static bool fused(int64_t blocks, int values) { return blocks <= FUSE_MAX_BLOCKS && values <= FUSE_MAX_VALUES; }
 
 static unsigned *scratch_counter(double *scratch) { return reinterpret_cast<unsigned *>(scratch + vec_scratch_doubles() - 8); }
 
@@ -69,25 +73,40 @@ void vec_scratch_init(double *scratch, hipStream_t s) {
     DMRG_HIP_CHECK(hipMemsetAsync(scratch_counter(scratch), 0, 8 * sizeof(double), s));
 }
 
-// partial: [block][nv]; value v goes to out[v], or self_out[v & 1] for the column v / 2 == j_self (when given).
+// A partial sum: at device scope where the kernel's last workgroup folds it, else an ordinary store.
+__device__ inline void publish(double *p, double v, bool device_scope) {
+    if(device_scope) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else *p = v;
+}
+
+// partial: [row block][nv]; value v goes to out[v], or self_out[v & 1] for the column v / 2 == j_self (when given).
 __device__ inline void fold_in_last_block(const double *partial, int nv, double *out, int j_self, double *self_out, unsigned *counter) {
     __shared__ int last;
-    __threadfence();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the partials of this wavefront are at device scope
     __syncthreads();
-    if(threadIdx.x == 0) last = atomicAdd(counter, 1u) == gridDim.x - 1 ? 1 : 0;
+    if(threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x * gridDim.y - 1 ? 1 : 0;
     __syncthreads();
     if(!last) return;
-    __threadfence();
-    // Thread t sums value t % nv over the workgroups b = t / nv, t / nv + per, ...; then thread v adds the per
+    // Thread t sums value t % nv over the row blocks b = t / nv, t / nv + per, ...; then thread v adds the per
     // sums of value v in order. nv <= blockDim.x.
     __shared__ double red[VT_THREADS];
     const int         per = blockDim.x / nv;
     const int         t   = threadIdx.x;
     if(t < per * nv) {
-        const int v = t % nv;
-        double    a = 0.0;
-        for(unsigned b = t / nv; b < gridDim.x; b += per)
-            a += __hip_atomic_load(partial + static_cast<int64_t>(b) * nv + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int     v  = t % nv;
+        const int     nb = static_cast<int>(gridDim.x);
+        double        a  = 0.0;
+        constexpr int UN = 8;
+        for(int b = t / nv; b < nb; b += UN * per) {
+            double x[UN];
+#pragma unroll
+            for(int u = 0; u < UN; ++u)
+                x[u] = __hip_atomic_load(partial + static_cast<int64_t>(min(b + u * per, nb - 1)) * nv + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for(int u = 0; u < UN; ++u)
+                if(b + u * per < nb) a += x[u];
+        }
         red[t] = a;
     }
     __syncthreads();
@@ -101,7 +120,12 @@ __device__ inline void fold_in_last_block(const double *partial, int nv, double 
 }
 
 // ------------------------------------------------------------------------------------------- multidot
-constexpr int MD_CH        = 16;  // basis columns per pass (32 double accumulators per thread)
+// Basis columns per pass (two double accumulators each). Long vectors: 16, so that x is read once per 16 columns. Short
+// ones: 4, with the groups of columns in their own workgroups: the rows alone give too few of them, and the reduction
+// across a wavefront shrinks from 32 values to 8 (n = 8192, 14 columns: 8 workgroups 14.3 us, 128 workgroups 4.5 us).
+constexpr int MD_CH        = 16;
+constexpr int MD_CH_SHORT  = 4;
+constexpr int64_t MD_SHORT = int64_t(1) << 17; // up to here the basis is read from the caches, and latency is what counts
 constexpr int MD_PER_THREAD = 4;  // rows per thread and pass at full grid: amortises the block reduction
 
 // Reduce-scatter of NV values across the 64 lanes of a wavefront: after the call lane l holds in v[0] the
@@ -146,22 +170,23 @@ struct DgksTest {
     int          *flag = nullptr;
 };
 
-// Columns j < m are V[:, j]; column m (when with_self) is x itself, so x^H x comes out of the same pass.
-template <typename T>
+// Columns j < m are V[:, j]; column m (when with_self) is x itself, so x^H x comes out of the same pass. Workgroup
+// (b, g) takes the rows of b and the columns [CH g, CH (g + 1)) and then every CH gridDim.y-th group.
+template <typename T, int CH>
 __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m, int mc, const T *V, int64_t ldv, const T *x,
                                                                const int *skip, double *partial, unsigned *counter, double *out,
                                                                int m_out, double *self_out, DgksTest dg) {
     if(dg.flag) {
         const bool run = dg.post[0] < dg.eta2 * dg.pre[0];
-        if(blockIdx.x == 0 && threadIdx.x == 0) dg.flag[0] = run ? 1 : 0;
+        if(blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) dg.flag[0] = run ? 1 : 0;
         if(!run) return;
     } else if(skip && *skip == 0) {
         return;
     }
-    constexpr int     NV = 2 * MD_CH;
+    constexpr int     NV = 2 * CH;
     __shared__ double red[NV][VT_THREADS / 64];
     const int         lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for(int j0 = 0; j0 < mc; j0 += MD_CH) {
+    for(int j0 = blockIdx.y * CH; j0 < mc; j0 += CH * static_cast<int>(gridDim.y)) {
         double acc[NV];
 #pragma unroll
         for(int c = 0; c < NV; ++c) acc[c] = 0.0;
@@ -169,7 +194,7 @@ __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m,
             double xr, xi;
             ld(x[i], xr, xi);
 #pragma unroll
-            for(int c = 0; c < MD_CH; ++c) {
+            for(int c = 0; c < CH; ++c) {
                 if(j0 + c < mc) {
                     double vr, vi;
                     if(j0 + c < m) ld(V[i + (j0 + c) * ldv], vr, vi);
@@ -188,7 +213,7 @@ __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m,
                 double t = 0;
 #pragma unroll
                 for(int w = 0; w < VT_THREADS / 64; ++w) t += red[threadIdx.x][w];
-                partial[2 * (static_cast<int64_t>(blockIdx.x) * mc + j0 + c) + (threadIdx.x & 1)] = t;
+                publish(partial + 2 * (static_cast<int64_t>(blockIdx.x) * mc + j0 + c) + (threadIdx.x & 1), t, counter != nullptr);
             }
         }
         __syncthreads();
@@ -221,38 +246,34 @@ __global__ __launch_bounds__(VT_THREADS) void fold_columns(int nblk, int m, cons
 }
 
 template <typename T>
-void multidot(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_out, double *scratch, hipStream_t s) {
-    if(m <= 0) return;
-    DMRG_REQUIRE(m <= VEC_MAX_M, DMRG_ERR_ARG, "multidot: too many columns");
-    const int g = md_grid(n);
-    if(g <= FUSE_MAX_BLOCKS && 2 * m <= FUSE_MAX_VALUES) {
-        hipLaunchKernelGGL(multidot_partial<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, m, V, ldv, x, nullptr, scratch,
-                           scratch_counter(scratch), d_out, -1, nullptr, DgksTest{});
-    } else {
-        hipLaunchKernelGGL(multidot_partial<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, m, V, ldv, x, nullptr, scratch, nullptr,
-                           nullptr, -1, nullptr, DgksTest{});
-        hipLaunchKernelGGL(fold_columns, dim3(m), dim3(VT_THREADS), 0, s, g, m, scratch, d_out, -1, nullptr, nullptr);
-    }
-    DMRG_HIP_CHECK(hipGetLastError());
-}
-
-template <typename T>
 static void multidot_x_impl(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_out, double *d_self, const int *skip,
                             const DgksTest &dg, double *scratch, hipStream_t s) {
     const int mc = m + (d_self ? 1 : 0);
     if(mc <= 0) return;
     DMRG_REQUIRE(mc <= VEC_MAX_M, DMRG_ERR_ARG, "multidot: too many columns");
-    const int  g     = md_grid(n);
     const int *fskip = dg.flag ? dg.flag : skip; // the fold follows the pass's decision
-    if(g <= FUSE_MAX_BLOCKS && 2 * mc <= FUSE_MAX_VALUES) {
-        hipLaunchKernelGGL(multidot_partial<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch,
-                           scratch_counter(scratch), d_out, d_self ? m : -1, d_self, dg);
+    if(n <= MD_SHORT) {
+        // One row per thread, or two where that lets the last workgroup fold.
+        const int groups = (mc + MD_CH_SHORT - 1) / MD_CH_SHORT, most = std::max(1, FUSE_MAX_BLOCKS / groups);
+        const int want   = static_cast<int>(std::max<int64_t>(1, (n + VT_THREADS - 1) / VT_THREADS));
+        const bool in_last = want <= 2 * most && fused(static_cast<int64_t>(std::min(want, most)) * groups, 2 * mc);
+        const int  rows    = in_last ? std::min(want, most) : std::min(want, 256);
+        hipLaunchKernelGGL((multidot_partial<T, MD_CH_SHORT>), dim3(rows, groups), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch,
+                           in_last ? scratch_counter(scratch) : nullptr, d_out, d_self ? m : -1, d_self, dg);
+        if(!in_last)
+            hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, rows, mc, scratch, d_out, d_self ? m : -1, d_self, fskip);
     } else {
-        hipLaunchKernelGGL(multidot_partial<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch, nullptr,
+        const int g = md_grid(n);
+        hipLaunchKernelGGL((multidot_partial<T, MD_CH>), dim3(g), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch, nullptr,
                            nullptr, -1, nullptr, dg);
         hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, g, mc, scratch, d_out, d_self ? m : -1, d_self, fskip);
     }
     DMRG_HIP_CHECK(hipGetLastError());
+}
+
+template <typename T>
+void multidot(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_out, double *scratch, hipStream_t s) {
+    multidot_x_impl<T>(n, m, V, ldv, x, d_out, nullptr, nullptr, DgksTest{}, scratch, s);
 }
 
 template <typename T>
@@ -273,6 +294,21 @@ void multidot_dgks(int64_t n, int m, const T *V, int64_t ldv, const T *x, double
 }
 
 // ------------------------------------------------------------------------------------------- gemv
+// use(j, load(j)) for j < m in order, with eight loads in flight: one at a time, a row of a basis of 13 waits for 13
+// memory latencies (n = 8192: update 8 -> 4.0 us, Ritz vector and residual 10 -> 6.8 us).
+template <typename T, typename L, typename F>
+__device__ __forceinline__ void columns(int m, L &&load, F &&use) {
+    constexpr int UN = 8;
+    for(int j0 = 0; j0 < m; j0 += UN) {
+        T v[UN];
+#pragma unroll
+        for(int u = 0; u < UN; ++u) v[u] = load(min(j0 + u, m - 1));
+#pragma unroll
+        for(int u = 0; u < UN; ++u)
+            if(j0 + u < m) use(j0 + u, v[u]);
+    }
+}
+
 template <typename T>
 __global__ __launch_bounds__(VT_THREADS) void gemv_update_kernel(int64_t n, int m, const T *V, int64_t ldv, const double *h,
                                                                  double alpha, double beta, T *x) {
@@ -281,12 +317,13 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_kernel(int64_t n, int 
     __syncthreads();
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
         double ar = 0, ai = 0;
-        for(int j = 0; j < m; ++j) {
-            double vr, vi;
-            ld(V[i + j * ldv], vr, vi);
-            ar += vr * hs[2 * j] - vi * hs[2 * j + 1];
-            ai += vr * hs[2 * j + 1] + vi * hs[2 * j];
-        }
+        columns<T>(m, [&](int j) { return V[i + j * ldv]; },
+                   [&](int j, const T &v) {
+                       double vr, vi;
+                       ld(v, vr, vi);
+                       ar += vr * hs[2 * j] - vi * hs[2 * j + 1];
+                       ai += vr * hs[2 * j + 1] + vi * hs[2 * j];
+                   });
         double xr = 0, xi = 0;
         if(beta != 0.0) ld(x[i], xr, xi);
         x[i] = mk<T>(beta * xr + alpha * ar, beta * xi + alpha * ai);
@@ -307,12 +344,13 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_norm_kernel(int64_t n,
     double acc[2] = {0.0, 0.0};
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
         double ar = 0, ai = 0;
-        for(int j = 0; j < m; ++j) {
-            double vr, vi;
-            ld(V[i + j * ldv], vr, vi);
-            ar += vr * hs[2 * j] - vi * hs[2 * j + 1];
-            ai += vr * hs[2 * j + 1] + vi * hs[2 * j];
-        }
+        columns<T>(m, [&](int j) { return V[i + j * ldv]; },
+                   [&](int j, const T &v) {
+                       double vr, vi;
+                       ld(v, vr, vi);
+                       ar += vr * hs[2 * j] - vi * hs[2 * j + 1];
+                       ai += vr * hs[2 * j + 1] + vi * hs[2 * j];
+                   });
         double xr = 0, xi = 0;
         if(beta != 0.0) ld(x[i], xr, xi);
         const T yv = mk<T>(beta * xr + alpha * ar, beta * xi + alpha * ai);
@@ -323,8 +361,8 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_norm_kernel(int64_t n,
     }
     bsum<2>(acc, red);
     if(threadIdx.x == 0) {
-        partial[2 * blockIdx.x]     = acc[0];
-        partial[2 * blockIdx.x + 1] = 0.0;
+        publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
+        publish(partial + 2 * blockIdx.x + 1, 0.0, counter != nullptr);
     }
     if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
 }
@@ -343,7 +381,7 @@ void gemv_update_norm(int64_t n, int m, const T *V, int64_t ldv, const double *d
                       double *d_nrm2, const int *skip, double *scratch, hipStream_t s) {
     DMRG_REQUIRE(m <= VEC_MAX_M, DMRG_ERR_ARG, "gemv: too many columns");
     const int g = grid_for(n);
-    if(g <= FUSE_MAX_BLOCKS) {
+    if(fused(g, 2)) {
         hipLaunchKernelGGL(gemv_update_norm_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, alpha, beta, x, y, skip, scratch,
                            scratch_counter(scratch), d_nrm2);
     } else {
@@ -355,26 +393,40 @@ void gemv_update_norm(int64_t n, int m, const T *V, int64_t ldv, const double *d
 }
 
 // ------------------------------------------------------------------------------------------- Ritz vector + residual
+// The coefficients come with the launch (up to RITZ_ARGS of them) or from device memory (y).
+constexpr int RITZ_ARGS = 32;
+struct RitzCoef {
+    double y[2 * RITZ_ARGS];
+};
 template <typename T>
 __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *y,
-                                                          double theta, T *x, T *r, double *partial, unsigned *counter, double *out) {
+                                                          const RitzCoef c, double theta, T *x, T *r, double *partial, unsigned *counter,
+                                                          double *out) {
     __shared__ double ys[2 * VEC_MAX_M];
     __shared__ double red[2][VT_THREADS / 64];
-    for(int j = threadIdx.x; j < 2 * m; j += VT_THREADS) ys[j] = y[j];
+    if(y) {
+        for(int j = threadIdx.x; j < 2 * m; j += VT_THREADS) ys[j] = y[j];
+    } else if(threadIdx.x < 2 * m) {
+        ys[threadIdx.x] = c.y[threadIdx.x]; // 2 m <= 2 RITZ_ARGS < VT_THREADS
+    }
     __syncthreads();
     double acc[2] = {0.0, 0.0};
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
         double xr = 0, xi = 0, wr = 0, wi = 0;
-        for(int j = 0; j < m; ++j) {
-            double vr, vi, ur, ui;
-            ld(V[i + j * ldv], vr, vi);
-            ld(W[i + j * ldv], ur, ui);
-            const double yr = ys[2 * j], yi = ys[2 * j + 1];
-            xr += vr * yr - vi * yi;
-            xi += vr * yi + vi * yr;
-            wr += ur * yr - ui * yi;
-            wi += ur * yi + ui * yr;
-        }
+        struct VW {
+            T v, w;
+        };
+        columns<VW>(m, [&](int j) { return VW{V[i + j * ldv], W[i + j * ldv]}; },
+                    [&](int j, const VW &e) {
+                        double vr, vi, ur, ui;
+                        ld(e.v, vr, vi);
+                        ld(e.w, ur, ui);
+                        const double yr = ys[2 * j], yi = ys[2 * j + 1];
+                        xr += vr * yr - vi * yi;
+                        xi += vr * yi + vi * yr;
+                        wr += ur * yr - ui * yi;
+                        wi += ur * yi + ui * yr;
+                    });
         const double rr = wr - theta * xr, ri = wi - theta * xi;
         x[i] = mk<T>(xr, xi);
         r[i] = mk<T>(rr, ri);
@@ -383,25 +435,38 @@ __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, cons
     }
     bsum<2>(acc, red);
     if(threadIdx.x == 0) {
-        partial[2 * blockIdx.x]     = acc[0];
-        partial[2 * blockIdx.x + 1] = acc[1];
+        publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
+        publish(partial + 2 * blockIdx.x + 1, acc[1], counter != nullptr);
     }
     if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
 }
 
 template <typename T>
-void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *d_y, double theta, T *x, T *r,
-                   double *d_out, double *scratch, hipStream_t s) {
+static void ritz_launch(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *d_y, const RitzCoef &c, double theta, T *x, T *r,
+                        double *d_out, double *scratch, hipStream_t s) {
     DMRG_REQUIRE(m <= VEC_MAX_M, DMRG_ERR_ARG, "ritz: too many columns");
     const int g = grid_for(n);
-    if(g <= FUSE_MAX_BLOCKS) {
-        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, theta, x, r, scratch,
+    if(fused(g, 2)) {
+        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch,
                            scratch_counter(scratch), d_out);
     } else {
-        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, theta, x, r, scratch, nullptr, nullptr);
+        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch, nullptr, nullptr);
         hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_out, -1, nullptr, nullptr);
     }
     DMRG_HIP_CHECK(hipGetLastError());
+}
+
+template <typename T>
+void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *h_y, double *d_y, double theta, T *x, T *r,
+                   double *d_out, double *scratch, hipStream_t s) {
+    RitzCoef c{};
+    if(m <= RITZ_ARGS) {
+        std::copy(h_y, h_y + 2 * m, c.y);
+        d_y = nullptr;
+    } else {
+        DMRG_HIP_CHECK(hipMemcpyAsync(d_y, h_y, 2 * static_cast<size_t>(m) * sizeof(double), hipMemcpyHostToDevice, s));
+    }
+    ritz_launch<T>(n, m, V, W, ld, d_y, c, theta, x, r, d_out, scratch, s);
 }
 
 // ------------------------------------------------------------------------------------------- elementwise
@@ -507,7 +572,7 @@ __global__ __launch_bounds__(VT_THREADS) void cg_shift_kernel(int64_t n, const T
 // r = -sigma (r - x c) with c = x^H r (dots[0..1]); p = r; t = 0; partial |r|^2 per block.
 template <typename T>
 __global__ __launch_bounds__(VT_THREADS) void cg_init_kernel(int64_t n, const T *x, const double *c, double sigma, T *r, T *p, T *t,
-                                                             double *partial) {
+                                                             double *partial, unsigned *counter, double *out) {
     __shared__ double red[1][VT_THREADS / 64];
     const double      cr = c[0], ci = c[1];
     double            acc[1] = {0.0};
@@ -526,9 +591,10 @@ __global__ __launch_bounds__(VT_THREADS) void cg_init_kernel(int64_t n, const T 
     }
     bsum<1>(acc, red);
     if(threadIdx.x == 0) {
-        partial[2 * blockIdx.x]     = acc[0];
-        partial[2 * blockIdx.x + 1] = 0.0;
+        publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
+        publish(partial + 2 * blockIdx.x + 1, 0.0, counter != nullptr);
     }
+    if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
 }
 
 // state <- start of the iteration: rho_0 = |r|^2 (rr[0]); stopped when r = 0.
@@ -545,7 +611,8 @@ __global__ void cg_start_kernel(const double *rr, double *state) {
 // alpha = rho / p^H q; t += alpha p; r -= alpha (q - x (x^H q)); partial |r|^2. No update on a breakdown (p^H q <= 0).
 template <typename T>
 __global__ __launch_bounds__(VT_THREADS) void cg_update_kernel(int64_t n, const T *x, const T *p, const T *q, const double *dots,
-                                                               const double *state, int k, T *t, T *r, double *partial) {
+                                                               const double *state, int k, T *t, T *r, double *partial,
+                                                               unsigned *counter, double *out) {
     __shared__ double red[1][VT_THREADS / 64];
     const double      pq   = dots[2];
     const bool        live = state[CG_STOP + (k & 1)] == 0.0 && pq > 0.0;
@@ -571,9 +638,10 @@ __global__ __launch_bounds__(VT_THREADS) void cg_update_kernel(int64_t n, const 
     }
     bsum<1>(acc, red);
     if(threadIdx.x == 0) {
-        partial[2 * blockIdx.x]     = acc[0];
-        partial[2 * blockIdx.x + 1] = 0.0;
+        publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
+        publish(partial + 2 * blockIdx.x + 1, 0.0, counter != nullptr);
     }
+    if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
 }
 
 // beta = |r|^2 / rho; p = r + beta p; block 0 advances the state (rho, stop flag, step count).
@@ -604,8 +672,10 @@ template <typename T>
 void cg_init(int64_t n, const T *x, const double *d_c, double sigma, T *r, T *p, T *t, double *d_rr, double *state, double *scratch,
              hipStream_t s) {
     const int g = grid_for(n);
-    hipLaunchKernelGGL(cg_init_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, x, d_c, sigma, r, p, t, scratch);
-    hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr);
+    const bool in_last = fused(g, 2);
+    hipLaunchKernelGGL(cg_init_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, x, d_c, sigma, r, p, t, scratch,
+                       in_last ? scratch_counter(scratch) : nullptr, d_rr);
+    if(!in_last) hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr);
     hipLaunchKernelGGL(cg_start_kernel, dim3(1), dim3(1), 0, s, d_rr, state);
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -620,8 +690,10 @@ template <typename T>
 void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t, T *r, double *d_rr, double *state, int k,
              double rtol2, double *scratch, hipStream_t s) {
     const int g = grid_for(n);
-    hipLaunchKernelGGL(cg_update_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, x, p, q, d_dots, state, k, t, r, scratch);
-    hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr);
+    const bool in_last = fused(g, 2);
+    hipLaunchKernelGGL(cg_update_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, x, p, q, d_dots, state, k, t, r, scratch,
+                       in_last ? scratch_counter(scratch) : nullptr, d_rr);
+    if(!in_last) hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr);
     hipLaunchKernelGGL(cg_direction_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, r, d_dots, d_rr, state, k, rtol2, p);
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -629,8 +701,8 @@ void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t
 #define DMRG_VEC_INST(T)                                                                                                 \
     template void multidot<T>(int64_t, int, const T *, int64_t, const T *, double *, double *, hipStream_t);          \
     template void gemv_update<T>(int64_t, int, const T *, int64_t, const double *, double, double, T *, hipStream_t); \
-    template void ritz_residual<T>(int64_t, int, const T *, const T *, int64_t, const double *, double, T *, T *,      \
-                                   double *, double *, hipStream_t);                                                   \
+    template void ritz_residual<T>(int64_t, int, const T *, const T *, int64_t, const double *, double *, double, T *,  \
+                                   T *, double *, double *, hipStream_t);                                              \
     template void scale_by_inv_norm<T>(int64_t, T *, const double *, hipStream_t);                                    \
     template void scale<T>(int64_t, T *, double, hipStream_t);                                                         \
     template void random_fill<T>(int64_t, T *, uint64_t, hipStream_t);                                               \

@@ -64,9 +64,10 @@ void multidot_dgks(int64_t n, int m, const T *V, int64_t ldv, const T *x, double
 // x = beta x + alpha V h   (h: complex double, m entries, device).
 template <typename T>
 void gemv_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h, double alpha, double beta, T *x, hipStream_t s);
-// x = V y, r = W y - theta x, d_out[0] = |r|^2, d_out[1] = |x|^2 (y: complex double, device).
+// x = V y, r = W y - theta x, d_out[0] = |r|^2, d_out[1] = |x|^2 (h_y: m complex doubles on the host, pinned; d_y: room for
+// them on the device, used when they are too many for the launch's arguments; h_y is then read by a queued copy).
 template <typename T>
-void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *d_y, double theta, T *x, T *r,
+void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *h_y, double *d_y, double theta, T *x, T *r,
                    double *d_out, double *scratch, hipStream_t s);
 // x *= 1 / sqrt(d_nrm2[0]) (the squared norm read on the device).
 template <typename T>
