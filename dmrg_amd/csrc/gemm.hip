@@ -22,11 +22,14 @@
 #include "gemm_plan.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
+#include <cstring>
 #include <map>
 #include <mutex>
 #include <string>
 #include <type_traits>
+#include <unordered_map>
 #include <vector>
 
 namespace dmrg {
@@ -684,25 +687,36 @@ static void splitk_sum(const GemmDesc &g, hipStream_t s) {
     }
 }
 
-// Launches g in a pipelined shape with up to ksplit K slices; false where the pipelined kernel does not take it.
-static bool launch_pipelined(const GemmDesc &g0, pipe::Shape shape, int ksplit, hipStream_t s) {
-    GemmDesc              g = oriented(g0);
+// A GEMM described for a pipelined shape, all but its pointers fixed.
+struct Prepared {
+    pipe::Launch l;
+    pipe::Shape  shape;
+    dim3         grid;
+};
+
+// Describes g (oriented) for a shape with up to ksplit K slices; false where the pipelined kernel does not take it.
+static bool prepare_pipelined(const GemmDesc &g, pipe::Shape shape, int ksplit, Prepared &p) {
     const pipe::ShapeInfo i = pipe::shape_info(g.dtype, shape);
-    pipe::Launch          l;
-    if(!pipe::describe(g, i, ksplit, l)) return false;
-    const dim3 grid(static_cast<unsigned>((g.M + i.BM - 1) / i.BM) * static_cast<unsigned>((g.N + i.BN - 1) / i.BN), l.d.ksplit, g.batch);
+    if(!pipe::describe(g, i, ksplit, p.l)) return false;
+    p.shape = shape;
+    p.grid  = dim3(static_cast<unsigned>((g.M + i.BM - 1) / i.BM) * static_cast<unsigned>((g.N + i.BN - 1) / i.BN), p.l.d.ksplit, g.batch);
+    return true;
+}
+
+// g: oriented, with the pointers of p's description.
+static void run_pipelined(GemmDesc g, const Prepared &p, hipStream_t s) {
     switch(g.dtype) {
-        case DMRG_FP64: pipe::launch_f64(l, shape, grid, s); break;
-        case DMRG_CX64: pipe::launch_c128(l, shape, grid, s); break;
-        case DMRG_FP32: pipe::launch_f32(l, shape, grid, s); break;
-        case DMRG_CX32: pipe::launch_c64(l, shape, grid, s); break;
+        case DMRG_FP64: pipe::launch_f64(p.l, p.shape, p.grid, s); break;
+        case DMRG_CX64: pipe::launch_c128(p.l, p.shape, p.grid, s); break;
+        case DMRG_FP32: pipe::launch_f32(p.l, p.shape, p.grid, s); break;
+        case DMRG_CX32: pipe::launch_c64(p.l, p.shape, p.grid, s); break;
     }
     if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
-    if(l.d.ksplit > 1) {
-        g.ksplit = l.d.ksplit;
+    if(p.l.d.ksplit > 1) {
+        g.ksplit = p.l.d.ksplit;
         splitk_sum(g, s);
     }
-    return true;
+    DMRG_HIP_CHECK(hipGetLastError());
 }
 
 template <typename R, bool CPLX>
@@ -745,6 +759,7 @@ static int                               g_autotune     = 1;
 // GEMMs below this many (complex or real) multiply-adds, and with fewer than a sixteenth as many bytes of operands,
 // take the size heuristic instead of being tuned.
 static int64_t                           g_tune_min_macs = int64_t(1) << 29;
+static std::atomic<uint64_t>             g_plan_state{0}; // counts the changes that can change a plan
 static int                               g_override_cfg = -1, g_override_ks = 0;
 static int                               g_override_nsplit = 0, g_override_ks2 = 1;
 
@@ -788,9 +803,13 @@ static void launch_plan_single(GemmDesc g, const LaunchPlan &p0, hipStream_t str
         if(!g.part || g.part_capacity < need) p.ksplit = 1;
     }
     const pipe::Shape shape = shape_of(p.cfg, g.dtype);
-    if(shape != pipe::N_SHAPES && launch_pipelined(g, shape, p.ksplit, stream)) {
-        DMRG_HIP_CHECK(hipGetLastError());
-        return;
+    if(shape != pipe::N_SHAPES) {
+        const GemmDesc h = oriented(g);
+        Prepared       pr;
+        if(prepare_pipelined(h, shape, p.ksplit, pr)) {
+            run_pipelined(h, pr, stream);
+            return;
+        }
     }
     g.ksplit     = 1;
     const int kr = 32; // K extent per slice: a multiple of every configuration's BK
@@ -1042,18 +1061,26 @@ static void append_tune_cache_locked(const std::string &key, const LaunchPlan &p
     }
 }
 
-void set_autotune(int on) { g_autotune = on; }
-void set_tune_min_macs(int64_t macs) { g_tune_min_macs = macs; }
+void set_autotune(int on) {
+    g_autotune = on;
+    ++g_plan_state;
+}
+void set_tune_min_macs(int64_t macs) {
+    g_tune_min_macs = macs;
+    ++g_plan_state;
+}
 int  autotune_enabled() { return g_autotune; }
 void set_plan_override(int cfg, int ks, int nsplit, int ks2) {
     g_override_cfg    = cfg;
     g_override_ks     = ks;
     g_override_nsplit = nsplit;
     g_override_ks2    = ks2;
+    ++g_plan_state;
 }
 void clear_tuning() {
     std::lock_guard<std::mutex> lock(g_tune_mu);
     g_tuned.clear();
+    ++g_plan_state;
 }
 int tuned_entries() {
     std::lock_guard<std::mutex> lock(g_tune_mu);
@@ -1064,6 +1091,46 @@ static thread_local bool g_tls_no_tune = false;
 NoTuneScope::NoTuneScope() : prev_(g_tls_no_tune) { g_tls_no_tune = true; }
 NoTuneScope::~NoTuneScope() { g_tls_no_tune = prev_; }
 
+// Plans of GEMMs already met on this thread, by everything but their pointers: planning and describing a GEMM takes
+// about 10 us on the host, a launch about 3. An entry is good for one state of the tuner (g_plan_state); at most
+// PLAN_CACHE_MAX entries of about 700 bytes are kept, and given back when the thread ends.
+constexpr size_t PLAN_CACHE_MAX = 4096;
+struct PlanKey {
+    int64_t v[32];
+    bool    operator==(const PlanKey &o) const { return std::memcmp(v, o.v, sizeof(v)) == 0; }
+};
+struct PlanKeyHash {
+    size_t operator()(const PlanKey &k) const {
+        uint64_t h = 0x9E3779B97F4A7C15ull;
+        for(int64_t x : k.v) h = (h ^ static_cast<uint64_t>(x)) * 0xD6E8FEB86659FD93ull, h ^= h >> 32;
+        return static_cast<size_t>(h);
+    }
+};
+struct PlanEntry {
+    uint64_t   state;
+    bool       pipelined; // p is complete; otherwise plan is launched as it stands
+    LaunchPlan plan;
+    Prepared   p;
+};
+static PlanKey plan_key(const GemmDesc &g) {
+    PlanKey k{};
+    int     n = 0;
+    auto    add = [&](int64_t x) { k.v[n++] = x; };
+    add(static_cast<int64_t>(g.dtype) | static_cast<int64_t>(g.conjA != 0) << 8 | static_cast<int64_t>(g.conjB != 0) << 9 |
+        static_cast<int64_t>(g.accumulate != 0) << 10 | static_cast<int64_t>(g.part != nullptr) << 11 |
+        static_cast<int64_t>(g.xcd_remap != 0) << 12 | static_cast<int64_t>(reinterpret_cast<uintptr_t>(g.A) & 3) << 16 |
+        static_cast<int64_t>(reinterpret_cast<uintptr_t>(g.B) & 3) << 18);
+    add(static_cast<int64_t>(g.M) << 32 | static_cast<uint32_t>(g.N));
+    add(static_cast<int64_t>(g.K) << 32 | static_cast<uint32_t>(g.batch));
+    for(const Idx2 &x : {g.am, g.ak, g.bk, g.bn, g.cm, g.cn}) {
+        add(x.s0);
+        add(x.s1);
+        add(x.c);
+    }
+    add(g.a_batch), add(g.b_batch), add(g.c_batch), add(g.part_capacity);
+    return k;
+}
+
 void gemm(const GemmDesc &gin, hipStream_t stream, TileCfg cfg, int ksplit) {
     if(gin.M <= 0 || gin.N <= 0 || gin.batch <= 0) return;
     GemmDesc g = gin;
@@ -1073,44 +1140,79 @@ void gemm(const GemmDesc &gin, hipStream_t stream, TileCfg cfg, int ksplit) {
     DMRG_REQUIRE(static_cast<int64_t>(g.M) * g.N < (int64_t(1) << 31), DMRG_ERR_DIMS, "gemm: output too large for 32-bit tile indexing");
     g.a_fast_m = fast_score(g.am) >= fast_score(g.ak) ? 1 : 0;
     g.b_fast_k = fast_score(g.bk) >= fast_score(g.bn) ? 1 : 0;
-    LaunchPlan p;
     if(g_override_cfg >= 0) {
-        p = {static_cast<TileCfg>(g_override_cfg), std::max(1, g_override_ks), g_override_nsplit, std::max(1, g_override_ks2)};
-    } else if(cfg != TileCfg::AUTO) {
-        p = {cfg, std::max(1, ksplit)};
-    } else {
-        // Tuning needs synchronisation, so it is skipped for accumulating GEMMs (repeated launches would
-        // add up) and while the stream is being captured into a graph.
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        DMRG_HIP_CHECK(hipStreamIsCapturing(stream, &cs));
-        // Only large GEMMs are timed (at least g_tune_min_macs multiply-adds, or g_tune_min_macs / 16 bytes of
-        // operands for the memory-bound ones): a sweep or a request stream meets thousands of small shapes once
-        // each, whose tuning (about 180 timed, synchronised launches) costs more than any plan saves.
-        const double macs  = static_cast<double>(g.M) * g.N * std::max(g.K, 1) * g.batch;
-        const double bytes = (static_cast<double>(g.M) * g.K + static_cast<double>(g.K) * g.N + static_cast<double>(g.M) * g.N) *
-                             g.batch * static_cast<double>(dtype_size(g.dtype));
-        const bool   large = macs >= static_cast<double>(g_tune_min_macs) || bytes * 16.0 >= static_cast<double>(g_tune_min_macs);
-        const bool   can_tune = g_autotune && !g.accumulate && cs == hipStreamCaptureStatusNone && !g_tls_no_tune && large;
-        const std::string key = tune_key(g);
-        bool              found = false;
-        {
+        launch_plan(g, {static_cast<TileCfg>(g_override_cfg), std::max(1, g_override_ks), g_override_nsplit, std::max(1, g_override_ks2)}, stream);
+        return;
+    }
+    if(cfg != TileCfg::AUTO) {
+        launch_plan(g, {cfg, std::max(1, ksplit)}, stream);
+        return;
+    }
+    static thread_local std::unordered_map<PlanKey, PlanEntry, PlanKeyHash> cache;
+    const uint64_t state = g_plan_state.load(std::memory_order_acquire);
+    const PlanKey  ck    = plan_key(g);
+    if(ksplit <= 0) {
+        const auto it = cache.find(ck);
+        if(it != cache.end() && it->second.state == state) {
+            PlanEntry &e = it->second;
+            if(!e.pipelined) {
+                launch_plan(g, e.plan, stream);
+                return;
+            }
+            const GemmDesc h = oriented(g);
+            e.p.l.d.a.p  = h.A;
+            e.p.l.d.b.p  = h.B;
+            e.p.l.d.C    = h.C;
+            e.p.l.d.part = h.part;
+            run_pipelined(h, e.p, stream);
+            return;
+        }
+    }
+    // Tuning needs synchronisation, so it is skipped for accumulating GEMMs (repeated launches would
+    // add up) and while the stream is being captured into a graph.
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    DMRG_HIP_CHECK(hipStreamIsCapturing(stream, &cs));
+    // Only large GEMMs are timed (at least g_tune_min_macs multiply-adds, or g_tune_min_macs / 16 bytes of
+    // operands for the memory-bound ones): a sweep or a request stream meets thousands of small shapes once
+    // each, whose tuning (dozens of timed, synchronised launches) costs more than any plan saves.
+    const double macs  = static_cast<double>(g.M) * g.N * std::max(g.K, 1) * g.batch;
+    const double bytes = (static_cast<double>(g.M) * g.K + static_cast<double>(g.K) * g.N + static_cast<double>(g.M) * g.N) *
+                         g.batch * static_cast<double>(dtype_size(g.dtype));
+    const bool   large = macs >= static_cast<double>(g_tune_min_macs) || bytes * 16.0 >= static_cast<double>(g_tune_min_macs);
+    const bool   tunable  = g_autotune && !g.accumulate && large;
+    const bool   can_tune = tunable && cs == hipStreamCaptureStatusNone && !g_tls_no_tune;
+    const std::string key = tune_key(g);
+    LaunchPlan        p;
+    bool              found = false;
+    {
+        std::lock_guard<std::mutex> lock(g_tune_mu);
+        load_tune_cache_locked();
+        auto                        it = g_tuned.find(key);
+        if(it != g_tuned.end()) {
+            p     = it->second;
+            found = true;
+        }
+    }
+    if(!found) {
+        p = can_tune ? tune(g, stream) : heuristic_plan(g);
+        if(can_tune) {
             std::lock_guard<std::mutex> lock(g_tune_mu);
-            load_tune_cache_locked();
-            auto                        it = g_tuned.find(key);
-            if(it != g_tuned.end()) {
-                p     = it->second;
-                found = true;
-            }
+            g_tuned[key] = p;
+            append_tune_cache_locked(key, p);
         }
-        if(!found) {
-            p = can_tune ? tune(g, stream) : heuristic_plan(g);
-            if(can_tune) {
-                std::lock_guard<std::mutex> lock(g_tune_mu);
-                g_tuned[key] = p;
-                append_tune_cache_locked(key, p);
-            }
-        }
-        if(ksplit > 0) p = LaunchPlan{p.cfg, ksplit};
+    }
+    if(ksplit > 0) {
+        launch_plan(g, LaunchPlan{p.cfg, ksplit}, stream);
+        return;
+    }
+    // Kept unless a later call may time this GEMM and decide otherwise.
+    if(found || can_tune || !tunable) {
+        if(cache.size() >= PLAN_CACHE_MAX) cache.clear();
+        PlanEntry        e{state, false, p, {}};
+        const pipe::Shape shape = shape_of(p.cfg, g.dtype);
+        const bool        slices = p.ksplit <= 1 || (g.part && g.part_capacity >= static_cast<int64_t>(g.M) * g.N * g.batch * p.ksplit);
+        if(shape != pipe::N_SHAPES && p.nsplit <= 0) e.pipelined = prepare_pipelined(oriented(g), shape, slices ? p.ksplit : 1, e.p);
+        cache[ck] = e;
     }
     launch_plan(g, p, stream);
 }
