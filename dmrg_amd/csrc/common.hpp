@@ -101,11 +101,9 @@ struct GemmDesc {
 // Tile configuration id. 64x64, 32x64 and 64x32, 128x64, 32x32 (T32x32K: the same) are shapes of the pipelined kernels
 // (gemm_plan.hpp; 32x64 and 64x32 are one shape, its long side along consecutive elements of C; types without a shape
 // take the next smaller one); T16x128 is a register-staged kernel.
-// SMALLK: a column-streaming kernel for GEMMs whose K (and M) are tiny, such as the MPO leg of the matvec
-// (K = d * D); it is HBM-bound and skips the tile machinery. GEMMs outside its limits fall back to T64x64.
+// SMALLK: the streaming kernel for tiny K and M (gemm_stream.hip), such as the MPO leg of the matvec (K = d * D); GEMMs
+// outside its limits fall back to T64x64.
 enum class TileCfg : int { T64x64 = 0, T32x64 = 1, T64x32 = 2, T16x128 = 3, T128x64 = 4, T32x32 = 5, SMALLK = 6, T32x32K = 7, AUTO = -1 };
-constexpr int SMALLK_MAX_K = 32;
-constexpr int SMALLK_MAX_M = 64;
 
 // Launch one GEMM. cfg/ksplit = AUTO/0 pick from the tuning table or the size heuristic.
 void gemm(const GemmDesc &g, hipStream_t stream, TileCfg cfg = TileCfg::AUTO, int ksplit = 0);

@@ -220,23 +220,25 @@ void env_build_block(dmrg_dtype t, char side, const Dims &D, void *out, const vo
     } else if(side == 'R') {
         // R'[a,a',w] = sum theta[s,a,b] R[b,b',w'] W[w,w',s,s'] conj theta[s',a',b']   (EnvBase.cpp:146-149)
         void *X = w0;                                       // X[s',a',b,w']  (d*chiL) x (chiR*DR)
-        void *Y = w0 + static_cast<size_t>(d * cL * cR * DR) * es; // Y[s,b,a',w]   (d*chiR) x (chiL*DL)
+        void *Y = w0 + static_cast<size_t>(d * cL * cR * DR) * es; // Y[s,a',b,w]   (d*chiL) x (chiR*DL)
         // X[(s',a'),(b,w')] = sum_b' conj theta[s',a',b'] R[b,b',w']      m=(s',a') k=b' n=(b,w')
         GemmDesc e1 = make(t, d * cL, cR * DR, cR, 1);
         e1.A = theta, e1.am = plain(1), e1.ak = plain(d * cL), e1.conjA = 1;
         e1.B = other, e1.bk = plain(cR), e1.bn = fused(1, cR * cR, cR);
         e1.C = X, e1.cm = plain(1), e1.cn = plain(d * cL);
         gemm(e1, s);
-        // Y[(s,b),(a',w)] = sum_{s',w'} W[w,w',s,s'] X[s',a',b,w']        m=(s,w) k=(s',w') n=(b,a')
-        GemmDesc e2 = make(t, d * DL, cR * cL, d * DR, 1);
+        // Y[s,a',b,w] = sum_{s',w'} W[w,w',s,s'] X[s',a',b,w']            m=(s,w) k=(s',w') n=(a',b)
+        // Y keeps X's order of a' and b, so that the leg reads and writes memory in order (with Y[s,b,a',w] it read X
+        // across its lines: chi = 201x164, D = 25 real 22.8 us, 16.2 here).
+        GemmDesc e2 = make(t, d * DL, cL * cR, d * DR, 1);
         e2.A = mpo, e2.am = fused(DL * DR, 1, d), e2.ak = fused(DL * DR * d, DL, d);
-        e2.B = X, e2.bk = fused(1, d * cL * cR, d), e2.bn = fused(d * cL, d, cR);
-        e2.C = Y, e2.cm = fused(1, d * cR * cL, d), e2.cn = fused(d, d * cR, cR);
+        e2.B = X, e2.bk = fused(1, d * cL * cR, d), e2.bn = plain(d);
+        e2.C = Y, e2.cm = fused(1, d * cL * cR, d), e2.cn = plain(d);
         gemm(e2, s);
-        // R'[a,(a',w)] = sum_{(s,b)} theta[s,a,b] Y[(s,b),(a',w)]          m=a k=(s,b) n=(a',w)
+        // R'[a,(a',w)] = sum_{(s,b)} theta[s,a,b] Y[s,a',b,w]              m=a k=(s,b) n=(a',w)
         GemmDesc e3 = make(t, cL, cL * DL, d * cR, 1);
         e3.A = theta, e3.am = plain(d), e3.ak = fused(1, d * cL, d);
-        e3.B = Y, e3.bk = plain(1), e3.bn = plain(d * cR);
+        e3.B = Y, e3.bk = fused(1, d * cL, d), e3.bn = fused(d, d * cL * cR, cL);
         e3.C = out, e3.cm = plain(1), e3.cn = plain(cL);
         e3.part = w0 + static_cast<size_t>(d * cL * cR * (DL + DR)) * es, e3.part_capacity = MAX_KSPLIT * cL * cL * DL;
         gemm(e3, s);

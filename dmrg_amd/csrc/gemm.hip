@@ -20,6 +20,7 @@
 // the epilogue stores are coalesced either way.
 #include "common.hpp"
 #include "gemm_plan.hpp"
+#include "gemm_stream.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -441,54 +442,6 @@ __global__ __launch_bounds__(64 * WM *WN) void gemm_grouped_kernel(const GemmDes
     gemm_body<R, CPLX, BM, BN, BK, WM, WN, SWAP, ALIGNED>(descs[lo], x - tile_start[lo], 0, 0);
 }
 
-// GEMM with tiny K and M (K <= SMALLK_MAX_K, M <= SMALLK_MAX_M): A sits in LDS, every thread streams one column
-// n of B (K elements, kept in registers) and writes the M elements of C's column n. Consecutive threads take
-// consecutive n, so B and C are read and written along their n index maps; the kernel is HBM-bound.
-template <typename R, bool CPLX, int KMAX>
-__global__ __launch_bounds__(256) void smallk_kernel(const GemmDesc g) {
-    using E = elem_t<R, CPLX>;
-    __shared__ E As[SMALLK_MAX_M * SMALLK_MAX_K];
-    const int    b  = blockIdx.y;
-    const E     *A  = static_cast<const E *>(g.A) + b * g.a_batch;
-    const E     *B  = static_cast<const E *>(g.B) + b * g.b_batch;
-    E           *C  = static_cast<E *>(g.C) + b * g.c_batch;
-    for(int t = threadIdx.x; t < g.M * g.K; t += blockDim.x) {
-        const int m = t % g.M, k = t / g.M;
-        As[t]       = conj_elem(A[idx_off(g.am, m) + idx_off(g.ak, k)], g.conjA != 0);
-    }
-    __syncthreads();
-    for(int64_t n = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; n < g.N; n += static_cast<int64_t>(gridDim.x) * blockDim.x) {
-        const int64_t boff = idx_off(g.bn, static_cast<uint32_t>(n));
-        const int64_t coff = idx_off(g.cn, static_cast<uint32_t>(n));
-        E             bv[KMAX];
-#pragma unroll
-        for(int k = 0; k < KMAX; ++k)
-            if(k < g.K) bv[k] = conj_elem(B[boff + idx_off(g.bk, k)], g.conjB != 0);
-        for(int m = 0; m < g.M; ++m) {
-            R ar = 0, ai = 0;
-#pragma unroll
-            for(int k = 0; k < KMAX; ++k)
-                if(k < g.K) {
-                    const E a = As[m + g.M * k];
-                    if constexpr(CPLX) {
-                        ar = fma(a.re, bv[k].re, fma(-a.im, bv[k].im, ar));
-                        ai = fma(a.re, bv[k].im, fma(a.im, bv[k].re, ai));
-                    } else {
-                        ar = fma(a, bv[k], ar);
-                    }
-                }
-            E *dst = C + coff + idx_off(g.cm, m);
-            if constexpr(CPLX) {
-                if(g.accumulate) ar += dst->re, ai += dst->im;
-                *dst = E{ar, ai};
-            } else {
-                if(g.accumulate) ar += *dst;
-                *dst = ar;
-            }
-        }
-    }
-}
-
 // Sums the split-K partial slabs in a fixed order and writes C through its index map.
 template <typename E>
 __global__ void splitk_reduce(const GemmDesc g) {
@@ -597,18 +550,21 @@ static pipe::Shape shape_of(TileCfg c, dmrg_dtype t) {
     return s;
 }
 
-// Microseconds that the pipelined kernel takes for g in shape s with ks K slices: a CU's workgroups share its matrix
-// cores, so r of them advance one stage in r stage times of MFMA work, but none of them faster than its own chain of
-// barrier, LDS read and MFMA (about 170 clocks beyond its MFMAs). Within 15 % of the measured times of the matvec legs
-// of chi 24 to 1024 (e.g. FP64 402x165x825: 32x32 tiles 15.7 us, 3 slices 12.5, against 14.6 and 11.9 here).
-static double pipe_cost_us(const GemmDesc &g, pipe::Shape s, int ks) {
+// Microseconds that the pipelined kernel takes for g in shape s with ks K slices, with loads of W bytes per lane: a CU's
+// workgroups share its matrix cores, so r of them advance one stage in r stage times of MFMA work, but none of them faster
+// than its own chain of barrier, LDS read and MFMA (about 170 clocks beyond its MFMAs), and all of them together no faster
+// than their loads, about 17 clocks each. Within 15 % of the measured times of the matvec legs of chi 24 to 1024 (e.g.
+// FP64 402x165x825: 32x32 tiles 15.7 us, 3 slices 12.5, against 14.6 and 11.9 here; 328x5000x200 with 4-byte loads in
+// 32x32 tiles 28.1, with 16-byte loads in 64x64 tiles 21.7, against 26.6 and 19.5).
+static double pipe_cost_us(const GemmDesc &g, pipe::Shape s, int ks, int W) {
     const pipe::ShapeInfo i = pipe::shape_info(g.dtype, s);
     const bool   cplx = dtype_is_complex(g.dtype), sp = dtype_is_single(g.dtype);
     const double clk = 2300.0, cus = device_cu_count();
     const double stages = std::ceil((g.K + i.BK - 1) / i.BK / static_cast<double>(ks));
     const double mfma   = i.TM * i.TN * (i.BK / 4) * (cplx ? 3 : 1) * (sp ? 32.0 : 64.0);
+    const double loads  = (i.BM + i.BN) * i.BK * static_cast<double>(dtype_size(g.dtype)) / (64.0 * W) * 17.0;
     const double tiles  = static_cast<double>((g.M + i.BM - 1) / i.BM) * ((g.N + i.BN - 1) / i.BN) * g.batch * ks;
-    auto         round  = [&](double r) { return stages * std::max(r * mfma * 1.04, mfma + 170.0); };
+    auto         round  = [&](double r) { return stages * std::max({r * mfma * 1.04, r * loads, mfma + 170.0}); };
     const double per_cu = std::ceil(tiles / cus), full = std::floor(per_cu / i.resident), rest = per_cu - full * i.resident;
     double       us     = 3.0 + (full * (round(i.resident) + 1500.0) + (rest > 0 ? round(rest) : 0.0)) / clk;
     const double out    = static_cast<double>(g.M) * g.N * g.batch * static_cast<double>(dtype_size(g.dtype));
@@ -624,10 +580,12 @@ static std::vector<std::pair<double, LaunchPlan>> ranked_plans(const GemmDesc &g
     for(TileCfg c : {TileCfg::T128x64, TileCfg::T64x64, TileCfg::T64x32, TileCfg::T32x32}) {
         const pipe::Shape s = shape_of(c, g.dtype);
         if((c == TileCfg::T128x64 && s != pipe::S128x64) || (c == TileCfg::T64x32 && s != pipe::S64x32)) continue;
-        const int bk = pipe::shape_info(g.dtype, s).BK;
+        const int    bk = pipe::shape_info(g.dtype, s).BK;
+        pipe::Launch l;
+        const int    W = pipe::describe(g, pipe::shape_info(g.dtype, s), 1, l) ? l.W : 4;
         for(int ks : {1, 2, 3, 4, 6, 8}) {
             if(ks > 1 && (g.K < 4 * bk * ks || !g.part || g.part_capacity < static_cast<int64_t>(g.M) * g.N * g.batch * ks)) continue;
-            v.emplace_back(pipe_cost_us(g, s, ks), LaunchPlan{c, ks});
+            v.emplace_back(pipe_cost_us(g, s, ks, W), LaunchPlan{c, ks});
         }
     }
     std::stable_sort(v.begin(), v.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
@@ -635,6 +593,8 @@ static std::vector<std::pair<double, LaunchPlan>> ranked_plans(const GemmDesc &g
 }
 
 static LaunchPlan heuristic_plan(const GemmDesc &g) {
+    // The streaming kernel where the columns dominate: below 8 columns per row the tiles' reuse of B is worth more.
+    if((g.M <= 16 || g.N >= 8 * g.M) && stream::takes(g)) return LaunchPlan{TileCfg::SMALLK, 1};
     if(g.M <= 16) return LaunchPlan{TileCfg::T16x128, 1};
     return ranked_plans(g).front().second;
 }
@@ -726,18 +686,10 @@ static void launch_typed(const GemmDesc &g, TileCfg cfg, bool swap, hipStream_t 
     constexpr int E  = static_cast<int>(sizeof(elem_t<R, CPLX>));
     constexpr int BK = E == 4 ? 32 : 16;
     constexpr int BH = E == 16 ? 8 : BK;
-    if(cfg == TileCfg::SMALLK && (g.K > SMALLK_MAX_K || g.M > SMALLK_MAX_M)) cfg = TileCfg::T64x64;
+    if(cfg == TileCfg::SMALLK && !stream::takes(g)) cfg = TileCfg::T64x64;
     switch(cfg) {
         case TileCfg::T16x128: launch_cfg<R, CPLX, 16, 128, BH, 1, 4>(g, swap, s); break;
-        case TileCfg::SMALLK: {
-            const int64_t blocks = std::min<int64_t>((static_cast<int64_t>(g.N) + 255) / 256, 8192);
-            const dim3    grid(static_cast<unsigned>(blocks), g.batch);
-            if(g.K <= 8) hipLaunchKernelGGL((smallk_kernel<R, CPLX, 8>), grid, dim3(256), 0, s, g);
-            else if(g.K <= 16) hipLaunchKernelGGL((smallk_kernel<R, CPLX, 16>), grid, dim3(256), 0, s, g);
-            else hipLaunchKernelGGL((smallk_kernel<R, CPLX, SMALLK_MAX_K>), grid, dim3(256), 0, s, g);
-            if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
-            break;
-        }
+        case TileCfg::SMALLK: stream::launch(g, device_cu_count(), s); break;
         case TileCfg::AUTO: throw Error(DMRG_ERR_ARG, "bad tile config");
         default: {
             const dim3 grid(((g.M + 63) / 64) * ((g.N + 63) / 64), g.ksplit, g.batch), block(256);
@@ -966,7 +918,7 @@ void grouped_free(std::vector<GroupedGemm> &gg) {
 
 static std::vector<LaunchPlan> candidates(const GemmDesc &g) {
     std::vector<LaunchPlan> c;
-    if(g.K <= SMALLK_MAX_K && g.M <= SMALLK_MAX_M) c.push_back({TileCfg::SMALLK, 1});
+    if(stream::takes(g)) c.push_back({TileCfg::SMALLK, 1});
     if(g.M <= 32) c.push_back({TileCfg::T16x128, 1});
     // The pipelined plans within a third of the cheapest.
     const auto ranked = ranked_plans(g);
@@ -995,33 +947,36 @@ static LaunchPlan tune(const GemmDesc &g, hipStream_t stream) {
     hipEvent_t e0, e1;
     DMRG_HIP_CHECK(hipEventCreate(&e0));
     DMRG_HIP_CHECK(hipEventCreate(&e1));
-    LaunchPlan best = heuristic_plan(g);
-    float      best_ms = 1e30f;
+    std::vector<float> t(cands.size(), 1e30f);
     try {
-        for(const auto &p : cands) {
-            launch_plan(g, p, stream); // warm-up (first-use code load, caches)
-            // Fastest of 5 timed launches, so that one launch slowed by a clock change does not decide the plan
-            // (with the mean of 3 launches, the MPO leg at chi = 512 went to a plan 20 % slower in some runs).
-            float tmin = 1e30f;
-            for(int r = 0; r < 5; ++r) {
-                DMRG_HIP_CHECK(hipEventRecord(e0, stream));
-                launch_plan(g, p, stream);
-                DMRG_HIP_CHECK(hipEventRecord(e1, stream));
-                DMRG_HIP_CHECK(hipEventSynchronize(e1));
-                float ms = 0;
-                DMRG_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
-                tmin = std::min(tmin, ms);
+        // Two passes over the candidates, the fastest of 3 launches in each: the clocks move by several per cent within
+        // one pass.
+        for(int pass = 0; pass < 2; ++pass)
+            for(size_t c = 0; c < cands.size(); ++c) {
+                if(pass == 0) launch_plan(g, cands[c], stream); // warm-up (first-use code load, caches)
+                for(int r = 0; r < 3; ++r) {
+                    DMRG_HIP_CHECK(hipEventRecord(e0, stream));
+                    launch_plan(g, cands[c], stream);
+                    DMRG_HIP_CHECK(hipEventRecord(e1, stream));
+                    DMRG_HIP_CHECK(hipEventSynchronize(e1));
+                    float ms = 0;
+                    DMRG_HIP_CHECK(hipEventElapsedTime(&ms, e0, e1));
+                    t[c] = std::min(t[c], ms);
+                }
             }
-            if(tmin < best_ms) {
-                best_ms = tmin;
-                best    = p;
-            }
-        }
     } catch(...) {
         (void) hipEventDestroy(e0);
         (void) hipEventDestroy(e1);
         throw;
     }
+    // The fastest, but an earlier candidate (they are in the model's order) that is within 2 % of it.
+    const float fastest = *std::min_element(t.begin(), t.end());
+    LaunchPlan  best    = cands[0];
+    for(size_t c = 0; c < cands.size(); ++c)
+        if(t[c] <= 1.02f * fastest) {
+            best = cands[c];
+            break;
+        }
     (void) hipEventDestroy(e0);
     (void) hipEventDestroy(e1);
     return best;

@@ -491,7 +491,7 @@ dmrg_status dmrg_autotune_reset(void);
 dmrg_status dmrg_autotune_min_macs(int64_t macs);
 int         dmrg_autotune_entries(void);
 /* Testing hook: force every GEMM to tile configuration cfg (0..5: 64x64, 32x64, 64x32, 16x128, 128x64, 32x32;
- * 6: the column-streaming kernel for tiny K, which falls back to 64x64 beyond K = 32 or M = 64; 7: as 5; 1 and 2
+ * 6: the streaming kernel for tiny K, which falls back to 64x64 beyond K = 64 or M = 64; 7: as 5; 1 and 2
  * are one shape, its long side along consecutive outputs) with up to ksplit K slices; cfg < 0 restores the
  * tuned/heuristic choice. */
 dmrg_status dmrg_gemm_plan_override(int cfg, int ksplit);

@@ -85,3 +85,24 @@ def test_operands_off_16_byte_alignment(dtype, off):
         for p in bufs:
             _lib.call("dmrg_free", p)
     assert rel(out, ref) <= (TOL64 if np.dtype(dtype).itemsize // (2 if np.issubdtype(dtype, np.complexfloating) else 1) == 8 else TOL32)
+
+
+# The streaming kernel of the MPO leg (M = d D', K = d D): row blocks of 16 and K steps of 4 and their remainders, the
+# largest sizes it takes (64) and the next ones, columns around one block and one workgroup (16, 64).
+@pytest.mark.parametrize("d,DL,DR", [(1, 1, 1), (1, 2, 5), (2, 2, 8), (2, 6, 3), (3, 3, 5), (2, 8, 9), (4, 8, 8), (2, 16, 17), (2, 25, 25), (2, 32, 32),
+                                     (2, 33, 32), (4, 16, 16)])
+def test_streaming_leg_edges(d, DL, DR):
+    _lib.call("dmrg_gemm_plan_override", 6, 1)
+    try:
+        rng = np.random.default_rng(d * 1000 + DL * 10 + DR)
+        for chiL, chiR in ((1, 1), (3, 5), (4, 4), (17, 8), (9, 23)):
+            for cplx in (False, True):
+                print(f"[case] d={d} D={DL},{DR} chi={chiL}x{chiR} cplx={cplx}", file=sys.stderr, flush=True)
+                th, W, L, R = general(rng, d, chiL, chiR, DL, DR, cplx)
+                ref = O.matrix_vector_product(th, W, L, R)
+                assert rel(G.matrix_vector_product(th, W, L, R), ref) <= TOL64
+                assert rel(G.matrix_vector_product(single(th), single(W), single(L), single(R)), ref) <= TOL32
+                for side, E in (("L", L), ("R", R)):
+                    assert rel(G.env_build_block(side, E, th, W), O.env_build_block(side, E, th, W)) <= TOL64
+    finally:
+        _lib.call("dmrg_gemm_plan_override", -1, 0)
