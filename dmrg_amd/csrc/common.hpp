@@ -119,23 +119,29 @@ struct NoTuneScope {
     bool prev_;
 };
 
-// Grouped GEMM: independent GEMMs (batch 1, no split-K) of one tile configuration run as one launch. The
-// descriptors and the tile prefix sums are device arrays filled by grouped_prepare (one group per
-// (swap, aligned) kind of GEMM); they stay valid as long as the GEMMs' buffers do, so a grouped launch can be
-// captured into a graph and replayed. Tile configurations: T64x64, T32x32, T16x128.
+// Grouped GEMM: independent GEMMs (batch 1, no split-K) run in one launch per kind of kernel. The descriptions and
+// the first workgroups are device arrays filled by grouped_prepare; they stay valid as long as the GEMMs' buffers do, so a
+// grouped launch can be captured into a graph and replayed. Tile configurations: T64x64, T32x32, or SMALLK (the streaming
+// kernel for the GEMMs it takes, T32x32 for the others).
 struct GroupedGemm {
-    dmrg_dtype dtype   = DMRG_FP64;
-    TileCfg    cfg     = TileCfg::T64x64;
-    bool       swap    = false;
-    bool       aligned = false;
-    int        ngemm   = 0;
-    int        tiles   = 0;
-    void      *descs   = nullptr; // device, ngemm GemmDesc
-    int       *starts  = nullptr; // device, ngemm + 1 tile offsets
-    bool       owned   = true;    // descs/starts allocated by grouped_prepare (else inside a caller's store)
+    // PIPELINED: tiles of the pipelined kernel; STREAMED: the streaming kernel; STAGED: 64x64 tiles of the register-staged
+    // kernel, for the index maps that the pipelined kernel does not take.
+    enum Kind { PIPELINED, STREAMED, STAGED, STAGED_SWAPPED, N_KINDS };
+    dmrg_dtype dtype      = DMRG_FP64;
+    Kind       kind       = PIPELINED;
+    TileCfg    cfg        = TileCfg::T64x64;
+    int        ngemm      = 0;
+    int        workgroups = 0;
+    int        max_k      = 0;
+    size_t     lds        = 0;       // STREAMED: LDS bytes of a workgroup
+    void      *descs      = nullptr; // device, ngemm descriptions
+    int       *starts     = nullptr; // device, ngemm + 1 first workgroups
+    bool       owned      = true;    // descs/starts allocated by grouped_prepare (else inside a caller's store)
 };
 // Tiles of g under configuration cfg.
 int grouped_tiles(const GemmDesc &g, TileCfg cfg);
+// Whether the streaming kernel takes g.
+bool grouped_streams(const GemmDesc &g);
 // Whether GEMM plans are tuned by timing (dmrg_autotune_enable).
 int autotune_enabled();
 

@@ -427,19 +427,11 @@ __global__ __launch_bounds__(64 * WM *WN) void gemm_kernel(const GemmDesc g) {
     gemm_body<R, CPLX, BM, BN, BK, WM, WN, SWAP, ALIGNED>(g, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// Grouped GEMM: one launch for several independent GEMMs of one tile configuration. Workgroup x belongs to
-// the GEMM whose tile range [tile_start[i], tile_start[i + 1]) holds x (no split-K, batch 1 each); the
-// descriptors and the prefix sums live in device memory, so a launch can be captured once and replayed.
-template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, bool SWAP, bool ALIGNED>
+// Grouped launches of the GEMMs that the pipelined kernel does not take (gemm_pipe.hpp holds its grouped form).
+template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, bool SWAP>
 __global__ __launch_bounds__(64 * WM *WN) void gemm_grouped_kernel(const GemmDesc *descs, const int *tile_start, int ngemm) {
-    const int x  = blockIdx.x;
-    int       lo = 0, hi = ngemm - 1; // last i with tile_start[i] <= x
-    while(lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if(tile_start[mid] <= x) lo = mid;
-        else hi = mid - 1;
-    }
-    gemm_body<R, CPLX, BM, BN, BK, WM, WN, SWAP, ALIGNED>(descs[lo], x - tile_start[lo], 0, 0);
+    const int i = pipe::group_of(tile_start, ngemm, blockIdx.x);
+    gemm_body<R, CPLX, BM, BN, BK, WM, WN, SWAP, false>(descs[i], blockIdx.x - tile_start[i], 0, 0);
 }
 
 // Sums the split-K partial slabs in a fixed order and writes C through its index map.
@@ -785,123 +777,152 @@ static void launch_plan_single(GemmDesc g, const LaunchPlan &p0, hipStream_t str
 // ---------------------------------------------------------------------------------------
 // Grouped launches
 
-static int group_bk(dmrg_dtype t, TileCfg cfg) {
-    const int e = static_cast<int>(dtype_size(t));
-    const int bk = e == 4 ? 32 : 16;
-    return (cfg == TileCfg::T16x128 || cfg == TileCfg::T128x64) && e == 16 ? 8 : bk;
-}
-
 int grouped_tiles(const GemmDesc &g, TileCfg cfg) {
     const CfgShape sh = cfg_shape(cfg);
     return ((g.M + sh.BM - 1) / sh.BM) * ((g.N + sh.BN - 1) / sh.BN);
 }
 
-// Four launch kinds at most, each with ngemm descriptors and ngemm + 1 starts, 256-byte aligned.
+bool grouped_streams(const GemmDesc &g) { return stream::takes(g); }
+
+// At most four launches (GroupedGemm::Kind), each with its GEMMs' descriptions and their first workgroups, 256-byte aligned.
+static size_t    aligned256(size_t b) { return (b + 255) / 256 * 256; }
+constexpr size_t GROUP_DESC_MAX = std::max({sizeof(GemmDesc), sizeof(pipe::Desc), sizeof(stream::Desc)});
 size_t grouped_store_bytes(size_t ngemm) {
-    auto al = [](size_t b) { return (b + 255) / 256 * 256; };
-    return 4 * (al(sizeof(GemmDesc) * ngemm) + al(sizeof(int) * (ngemm + 1)));
+    return aligned256(GROUP_DESC_MAX * ngemm) + aligned256(sizeof(int) * (ngemm + 4)) + 8 * 256;
 }
+
+namespace {
+// The GEMMs of one launch: descriptions as bytes, and their first workgroups.
+struct GroupBuilder {
+    std::vector<char> descs;
+    std::vector<int>  starts{0};
+    int               max_k = 0;
+    size_t            lds   = 0;
+
+    template <typename D>
+    void add(const D &d, int64_t workgroups, int K, size_t lds_bytes = 0) {
+        const int64_t next = static_cast<int64_t>(starts.back()) + workgroups;
+        DMRG_REQUIRE(next < (int64_t(1) << 31), DMRG_ERR_DIMS, "grouped GEMM: too many tiles");
+        starts.push_back(static_cast<int>(next));
+        const char *p = reinterpret_cast<const char *>(&d);
+        descs.insert(descs.end(), p, p + sizeof(D));
+        max_k = std::max(max_k, K);
+        lds   = std::max(lds, lds_bytes);
+    }
+};
+} // namespace
 
 std::vector<GroupedGemm> grouped_prepare(const std::vector<GemmDesc> &gs, TileCfg cfg, void *store, size_t store_bytes) {
     DMRG_REQUIRE(!store || store_bytes >= grouped_store_bytes(gs.size()), DMRG_ERR_ARG, "grouped GEMM: descriptor store too small");
-    size_t store_off = 0;
-    DMRG_REQUIRE(cfg == TileCfg::T64x64 || cfg == TileCfg::T32x32 || cfg == TileCfg::T16x128, DMRG_ERR_ARG,
+    DMRG_REQUIRE(cfg == TileCfg::T64x64 || cfg == TileCfg::T32x32 || cfg == TileCfg::SMALLK, DMRG_ERR_ARG,
                  "grouped GEMM: tile configuration not available");
-    const CfgShape sh = cfg_shape(cfg);
-    const int      bk = group_bk(gs.empty() ? DMRG_FP64 : gs[0].dtype, cfg);
-    // (swap, aligned) -> member GEMMs
-    std::vector<GemmDesc> kinds[4];
+    const TileCfg         tiled = cfg == TileCfg::SMALLK ? TileCfg::T32x32 : cfg;
+    std::vector<GemmDesc> members;
+    int64_t               blocks = 0; // 16-column blocks of the streamed GEMMs
     for(GemmDesc g : gs) {
         if(g.M <= 0 || g.N <= 0) continue;
         DMRG_REQUIRE(g.batch == 1 && !g.accumulate && g.K > 0, DMRG_ERR_ARG, "grouped GEMM: batch 1, K > 0, no accumulation");
         DMRG_REQUIRE(g.dtype == gs[0].dtype, DMRG_ERR_ARG, "grouped GEMM: one dtype per group");
         DMRG_REQUIRE(static_cast<int64_t>(g.M) * g.N < (int64_t(1) << 31), DMRG_ERR_DIMS, "gemm: output too large");
-        g.a_fast_m      = fast_score(g.am) >= fast_score(g.ak) ? 1 : 0;
-        g.b_fast_k      = fast_score(g.bk) >= fast_score(g.bn) ? 1 : 0;
         g.ksplit        = 1;
-        g.kchunk        = (g.K + 31) / 32 * 32;
         g.xcd_remap     = 0;
         g.part          = nullptr;
         g.part_capacity = 0;
         g.ev_after_main = nullptr;
+        if(cfg == TileCfg::SMALLK && stream::takes(g)) blocks += (g.N + 15) / 16;
+        members.push_back(g);
+    }
+    // Workgroups start in the order of their numbers: the longest sums first, so that the launch ends evenly.
+    std::stable_sort(members.begin(), members.end(), [](const GemmDesc &a, const GemmDesc &b) { return a.K > b.K; });
+    const int64_t waves = static_cast<int64_t>(device_cu_count()) * 16;
+    GroupBuilder  build[GroupedGemm::N_KINDS];
+    for(GemmDesc &g : members) {
+        if(cfg == TileCfg::SMALLK && stream::takes(g)) {
+            const stream::Desc d = stream::describe(g, std::max<int64_t>(1, waves * ((g.N + 15) / 16) / blocks));
+            build[GroupedGemm::STREAMED].add(d, stream::workgroups(d), g.K, stream::lds_bytes(g));
+            continue;
+        }
+        const GemmDesc    h     = oriented(g);
+        const pipe::Shape shape = shape_of(tiled, g.dtype);
+        pipe::Launch      l;
+        if(pipe::describe(h, pipe::shape_info(g.dtype, shape), 1, l, true)) {
+            build[GroupedGemm::PIPELINED].add(l.d, grouped_tiles(h, tiled), h.K);
+            continue;
+        }
+        g.a_fast_m      = fast_score(g.am) >= fast_score(g.ak) ? 1 : 0;
+        g.b_fast_k      = fast_score(g.bk) >= fast_score(g.bn) ? 1 : 0;
+        g.kchunk        = (g.K + 31) / 32 * 32;
         const bool swap = (g.cm.s0 == 1 && g.cm.c >= 16) && !(g.cn.s0 == 1 && g.cn.c >= 16);
-        const int  es   = static_cast<int>(dtype_size(g.dtype));
-        const bool aligned = separable(g.am, sh.BM) && separable(g.ak, bk) && separable(g.bn, sh.BN) && separable(g.bk, bk) &&
-                             (g.kchunk % bk) == 0 && small_tile_offsets(g.am, sh.BM, g.ak, bk, es) &&
-                             small_tile_offsets(g.bn, sh.BN, g.bk, bk, es);
-        kinds[(swap ? 2 : 0) + (aligned ? 1 : 0)].push_back(g);
+        build[swap ? GroupedGemm::STAGED_SWAPPED : GroupedGemm::STAGED].add(g, grouped_tiles(g, TileCfg::T64x64), g.K);
     }
     std::vector<GroupedGemm> out;
-    for(int k = 0; k < 4; ++k) {
-        if(kinds[k].empty()) continue;
+    size_t                   store_off = 0;
+    for(int k = 0; k < GroupedGemm::N_KINDS; ++k) {
+        const GroupBuilder &b = build[k];
+        if(b.descs.empty()) continue;
         GroupedGemm gg;
-        gg.dtype   = kinds[k][0].dtype;
-        gg.cfg     = cfg;
-        gg.swap    = (k & 2) != 0;
-        gg.aligned = (k & 1) != 0;
-        gg.ngemm   = static_cast<int>(kinds[k].size());
-        std::vector<int> st(gg.ngemm + 1, 0);
-        for(int i = 0; i < gg.ngemm; ++i) {
-            const int64_t next = static_cast<int64_t>(st[i]) + grouped_tiles(kinds[k][i], cfg);
-            DMRG_REQUIRE(next < (int64_t(1) << 31), DMRG_ERR_DIMS, "grouped GEMM: too many tiles");
-            st[i + 1] = static_cast<int>(next);
-        }
-        gg.tiles = st[gg.ngemm];
+        gg.dtype              = members[0].dtype;
+        gg.kind               = static_cast<GroupedGemm::Kind>(k);
+        gg.cfg                = tiled;
+        gg.ngemm              = static_cast<int>(b.starts.size()) - 1;
+        gg.workgroups         = b.starts.back();
+        gg.max_k              = b.max_k;
+        gg.lds                = b.lds;
+        const size_t starts_b = sizeof(int) * b.starts.size();
         if(store) {
-            auto al    = [](size_t b) { return (b + 255) / 256 * 256; };
             char *base = static_cast<char *>(store);
             gg.owned   = false;
             gg.descs   = base + store_off;
-            store_off += al(sizeof(GemmDesc) * gg.ngemm);
+            store_off += aligned256(b.descs.size());
             gg.starts = reinterpret_cast<int *>(base + store_off);
-            store_off += al(sizeof(int) * (gg.ngemm + 1));
-        } else if(hipMalloc(&gg.descs, sizeof(GemmDesc) * gg.ngemm) != hipSuccess ||
-                  hipMalloc(reinterpret_cast<void **>(&gg.starts), sizeof(int) * (gg.ngemm + 1)) != hipSuccess) {
+            store_off += aligned256(starts_b);
+        } else if(hipMalloc(&gg.descs, b.descs.size()) != hipSuccess || hipMalloc(reinterpret_cast<void **>(&gg.starts), starts_b) != hipSuccess) {
             (void) hipGetLastError();
             out.push_back(gg);
             grouped_free(out);
             throw Error(DMRG_ERR_OOM, "grouped GEMM: descriptor allocation failed");
         }
-        DMRG_HIP_CHECK(hipMemcpy(gg.descs, kinds[k].data(), sizeof(GemmDesc) * gg.ngemm, hipMemcpyHostToDevice));
-        DMRG_HIP_CHECK(hipMemcpy(gg.starts, st.data(), sizeof(int) * (gg.ngemm + 1), hipMemcpyHostToDevice));
         out.push_back(gg);
+        DMRG_HIP_CHECK(hipMemcpy(gg.descs, b.descs.data(), b.descs.size(), hipMemcpyHostToDevice));
+        DMRG_HIP_CHECK(hipMemcpy(gg.starts, b.starts.data(), starts_b, hipMemcpyHostToDevice));
     }
     return out;
 }
 
-template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN>
-static void grouped_launch_cfg(const GroupedGemm &g, hipStream_t s) {
-    const dim3 grid(g.tiles), block(64 * WM * WN);
-    const auto *d = static_cast<const GemmDesc *>(g.descs);
-    if(g.aligned) {
-        if(g.swap) hipLaunchKernelGGL((gemm_grouped_kernel<R, CPLX, BM, BN, BK, WM, WN, true, true>), grid, block, 0, s, d, g.starts, g.ngemm);
-        else hipLaunchKernelGGL((gemm_grouped_kernel<R, CPLX, BM, BN, BK, WM, WN, false, true>), grid, block, 0, s, d, g.starts, g.ngemm);
-    } else {
-        if(g.swap) hipLaunchKernelGGL((gemm_grouped_kernel<R, CPLX, BM, BN, BK, WM, WN, true, false>), grid, block, 0, s, d, g.starts, g.ngemm);
-        else hipLaunchKernelGGL((gemm_grouped_kernel<R, CPLX, BM, BN, BK, WM, WN, false, false>), grid, block, 0, s, d, g.starts, g.ngemm);
-    }
-}
-
 template <typename R, bool CPLX>
-static void grouped_launch_typed(const GroupedGemm &g, hipStream_t s) {
+static void grouped_staged(const GroupedGemm &g, hipStream_t s) {
     constexpr int E  = static_cast<int>(sizeof(elem_t<R, CPLX>));
     constexpr int BK = E == 4 ? 32 : 16;
-    constexpr int BH = E == 16 ? 8 : BK;
-    switch(g.cfg) {
-        case TileCfg::T64x64: grouped_launch_cfg<R, CPLX, 64, 64, BK, 2, 2>(g, s); break;
-        case TileCfg::T32x32: grouped_launch_cfg<R, CPLX, 32, 32, BK, 2, 2>(g, s); break;
-        case TileCfg::T16x128: grouped_launch_cfg<R, CPLX, 16, 128, BH, 1, 4>(g, s); break;
-        default: throw Error(DMRG_ERR_ARG, "grouped GEMM: tile configuration not available");
+    const dim3    grid(g.workgroups), block(256);
+    const auto   *d = static_cast<const GemmDesc *>(g.descs);
+    if(g.kind == GroupedGemm::STAGED_SWAPPED)
+        hipLaunchKernelGGL((gemm_grouped_kernel<R, CPLX, 64, 64, BK, 2, 2, true>), grid, block, 0, s, d, g.starts, g.ngemm);
+    else hipLaunchKernelGGL((gemm_grouped_kernel<R, CPLX, 64, 64, BK, 2, 2, false>), grid, block, 0, s, d, g.starts, g.ngemm);
+}
+
+static void grouped_pipelined(const GroupedGemm &g, hipStream_t s) {
+    const auto       *d     = static_cast<const pipe::Desc *>(g.descs);
+    const pipe::Shape shape = shape_of(g.cfg, g.dtype);
+    switch(g.dtype) {
+        case DMRG_FP64: pipe::launch_grouped_f64(d, g.starts, g.ngemm, g.workgroups, shape, s); break;
+        case DMRG_CX64: pipe::launch_grouped_c128(d, g.starts, g.ngemm, g.workgroups, shape, s); break;
+        case DMRG_FP32: pipe::launch_grouped_f32(d, g.starts, g.ngemm, g.workgroups, shape, s); break;
+        case DMRG_CX32: pipe::launch_grouped_c64(d, g.starts, g.ngemm, g.workgroups, shape, s); break;
     }
 }
 
 void grouped_launch(const GroupedGemm &g, hipStream_t s) {
-    if(g.tiles <= 0) return;
-    switch(g.dtype) {
-        case DMRG_FP64: grouped_launch_typed<double, false>(g, s); break;
-        case DMRG_CX64: grouped_launch_typed<double, true>(g, s); break;
-        case DMRG_FP32: grouped_launch_typed<float, false>(g, s); break;
-        case DMRG_CX32: grouped_launch_typed<float, true>(g, s); break;
+    if(g.workgroups <= 0) return;
+    if(g.kind == GroupedGemm::PIPELINED) grouped_pipelined(g, s);
+    else if(g.kind == GroupedGemm::STREAMED)
+        stream::launch_grouped(g.dtype, static_cast<const stream::Desc *>(g.descs), g.starts, g.ngemm, g.workgroups, g.max_k, g.lds, s);
+    else {
+        switch(g.dtype) {
+            case DMRG_FP64: grouped_staged<double, false>(g, s); break;
+            case DMRG_CX64: grouped_staged<double, true>(g, s); break;
+            case DMRG_FP32: grouped_staged<float, false>(g, s); break;
+            case DMRG_CX32: grouped_staged<float, true>(g, s); break;
+        }
     }
     DMRG_HIP_CHECK(hipGetLastError());
 }

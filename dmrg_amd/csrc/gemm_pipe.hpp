@@ -53,7 +53,19 @@ struct Desc {
     int32_t  M, N;
     int32_t  Kin, stages_per_chunk, stages, stages_per_slice; // stages: Kout chunks of stages_per_chunk
     int32_t  accumulate, ksplit, xcd_remap;
+    int32_t  wide; // loads of 16 bytes per lane (else 4); read by grouped launches only
 };
+
+// The last i with start[i] <= x.
+__device__ __forceinline__ int group_of(const int *start, int n, int x) {
+    int lo = 0, hi = n - 1;
+    while(lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if(start[mid] <= x) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
 
 template <int N, typename F>
 __device__ __forceinline__ void static_for(F &&f) {
@@ -188,8 +200,9 @@ struct alignas(16) Unit {
     E e[16 / sizeof(E)];
 };
 
-template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, int NS, bool AR, bool BR, int W>
-__device__ __forceinline__ void body(const Desc &g, int bx, int split, int b) {
+// stage(i): the LDS memory of stage i (an integral constant), BM BK + BN BK elements.
+template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, int NS, bool AR, bool BR, int W, typename Stage>
+__device__ __forceinline__ void body(const Desc &g, int bx, int split, int b, Stage &&stage) {
     using E            = std::conditional_t<CPLX, cpx<R>, R>;
     using MM           = mma<R>;
     constexpr int U    = 16 / static_cast<int>(sizeof(E));
@@ -202,27 +215,6 @@ __device__ __forceinline__ void body(const Desc &g, int bx, int split, int b) {
     static_assert(!BR || TN % U == 0, "R orientation needs whole units per wave");
     constexpr int LPS = LA::L + LB::L; // loads per wave and stage
     constexpr int DEP = NS - 1;        // stages in flight
-    // One array per stage, so that a fragment read is not taken to alias the loads in flight to the other stages.
-    __shared__ __attribute__((aligned(16))) char S0[LA::BYTES + LB::BYTES];
-    __shared__ __attribute__((aligned(16))) char S1[LA::BYTES + LB::BYTES];
-    __shared__ __attribute__((aligned(16))) char S2[NS > 2 ? LA::BYTES + LB::BYTES : 16];
-    __shared__ __attribute__((aligned(16))) char S3[NS > 3 ? LA::BYTES + LB::BYTES : 16];
-    __shared__ __attribute__((aligned(16))) char S4[NS > 4 ? LA::BYTES + LB::BYTES : 16];
-    __shared__ __attribute__((aligned(16))) char S5[NS > 5 ? LA::BYTES + LB::BYTES : 16];
-    __shared__ __attribute__((aligned(16))) char S6[NS > 6 ? LA::BYTES + LB::BYTES : 16];
-    __shared__ __attribute__((aligned(16))) char S7[NS > 7 ? LA::BYTES + LB::BYTES : 16];
-    auto stage = [&](auto s) -> char * {
-        constexpr int i = decltype(s)::value;
-        if constexpr(i == 0) return S0;
-        else if constexpr(i == 1) return S1;
-        else if constexpr(i == 2) return S2;
-        else if constexpr(i == 3) return S3;
-        else if constexpr(i == 4) return S4;
-        else if constexpr(i == 5) return S5;
-        else if constexpr(i == 6) return S6;
-        else return S7;
-    };
-
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % WM, wn = wave / WM;
     const int lg = lane >> 4, ll = lane & 15;
@@ -273,7 +265,7 @@ __device__ __forceinline__ void body(const Desc &g, int bx, int split, int b) {
             for(int j = 0; j < TN; ++j) acc[c][i][j] = typename MM::acc{0, 0, 0, 0};
     // Single precision: the sums are kept in two levels, of FLUSH rounds of NS stages (128 values of K) and of those,
     // so that the rounding error does not grow with the length of K. Complex matvec at chi = 512, D = 5 against 64 bits:
-    // 1.1e-6 in one level, 5.5e-7 in two of 256 values (7.4e-7 for the register-staged kernels with 8 K slices).
+    // 1.1e-6 in one level, 4.2e-7 in two (7.4e-7 for the register-staged kernels with 8 K slices).
     constexpr bool TWO   = sizeof(R) == 4;
     constexpr int  FLUSH = 128 / (BK * NS) > 0 ? 128 / (BK * NS) : 1;
     typename MM::acc tot[TWO ? NACC : 1][TWO ? TM : 1][TWO ? TN : 1];
@@ -499,9 +491,39 @@ __device__ __forceinline__ void body(const Desc &g, int bx, int split, int b) {
         }
 }
 
+// One array per stage, so that a fragment read is not taken to alias the loads in flight to the other stages.
+#define DMRG_PIPE_STAGES(BYTES, NS)                                                          \
+    __shared__ __attribute__((aligned(16))) char S0[(BYTES)];                                \
+    __shared__ __attribute__((aligned(16))) char S1[(BYTES)];                                \
+    __shared__ __attribute__((aligned(16))) char S2[(NS) > 2 ? (BYTES) : 16];                \
+    __shared__ __attribute__((aligned(16))) char S3[(NS) > 3 ? (BYTES) : 16];                \
+    static_assert((NS) >= 2 && (NS) <= 4, "number of stages");                               \
+    auto stage = [&](auto s) -> char * {                                                     \
+        constexpr int i = decltype(s)::value;                                                \
+        if constexpr(i == 0) return S0;                                                      \
+        else if constexpr(i == 1) return S1;                                                 \
+        else if constexpr(i == 2) return S2;                                                 \
+        else return S3;                                                                      \
+    }
+
 template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, int NS, bool AR, bool BR, int W>
 __global__ __launch_bounds__(64 * WM *WN, 2) void kernel(const Desc g) {
-    body<R, CPLX, BM, BN, BK, WM, WN, NS, AR, BR, W>(g, blockIdx.x, blockIdx.y, blockIdx.z);
+    DMRG_PIPE_STAGES((BM + BN) * BK * static_cast<int>(sizeof(R)) * (CPLX ? 2 : 1), NS);
+    body<R, CPLX, BM, BN, BK, WM, WN, NS, AR, BR, W>(g, blockIdx.x, blockIdx.y, blockIdx.z, stage);
+}
+
+// Several independent GEMMs in one launch: workgroup x belongs to the one whose tile range [start[i], start[i + 1])
+// holds x (one K slice and batch entry each). Units run along K or are loaded by 4 bytes, as each GEMM's description says:
+// one kernel then serves all members of a leg, where the register-staged tiles needed one launch per (orientation,
+// alignment). Bounded by the longest member's chain of K stages: 32 FP64 matvecs of chi 16 to 64, D = 5, take 29 us in three
+// launches of about 10 us, against 79 us in six to seven of 10 to 15 us.
+template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, int NS>
+__global__ __launch_bounds__(64 * WM *WN, 2) void grouped_kernel(const Desc *descs, const int *start, int n) {
+    DMRG_PIPE_STAGES((BM + BN) * BK * static_cast<int>(sizeof(R)) * (CPLX ? 2 : 1), NS);
+    const int  i = group_of(start, n, blockIdx.x);
+    const Desc g = descs[i];
+    if(g.wide) body<R, CPLX, BM, BN, BK, WM, WN, NS, false, false, 16>(g, blockIdx.x - start[i], 0, 0, stage);
+    else body<R, CPLX, BM, BN, BK, WM, WN, NS, false, false, 4>(g, blockIdx.x - start[i], 0, 0, stage);
 }
 
 } // namespace pipe

@@ -13,5 +13,13 @@ void launch_c128(const Launch &l, Shape s, dim3 grid, hipStream_t st) {
     }
 }
 
+void launch_grouped_c128(const Desc *d, const int *start, int n, int tiles, Shape s, hipStream_t st) {
+    switch(s) {
+        case S64x64: launch_grouped_shape<double, true, 64, 64, 8, 2, 2, 4>(d, start, n, tiles, st); break;
+        case S32x32: launch_grouped_shape<double, true, 32, 32, 8, 2, 2, 4>(d, start, n, tiles, st); break;
+        default: throw Error(DMRG_ERR_ARG, "no such grouped tile shape");
+    }
+}
+
 } // namespace pipe
 } // namespace dmrg

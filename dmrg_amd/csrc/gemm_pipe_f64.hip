@@ -14,5 +14,13 @@ void launch_f64(const Launch &l, Shape s, dim3 grid, hipStream_t st) {
     }
 }
 
+void launch_grouped_f64(const Desc *d, const int *start, int n, int tiles, Shape s, hipStream_t st) {
+    switch(s) {
+        case S64x64: launch_grouped_shape<double, false, 64, 64, 16, 2, 2, 4>(d, start, n, tiles, st); break;
+        case S32x32: launch_grouped_shape<double, false, 32, 32, 16, 2, 2, 4>(d, start, n, tiles, st); break;
+        default: throw Error(DMRG_ERR_ARG, "no such grouped tile shape");
+    }
+}
+
 } // namespace pipe
 } // namespace dmrg

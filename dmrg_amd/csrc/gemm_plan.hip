@@ -79,7 +79,7 @@ bool operand(Operand &o, const void *p, int64_t batch, const Idx2 &r, const Idx2
 
 } // namespace
 
-bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out) {
+bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bool k_units) {
     const int  es = static_cast<int>(dtype_size(g.dtype)), u = 16 / es;
     const Idx2 am = normal(g.am, g.M), ak = normal(g.ak, g.K), bk = normal(g.bk, g.K), bn = normal(g.bn, g.N);
     for(const Idx2 &x : {am, ak, bk, bn})
@@ -98,7 +98,7 @@ bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out) {
     // Orientation: along K where units are contiguous there, else along the non-K index; else loads of 4 bytes.
     auto along_k = [&](const Idx2 &k, int64_t in) { return u == 1 || (w.nin % u == 0 && (w.ratio ? unit_run(k, g.K, u) : in == 1)); };
     const bool aK = along_k(ak, w.a_in), bK = along_k(bk, w.b_in);
-    const bool aR = s.TM % u == 0 && unit_run(am, g.M, u), bR = s.TN % u == 0 && unit_run(bn, g.N, u);
+    const bool aR = !k_units && s.TM % u == 0 && unit_run(am, g.M, u), bR = !k_units && s.TN % u == 0 && unit_run(bn, g.N, u);
     out.W  = (aK || aR) && (bK || bR) && reinterpret_cast<uintptr_t>(g.A) % 4 == 0 && reinterpret_cast<uintptr_t>(g.B) % 4 == 0 ? 16 : 4;
     out.ar = out.W == 16 && !aK;
     out.br = out.W == 16 && !bK;
@@ -114,6 +114,7 @@ bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out) {
     d.N                = g.N;
     d.accumulate       = g.accumulate;
     d.xcd_remap        = g.xcd_remap;
+    d.wide             = out.W == 16;
     d.Kin              = static_cast<int32_t>(w.nin);
     d.stages_per_chunk = static_cast<int32_t>((w.nin + s.BK - 1) / s.BK);
     const int64_t st   = d.stages_per_chunk * w.nout;

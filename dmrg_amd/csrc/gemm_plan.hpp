@@ -41,12 +41,24 @@ struct Launch {
 };
 // Describes g (already oriented: consecutive m should be consecutive in C) for a tile shape; false where the pipelined
 // kernel does not take it (negative strides, K chunks that differ between the operands, operand tiles spanning 2 GiB).
-bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out);
+// k_units: units along K only, as grouped launches take them.
+bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bool k_units = false);
 // Launches on the grid of l.d.
 void launch_f64(const Launch &l, Shape s, dim3 grid, hipStream_t st);
 void launch_c128(const Launch &l, Shape s, dim3 grid, hipStream_t st);
 void launch_f32(const Launch &l, Shape s, dim3 grid, hipStream_t st);
 void launch_c64(const Launch &l, Shape s, dim3 grid, hipStream_t st);
+
+// Grouped launches: n descriptions and n + 1 tile offsets in device memory.
+void launch_grouped_f64(const Desc *d, const int *start, int n, int tiles, Shape s, hipStream_t st);
+void launch_grouped_c128(const Desc *d, const int *start, int n, int tiles, Shape s, hipStream_t st);
+void launch_grouped_f32(const Desc *d, const int *start, int n, int tiles, Shape s, hipStream_t st);
+void launch_grouped_c64(const Desc *d, const int *start, int n, int tiles, Shape s, hipStream_t st);
+
+template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, int NS>
+void launch_grouped_shape(const Desc *d, const int *start, int n, int tiles, hipStream_t st) {
+    hipLaunchKernelGGL((grouped_kernel<R, CPLX, BM, BN, BK, WM, WN, NS>), dim3(tiles), dim3(64 * WM * WN), 0, st, d, start, n);
+}
 
 template <typename R, bool CPLX, int BM, int BN, int BK, int WM, int WN, int NS>
 void launch_shape(const Launch &l, dim3 grid, hipStream_t st) {

@@ -18,42 +18,28 @@
 
 namespace dmrg {
 namespace stream {
-namespace {
-
 constexpr uint32_t PLAIN = 0x7fffffffu;
 
 // MFMA steps over K, at least two (the divisions by multiplication below have no divisor 1).
 __host__ __device__ inline int ksteps(int K) { return K <= 8 ? 2 : (K + 3) / 4; }
 
-struct Desc {
-    const void *A, *B;
-    void       *C;
-    Idx2        am, ak;                 // element strides
-    int64_t     a_batch, b_batch, c_batch; // bytes for b_batch, elements otherwise
-    Idx2        bk, bn;                 // byte strides
-    Idx2        cm, cn;                 // element strides
-    uint32_t    nmul, nsh, cmul, csh;   // i / bn.c and i / cn.c for i < 2^31
-    uint32_t    mmul, msh, kmul, ksh, qmul, qsh; // i / am.c, i / ak.c and i / (K steps)
-    int32_t     M, N, K, blocks, per_wave;
-    float       sa, sb;                 // -1: conjugate
-};
+namespace {
 
 template <typename R>
 using acc_t = typename pipe::mma<R>::acc;
 
+// Workgroup x of a GEMM, batch entry b. lds: A's fragments [16-row block][K step][lane], then the row offsets of C.
 template <typename R, bool CPLX, int KST>
-__global__ __launch_bounds__(256) void kernel(const Desc g) {
+__device__ __forceinline__ void body(const Desc &g, int x, int b, char *lds) {
     using E  = std::conditional_t<CPLX, cpx<R>, R>;
     using MM = pipe::mma<R>;
-    // Fragments of A: [16-row block][K step][lane], then the row offsets of C.
-    extern __shared__ __attribute__((aligned(16))) char lds[];
-    const int b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, lg = lane >> 4, ll = lane & 15;
+    const int tid = threadIdx.x, lane = tid & 63, lg = lane >> 4, ll = lane & 15;
     const int mb = (g.M + 15) / 16, kst = ksteps(g.K);
     E        *fa   = reinterpret_cast<E *>(lds);
     int64_t  *coff = reinterpret_cast<int64_t *>(lds + static_cast<size_t>(mb) * kst * 64 * sizeof(E));
     const E  *A    = static_cast<const E *>(g.A) + b * g.a_batch;
     const int wave = static_cast<int>(pipe::uni(static_cast<uint32_t>(tid >> 6)));
-    const int first = (blockIdx.x * 4 + wave) * g.per_wave, last = min(g.blocks, first + g.per_wave);
+    const int first = (x * 4 + wave) * g.per_wave, last = min(g.blocks, first + g.per_wave);
 
     const auto rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(static_cast<const char *>(g.B) + b * g.b_batch), static_cast<short>(0),
                                                       0x7fffffff, 0x00020000);
@@ -150,6 +136,20 @@ __global__ __launch_bounds__(256) void kernel(const Desc g) {
     }
 }
 
+template <typename R, bool CPLX, int KST>
+__global__ __launch_bounds__(256) void kernel(const Desc g) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    body<R, CPLX, KST>(g, blockIdx.x, blockIdx.y, lds);
+}
+// Several independent GEMMs in one launch; workgroup x belongs to the one whose range [start[i], start[i + 1]) holds x.
+template <typename R, bool CPLX, int KST>
+__global__ __launch_bounds__(256) void grouped_kernel(const Desc *descs, const int *start, int n) {
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    const int  i = pipe::group_of(start, n, blockIdx.x);
+    const Desc g = descs[i];
+    body<R, CPLX, KST>(g, blockIdx.x - start[i], 0, lds);
+}
+
 Idx2 normal(Idx2 x, int64_t ext) {
     if(x.c == 1) x = Idx2{x.s1, 0, PLAIN};
     if(ext <= static_cast<int64_t>(x.c) || x.s1 == x.s0 * static_cast<int64_t>(x.c)) x = Idx2{x.s0, 0, PLAIN};
@@ -171,10 +171,17 @@ void run(const Desc &d, dim3 grid, size_t lds, hipStream_t s) {
     else if(d.K <= 32) hipLaunchKernelGGL((kernel<R, CPLX, 8>), grid, dim3(256), lds, s, d);
     else hipLaunchKernelGGL((kernel<R, CPLX, 16>), grid, dim3(256), lds, s, d);
 }
+template <typename R, bool CPLX>
+void run_grouped(const Desc *d, const int *start, int n, int groups, int max_k, size_t lds, hipStream_t s) {
+    const dim3 grid(groups), block(256);
+    if(max_k <= 16) hipLaunchKernelGGL((grouped_kernel<R, CPLX, 4>), grid, block, lds, s, d, start, n);
+    else if(max_k <= 32) hipLaunchKernelGGL((grouped_kernel<R, CPLX, 8>), grid, block, lds, s, d, start, n);
+    else hipLaunchKernelGGL((grouped_kernel<R, CPLX, 16>), grid, block, lds, s, d, start, n);
+}
 
 } // namespace
 
-static size_t lds_bytes(const GemmDesc &g) {
+size_t lds_bytes(const GemmDesc &g) {
     return static_cast<size_t>((g.M + 15) / 16) * (static_cast<size_t>(ksteps(g.K)) * 64 * dtype_size(g.dtype) + 16 * sizeof(int64_t));
 }
 
@@ -186,7 +193,7 @@ bool takes(const GemmDesc &g) {
     return (span(normal(g.bk, g.K), g.K) + span(normal(g.bn, g.N), g.N) + 1) * es < static_cast<int64_t>(0x7fffffff);
 }
 
-void launch(const GemmDesc &g, int cus, hipStream_t s) {
+Desc describe(const GemmDesc &g, int64_t waves) {
     const int64_t es = static_cast<int64_t>(dtype_size(g.dtype));
     Desc          d;
     d.A = g.A, d.B = g.B, d.C = g.C;
@@ -203,10 +210,15 @@ void launch(const GemmDesc &g, int cus, hipStream_t s) {
     d.M = g.M, d.N = g.N, d.K = g.K;
     d.sa = g.conjA ? -1.0f : 1.0f, d.sb = g.conjB ? -1.0f : 1.0f;
     d.blocks = (g.N + 15) / 16;
-    // Enough workgroups to fill every CU with as many wavefronts as it holds, each wavefront walking consecutive columns.
-    const int64_t waves = static_cast<int64_t>(cus) * 16;
     d.per_wave          = static_cast<int32_t>(std::max<int64_t>(1, (static_cast<int64_t>(d.blocks) * g.batch + waves - 1) / waves));
-    const dim3   grid(static_cast<unsigned>((d.blocks + 4 * d.per_wave - 1) / (4 * d.per_wave)), g.batch);
+    return d;
+}
+int workgroups(const Desc &d) { return (d.blocks + 4 * d.per_wave - 1) / (4 * d.per_wave); }
+
+void launch(const GemmDesc &g, int cus, hipStream_t s) {
+    // Enough workgroups to fill every CU with as many wavefronts as it holds, each wavefront walking consecutive columns.
+    const Desc d = describe(g, static_cast<int64_t>(cus) * 16);
+    const dim3 grid(static_cast<unsigned>(workgroups(d)), g.batch);
     const size_t lds = lds_bytes(g);
     switch(g.dtype) {
         case DMRG_FP64: run<double, false>(d, grid, lds, s); break;
@@ -215,6 +227,15 @@ void launch(const GemmDesc &g, int cus, hipStream_t s) {
         case DMRG_CX32: run<float, true>(d, grid, lds, s); break;
     }
     if(g.ev_after_main) DMRG_HIP_CHECK(hipEventRecord(static_cast<hipEvent_t>(g.ev_after_main), s));
+}
+
+void launch_grouped(dmrg_dtype t, const Desc *d, const int *start, int n, int groups, int max_k, size_t lds, hipStream_t s) {
+    switch(t) {
+        case DMRG_FP64: run_grouped<double, false>(d, start, n, groups, max_k, lds, s); break;
+        case DMRG_CX64: run_grouped<double, true>(d, start, n, groups, max_k, lds, s); break;
+        case DMRG_FP32: run_grouped<float, false>(d, start, n, groups, max_k, lds, s); break;
+        case DMRG_CX32: run_grouped<float, true>(d, start, n, groups, max_k, lds, s); break;
+    }
 }
 
 } // namespace stream

@@ -1,6 +1,6 @@
 // Grouped H_eff matvecs (see group.hpp). The three legs of every operator's matvec are the GEMMs matvec()
 // launches one by one; here leg j of all k operators goes into one grouped launch, so k small problems that
-// each fill a few CUs share the whole GPU in 3 launches (plus at most 3 more when the GEMMs differ in kind).
+// each fill a few CUs share the whole GPU in 3 launches (more where a leg's GEMMs need different kernels).
 #include "group.hpp"
 
 #include <algorithm>
@@ -58,7 +58,7 @@ TileCfg tuned_leg_cfg(int leg, const std::vector<GemmDesc> &descs, const GroupSt
         DMRG_HIP_CHECK(hipEventCreate(&e0));
         DMRG_HIP_CHECK(hipEventCreate(&e1));
         std::vector<TileCfg> cands = {TileCfg::T64x64, TileCfg::T32x32};
-        if(mmax <= 32) cands.push_back(TileCfg::T16x128);
+        if(std::any_of(descs.begin(), descs.end(), grouped_streams)) cands.push_back(TileCfg::SMALLK);
         for(TileCfg c : cands) {
             std::vector<GroupedGemm> gg = storage ? grouped_prepare(descs, c, storage->stores[leg], storage->store_bytes[leg])
                                                   : grouped_prepare(descs, c);
@@ -130,17 +130,11 @@ MatvecGroup *matvec_group_create(MatVecOp *const *ops, int k, const void *const 
     // path (no caller-owned storage) every stream's work on them must be finished first. The batched engine owns
     // its vectors and synchronises its stream before it rebuilds a group.
     if(!storage && autotune_enabled()) DMRG_HIP_CHECK(hipDeviceSynchronize());
-    // Tiles: the MPO leg (M = d D, K = d D) in 16 x 128 tiles while M is small; the big legs in 64 x 64 tiles
-    // when that gives about two waves of workgroups on the GPU, else in 32 x 32 tiles.
+    // Size rule (used when tuning is off; with tuning the timed fastest): the MPO leg (K and M of d D) streamed, the big
+    // legs in 64x64 tiles when there are enough of them to fill the chip twice, in 32x32 tiles otherwise.
     for(int j = 0; j < 3; ++j) {
-        // Size rule (used when tuning is off): MPO leg with small M in 16x128 tiles, else 64x64 tiles when there
-        // are enough of them to fill the chip twice, 32x32 otherwise; with tuning the timed fastest.
-        TileCfg cfg;
-        if(j == 1) {
-            int mmax = 0;
-            for(const auto &g : leg[j]) mmax = std::max(mmax, g.M);
-            cfg = mmax <= 32 ? TileCfg::T16x128 : TileCfg::T32x32;
-        } else {
+        TileCfg cfg = TileCfg::SMALLK;
+        if(j != 1) {
             int64_t tiles = 0;
             for(const auto &g : leg[j]) tiles += grouped_tiles(g, TileCfg::T64x64);
             cfg = tiles >= 2 * device_cu_count() ? TileCfg::T64x64 : TileCfg::T32x32;
