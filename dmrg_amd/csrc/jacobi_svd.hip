@@ -4,8 +4,8 @@
 // Jacobi keeps high relative accuracy for small singular values.
 //
 // Each sweep runs the n(n-1)/2 pairs in n-1 rounds of disjoint pairs (circle method). When W and V fit in
-// LDS, one workgroup runs every sweep with both matrices resident and a barrier between rounds. Mid-size
-// problems launch one kernel per round with one workgroup (1 to 4 wavefronts, by column length) per pair; large
+// LDS, one workgroup runs every sweep with both matrices resident and a barrier between rounds (up to 128 x 64 the whole
+// SVD is that one launch). Mid-size problems launch one kernel per round with one workgroup (1 to 4 wavefronts, by column length) per pair; large
 // ones pair blocks of 16 columns instead (block one-sided Jacobi, three launches per round of block pairs). The
 // only host round trip per sweep reads whether any rotation was applied.
 #include "svd.hpp"
@@ -27,6 +27,24 @@ template <>
 struct jtraits<cpx<double>> {
     static constexpr bool cx = true;
 };
+
+// |gr + i gi| (gi = 0 for real T) without leaving the range: inner products of columns of norm 1e-130 are 1e-260.
+template <typename T>
+__device__ inline double magnitude(double gr, double gi) {
+    if constexpr(jtraits<T>::cx) return hypot(gr, gi);
+    else return fabs(gr);
+}
+
+// Whether columns of squared norms al and be with inner product g are rotated. A column whose squared norm is zero counts as
+// a zero column, also where rounding has left something below 1e-162 in it: linearly dependent columns shrink by eps a sweep.
+__device__ inline bool rotates(double g, double al, double be, double tol) {
+    const double b = sqrt(al) * sqrt(be);
+    return g > tol * b && b > 0.0;
+}
+// The smaller root of t^2 + 2 z t = 1, of z's sign.
+__device__ inline double tangent(double z) {
+    return fabs(z) > 1e8 ? 0.5 / z : (z >= 0 ? 1.0 : -1.0) / (fabs(z) + sqrt(1.0 + z * z));
+}
 
 __device__ inline double wave_sum(double v) {
 #pragma unroll
@@ -88,12 +106,12 @@ __global__ __launch_bounds__(NT) void jacobi_round(int m, int n, int np, int r, 
 #pragma unroll
         for(int k = 0; k < NT / 64; ++k) al += red[0][k], be += red[1][k], gr += red[2][k], gi += red[3][k];
     }
-    const double g = sqrt(gr * gr + gi * gi);
-    if(!(g > tol * sqrt(al * be)) || g == 0.0) return; // same decision in every thread of the workgroup
+    const double g = magnitude<T>(gr, gi);
+    if(!rotates(g, al, be, tol)) return; // same decision in every thread of the workgroup
     // Align the phase of column q so that the off-diagonal is |g|, then a real rotation zeroes it:
     // t = sign(z) / (|z| + sqrt(1 + z^2)), z = (be - al) / (2 |g|); w_p' = c w_p - s w_q^, w_q' = s w_p + c w_q^.
     const double z  = (be - al) / (2.0 * g);
-    const double t  = (z >= 0 ? 1.0 : -1.0) / (fabs(z) + sqrt(1.0 + z * z));
+    const double t  = tangent(z);
     const double c  = 1.0 / sqrt(1.0 + t * t), s = c * t;
     const double er = gr / g, ei = -gi / g; // e^{-i phi}
     if(tid == 0) atomicOr(flag, 1u);
@@ -218,12 +236,12 @@ __global__ __launch_bounds__(BJ_THREADS) void bj_eig(int n, int nbp, int r, int 
                 double       gr, gi;
                 if constexpr(jtraits<T>::cx) gr = gm.re, gi = gm.im;
                 else gr = gm, gi = 0.0;
-                const double g  = sqrt(gr * gr + gi * gi);
-                const bool   on = g > tol * sqrt(al * be) && g != 0.0;
+                const double g  = magnitude<T>(gr, gi);
+                const bool   on = rotates(g, al, be, tol);
                 ron[tid]        = on ? 1 : 0;
                 if(on) {
                     const double z = (be - al) / (2.0 * g);
-                    const double t = (z >= 0 ? 1.0 : -1.0) / (fabs(z) + sqrt(1.0 + z * z));
+                    const double t = tangent(z);
                     const double c = 1.0 / sqrt(1.0 + t * t);
                     rc[tid]        = c;
                     rs[tid]        = c * t;
@@ -274,6 +292,182 @@ __global__ __launch_bounds__(BJ_THREADS) void bj_eig(int n, int nbp, int r, int 
         T *qo = qbuf + static_cast<int64_t>(blockIdx.x) * B2 * B2;
         for(int idx = tid; idx < B2 * B2; idx += BJ_THREADS) qo[idx] = Qs[idx % B2][idx / B2];
     }
+}
+
+// LDS budget of the single-workgroup paths (gfx950 has 160 KiB per CU).
+constexpr size_t JACOBI_LDS_BYTES = 152 * 1024;
+
+// Sum over the 16 lanes of a row, in all of them, by data-parallel primitives: a step takes two moves and an addition in
+// registers, where a shuffle through LDS takes its latency.
+template <int CTRL>
+__device__ inline double dpp_move(double v) {
+    const auto b  = __builtin_bit_cast(uint64_t, v);
+    const int  lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xf, 0xf, true);
+    const int  hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32 | static_cast<uint32_t>(lo));
+}
+__device__ inline double row_sum(double v) {
+    v += dpp_move<0xb1>(v);  // lane ^ 1
+    v += dpp_move<0x4e>(v);  // lane ^ 2
+    v += dpp_move<0x141>(v); // 7 - lane within 8
+    v += dpp_move<0x140>(v); // 15 - lane within 16
+    return v;
+}
+
+// The whole SVD in one workgroup, W (n columns of up to 16 E rows) and V (n x n, up to 16 EV rows) resident in LDS: loads A
+// (its adjoint where tr), runs all sweeps, sorts and writes U, Vt and S[0:n], and the number of sweeps to S[n]. A row of 16
+// lanes has one pair of a round, with its elements of both columns in registers between the inner products and the
+// rotation; n <= 64 makes at most 32 pairs, so that every row has one pair a round and a barrier ends the round. A round is
+// one serial chain (LDS read, three sums, the rotation's angle, LDS write, barrier), which is what bounds it: hence the
+// sums without LDS and an angle of two dependent roots instead of five roots and quotients. Whole SVDs of a graded
+// spectrum: FP64 64x64 1.65 ms against 5.0 in rounds of block pairs with three launches each, complex 2.65 against 6.1;
+// FP64 32x32 0.32 ms against 1.19 with sums through LDS and the rest in launches of its own.
+template <typename T, int E, int EV>
+__global__ __launch_bounds__(512) void jacobi_resident(int m, int n, int tr, const T *A, double tol, int max_sweeps, T *U, T *Vt, double *S) {
+    constexpr bool cx = jtraits<T>::cx;
+    // 16 doubles of padding: neighbouring columns lie in different halves of the banks (complex rows fill all banks).
+    constexpr int  SW = 16 * E + (cx || E % 2 ? 0 : 16), SV = 16 * EV + (cx || EV % 2 ? 0 : 16);
+    extern __shared__ __attribute__((aligned(16))) unsigned char jacobi_lds_raw[];
+    T             *Ws = reinterpret_cast<T *>(jacobi_lds_raw), *Vs = Ws + n * SW;
+    __shared__ double nrm[64];
+    __shared__ int    perm[64];
+    __shared__ int    rotated;
+    const int tid = threadIdx.x, lane = tid & 15, grp = tid >> 4, np = n + (n & 1);
+    for(int t = tid; t < n * SW; t += blockDim.x) {
+        const int j = t / SW, i = t - j * SW;
+        T         v = jzero<T>();
+        if(i < m) v = tr ? jconj(A[j + static_cast<int64_t>(n) * i]) : A[i + static_cast<int64_t>(m) * j];
+        Ws[t] = v;
+    }
+    for(int t = tid; t < n * SV; t += blockDim.x) Vs[t] = jreal<T>(t / SV == t % SV ? 1.0 : 0.0);
+    int sweep = 0;
+    for(; sweep < max_sweeps; ++sweep) {
+        if(tid == 0) rotated = 0;
+        __syncthreads();
+        for(int r = 0; r < np - 1; ++r) {
+            int p = r, q = np - 1; // round_pair(np, r, grp, p, q), 0 <= r, grp < np - 1
+            if(grp > 0) {
+                p = r + grp, q = r - grp;
+                if(p >= np - 1) p -= np - 1;
+                if(q < 0) q += np - 1;
+            }
+            if(p > q) {
+                const int tt = p;
+                p            = q;
+                q            = tt;
+            }
+            if(grp < np / 2 && q < n) {
+                T *wp = Ws + p * SW + lane, *wq = Ws + q * SW + lane, *vp = Vs + p * SV + lane, *vq = Vs + q * SV + lane;
+                T  x[E], y[E], vx[EV], vy[EV];
+                double al = 0, be = 0, gr = 0, gi = 0;
+#pragma unroll
+                for(int e = 0; e < E; ++e) x[e] = wp[16 * e], y[e] = wq[16 * e];
+#pragma unroll
+                for(int e = 0; e < EV; ++e) vx[e] = vp[16 * e], vy[e] = vq[16 * e];
+#pragma unroll
+                for(int e = 0; e < E; ++e) {
+                    if constexpr(cx) {
+                        al += x[e].re * x[e].re + x[e].im * x[e].im;
+                        be += y[e].re * y[e].re + y[e].im * y[e].im;
+                        gr += x[e].re * y[e].re + x[e].im * y[e].im; // conj(x) y
+                        gi += x[e].re * y[e].im - x[e].im * y[e].re;
+                    } else {
+                        al += x[e] * x[e];
+                        be += y[e] * y[e];
+                        gr += x[e] * y[e];
+                    }
+                }
+                al = row_sum(al), be = row_sum(be), gr = row_sum(gr);
+                if constexpr(cx) gi = row_sum(gi);
+                const double g = magnitude<T>(gr, gi);
+                if(rotates(g, al, be, tol)) {
+                    // The rotation of jacobi_round: with d = be - al, h = sqrt(d^2 + (2 g)^2) and u = |d| + h the tangent is
+                    // sign(d) 2 g / u. d and g are scaled to about 1 first, so that no square leaves the range.
+                    const double d0 = be - al, e2 = fmax(fabs(d0), g);
+                    int          ex;
+                    (void) frexp(e2, &ex);
+                    const double d = ldexp(fabs(d0), -ex), g2 = ldexp(g, 1 - ex);
+                    const double u = d + sqrt(d * d + g2 * g2), w = rsqrt(u * u + g2 * g2);
+                    const double c = u * w, s = d0 >= 0 ? g2 * w : -(g2 * w);
+                    const double er = cx ? gr / g : (gr > 0 ? 1.0 : -1.0), ei = cx ? -gi / g : 0.0;
+                    if(lane == 0) rotated = 1;
+                    auto rot = [&](T &xv, T &yv) {
+                        if constexpr(cx) {
+                            const double yr = yv.re * er - yv.im * ei, yi = yv.re * ei + yv.im * er; // e^{-i phi} y
+                            const T      x0 = xv;
+                            xv              = T{c * x0.re - s * yr, c * x0.im - s * yi};
+                            yv              = T{s * x0.re + c * yr, s * x0.im + c * yi};
+                        } else {
+                            const double x0 = xv, y0 = yv * er;
+                            xv              = c * x0 - s * y0;
+                            yv              = s * x0 + c * y0;
+                        }
+                    };
+#pragma unroll
+                    for(int e = 0; e < E; ++e) {
+                        rot(x[e], y[e]);
+                        wp[16 * e] = x[e], wq[16 * e] = y[e];
+                    }
+#pragma unroll
+                    for(int e = 0; e < EV; ++e) {
+                        rot(vx[e], vy[e]);
+                        vp[16 * e] = vx[e], vq[16 * e] = vy[e];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        const int any = rotated;
+        __syncthreads();
+        if(any == 0) break;
+    }
+    for(int j = grp; j < n; j += static_cast<int>(blockDim.x) / 16) {
+        double a = 0;
+#pragma unroll
+        for(int e = 0; e < E; ++e) {
+            const T v = Ws[j * SW + lane + 16 * e];
+            if constexpr(cx) a += v.re * v.re + v.im * v.im;
+            else a += v * v;
+        }
+        a = row_sum(a);
+        if(lane == 0) nrm[j] = sqrt(a), perm[j] = j;
+    }
+    __syncthreads();
+    if(tid < n) { // descending, equal ones in their order
+        int rank = 0;
+        for(int i = 0; i < n; ++i) rank += nrm[i] > nrm[tid] || (nrm[i] == nrm[tid] && i < tid) ? 1 : 0;
+        perm[rank] = tid;
+        S[rank]    = nrm[tid];
+    }
+    if(tid == 0) S[n] = static_cast<double>(sweep);
+    __syncthreads();
+    // A = W' diag(S) V^H, W' the normalised columns; the factors of A^H the other way round.
+    T *left = tr ? Vt : U, *right = tr ? U : Vt;
+    for(int t = tid; t < m * n; t += blockDim.x) {
+        const int    k = tr ? t % n : t / m, i = tr ? t / n : t % m;
+        const double sk = nrm[perm[k]], f = sk > 0 ? 1.0 / sk : 0.0;
+        const T      v = jscale(f, Ws[perm[k] * SW + i]);
+        left[t]        = tr ? jconj(v) : v;
+    }
+    for(int t = tid; t < n * n; t += blockDim.x) {
+        const int k = tr ? t / n : t % n, j = tr ? t % n : t / n;
+        const T   v = Vs[perm[k] * SV + j];
+        right[t]    = tr ? v : jconj(v);
+    }
+}
+template <typename T>
+size_t resident_lds(int n, int E, int EV) {
+    const bool pad = !jtraits<T>::cx;
+    return static_cast<size_t>(n) * (16 * (E + EV) + (pad && E % 2 == 0 ? 16 : 0) + (pad && EV % 2 == 0 ? 16 : 0)) * sizeof(T);
+}
+template <typename T, int E, int EV>
+void launch_resident(int m, int n, int tr, const T *A, double tol, int max_sweeps, T *U, T *Vt, double *S, hipStream_t s) {
+    const size_t lds = resident_lds<T>(n, E, EV);
+    DMRG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&jacobi_resident<T, E, EV>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       static_cast<int>(JACOBI_LDS_BYTES)));
+    const int pairs = (n + 1) / 2;
+    hipLaunchKernelGGL((jacobi_resident<T, E, EV>), dim3(1), dim3((16 * pairs + 63) / 64 * 64), lds, s, m, n, tr, A, tol, max_sweeps, U, Vt, S);
+    DMRG_HIP_CHECK(hipGetLastError());
 }
 
 template <int G>
@@ -341,10 +535,10 @@ __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T
                 be = group_sum<G>(be);
                 gr = group_sum<G>(gr);
                 if constexpr(jtraits<T>::cx) gi = group_sum<G>(gi);
-                const double g = sqrt(gr * gr + gi * gi);
-                if(!live || !(g > tol * sqrt(al * be)) || g == 0.0) continue;
+                const double g = magnitude<T>(gr, gi);
+                if(!live || !rotates(g, al, be, tol)) continue;
                 const double z  = (be - al) / (2.0 * g);
-                const double t  = (z >= 0 ? 1.0 : -1.0) / (fabs(z) + sqrt(1.0 + z * z));
+                const double t  = tangent(z);
                 const double c  = 1.0 / sqrt(1.0 + t * t), s = c * t;
                 const double er = gr / g, ei = -gi / g;
                 if(lane == 0) rotated = 1;
@@ -435,8 +629,6 @@ __global__ void assemble_kernel(int m, int n, const int *perm, const double *S, 
     }
 }
 
-// LDS budget of the single-workgroup path (gfx950 has 160 KiB per CU).
-constexpr size_t JACOBI_LDS_BYTES = 152 * 1024;
 constexpr int    JACOBI_LDS_MAX_N = 32;
 // Block path from this many columns on (measured on gfx950, complex n x n, ms per SVD, per-pair rounds / block
 // rounds: 64: 2.86 / 2.4, 128: 7.4 / 5.8, 256: 19.5 / 14.4, 512: 61 / 35, 2048: 1325 / 289); B2 columns (two
@@ -458,6 +650,32 @@ void DeviceSvd::jacobi(int m, int n, const T *A, std::vector<double> &S) {
     const int  mm = tr ? n : m, nn = tr ? m : n;
     k_            = nn;
     const size_t es = sizeof(T);
+    const double tol = std::sqrt(static_cast<double>(mm)) * 2.3e-16; // gesvj's threshold, sqrt(m) eps
+    const int    E = mm <= 32 ? 2 : mm <= 64 ? 4 : mm <= 80 ? 5 : 8, EV = nn <= 32 ? 2 : 4;
+    // Up to the size that one workgroup's registers, rows of lanes and LDS hold, that is faster than any number of launches
+    // (complex 128x64 does not fit: 6.4 ms in rounds of block pairs).
+    if(mm <= 128 && nn <= 64 && resident_lds<T>(nn, E, EV) <= JACOBI_LDS_BYTES) {
+        u.reserve(static_cast<size_t>(mm) * nn * es);
+        vt.reserve(static_cast<size_t>(mm) * nn * es);
+        res.reserve(static_cast<size_t>(nn + 1) * sizeof(double));
+        auto run = [&](auto e, auto ev) {
+            launch_resident<T, decltype(e)::value, decltype(ev)::value>(mm, nn, tr ? 1 : 0, A, tol, 60, u.as<T>(), vt.as<T>(), res.as<double>(), s);
+        };
+        using std::integral_constant;
+        if(EV == 2 && E == 2) run(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+        else if(EV == 2 && E == 4) run(integral_constant<int, 4>{}, integral_constant<int, 2>{});
+        else if(EV == 2 && E == 5) run(integral_constant<int, 5>{}, integral_constant<int, 2>{});
+        else if(EV == 2) run(integral_constant<int, 8>{}, integral_constant<int, 2>{});
+        else if(E == 5) run(integral_constant<int, 5>{}, integral_constant<int, 4>{});
+        else if(E == 4) run(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+        else run(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+        S.resize(nn + 1);
+        DMRG_HIP_CHECK(hipMemcpyAsync(S.data(), res.p, (nn + 1) * sizeof(double), hipMemcpyDeviceToHost, s));
+        DMRG_HIP_CHECK(hipStreamSynchronize(s));
+        DMRG_REQUIRE(S[nn] < 60, DMRG_ERR_NOT_CONVERGED, "Jacobi SVD: no convergence in 60 sweeps");
+        S.resize(nn);
+        return;
+    }
     const size_t lds_need = (static_cast<size_t>(mm) * nn + static_cast<size_t>(nn) * nn) * es;
     const bool   resident = nn > 1 && nn <= JACOBI_LDS_MAX_N && lds_need <= JACOBI_LDS_BYTES;
     const bool   blocked  = !resident && nn >= JACOBI_BLOCK_MIN_N;
@@ -478,7 +696,6 @@ void DeviceSvd::jacobi(int m, int n, const T *A, std::vector<double> &S) {
     }
     unsigned    *flag = info.as<unsigned>();
     const int    np   = nn + (nn & 1);
-    const double tol  = std::sqrt(static_cast<double>(mm)) * 2.3e-16; // gesvj's threshold, sqrt(m) eps
     unsigned     hflag = 0;
     int          sweep = 0;
     const size_t lds   = lds_need;
@@ -487,17 +704,10 @@ void DeviceSvd::jacobi(int m, int n, const T *A, std::vector<double> &S) {
     // round with one wavefront per pair and the launches it saves dominate.
     if(resident) {
         int *dsweeps = reinterpret_cast<int *>(flag + 1);
-        // n <= 32: at most 16 pairs a round; 16 lanes a pair for columns up to 128 (4 wavefronts share each
-        // round's barrier), one wavefront a pair beyond
-        if(mm <= 128) {
-            DMRG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&jacobi_lds<T, 16>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               static_cast<int>(JACOBI_LDS_BYTES)));
-            hipLaunchKernelGGL((jacobi_lds<T, 16>), dim3(1), dim3(256), lds, s, mm, nn, np, W, V, tol, 60, dsweeps);
-        } else {
-            DMRG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&jacobi_lds<T, 64>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               static_cast<int>(JACOBI_LDS_BYTES)));
-            hipLaunchKernelGGL((jacobi_lds<T, 64>), dim3(1), dim3(1024), lds, s, mm, nn, np, W, V, tol, 60, dsweeps);
-        }
+        // n <= 32: at most 16 pairs a round, one wavefront each
+        DMRG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&jacobi_lds<T, 64>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           static_cast<int>(JACOBI_LDS_BYTES)));
+        hipLaunchKernelGGL((jacobi_lds<T, 64>), dim3(1), dim3(1024), lds, s, mm, nn, np, W, V, tol, 60, dsweeps);
         DMRG_HIP_CHECK(hipGetLastError());
         int hs = 0;
         DMRG_HIP_CHECK(hipMemcpyAsync(&hs, dsweeps, sizeof(int), hipMemcpyDeviceToHost, s));
