@@ -25,7 +25,8 @@ constexpr int SB_QC1  = 4 * VEC_MAX_M + 10; // coefficients of pass 1, 2 * VEC_M
 constexpr int SB_QC2  = 6 * VEC_MAX_M + 10; // coefficients of pass 2, 2 * VEC_MAX_M
 constexpr int SB_QN   = 8 * VEC_MAX_M + 10; // |z|^2 after both passes
 constexpr int SB_TAU  = 8 * VEC_MAX_M + 12; // -tau as a complex number (2 doubles)
-constexpr int SB_SIZE = 8 * VEC_MAX_M + 14;
+constexpr int SB_H2   = 8 * VEC_MAX_M + 14; // projections of the expansion's second pass, |t|^2 after the first
+constexpr int SB_SIZE = 10 * VEC_MAX_M + 16;
 
 // ------------------------------------------------------------------------------------------- correction solver
 constexpr int CG_CHECK = 4; // host look at the CG state every CG_CHECK steps
@@ -107,6 +108,9 @@ void Davidson<T>::matvec(const T *x, T *y, int nvec) {
 template <typename T>
 void Davidson<T>::orthonormalize_into(T *t, int m, double *dnrm_pre, double *dnrm_post) {
     double *sm = small.as<double>();
+    if(dnrm_post == dnrm_pre + 2 &&
+       expand_small<T>(n, m, V.as<T>(), nullptr, n, nullptr, 0.0, nullptr, nullptr, t, t, std::numeric_limits<double>::infinity(), nullptr, dnrm_pre, s))
+        return;
     multidot<T>(n, 1, t, n, t, dnrm_pre, scratch.as<double>(), s);
     for(int pass = 0; pass < 2; ++pass) { // classical Gram-Schmidt, twice
         if(m == 0) break;
@@ -126,7 +130,11 @@ void Davidson<T>::expand_from(const T *src, T *t, int m, double *dnrm_pre, doubl
     double *sm   = small.as<double>();
     int    *flag = reinterpret_cast<int *>(sm + SB_FLAG);
     double *scr  = scratch.as<double>();
+    if(dnrm_post == dnrm_pre + 2 &&
+       expand_small<T>(n, m, V.as<T>(), nullptr, n, nullptr, 0.0, nullptr, nullptr, src, t, 0.5, nullptr, dnrm_pre, s))
+        return;
     multidot_x<T>(n, m, V.as<T>(), n, src, sm + SB_COL, dnrm_pre, nullptr, scr, s);
+    if(dnrm_post == dnrm_pre + 2 && expand_update<T>(n, m, V.as<T>(), n, sm + SB_COL, src, t, 0.5, sm + SB_H2, dnrm_pre, scr, s)) return;
     gemv_update_norm<T>(n, m, V.as<T>(), n, sm + SB_COL, -1.0, 1.0, src, t, dnrm_post, nullptr, scr, s);
     if(m > 0) {
         multidot_dgks<T>(n, m, V.as<T>(), n, t, sm + SB_COL, dnrm_pre, dnrm_post, 0.5, flag, scr, s);
@@ -317,8 +325,7 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
     std::vector<cx> H(static_cast<size_t>(mmax) * mmax, cx(0.0, 0.0));
     auto            Hat = [&](int i, int j) -> cx & { return H[i + static_cast<size_t>(mmax) * j]; };
     for(int j = 0; j < m; ++j) {
-        multidot<T>(n, m, Vp, n, Wp + j * n, sm + SB_COL, scratch.as<double>(), s);
-        DMRG_HIP_CHECK(hipMemcpyAsync(host + SB_COL, sm + SB_COL, 2 * m * sizeof(double), hipMemcpyDeviceToHost, s));
+        multidot_to_host<T>(n, m, Vp, n, Wp + j * n, sm + SB_COL, host + SB_COL, 0, 0, scratch.as<double>(), s);
         DMRG_HIP_CHECK(hipStreamSynchronize(s));
         for(int i = 0; i < m; ++i) Hat(i, j) = cx(host[SB_COL + 2 * i], host[SB_COL + 2 * i + 1]);
     }
@@ -339,11 +346,14 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
     bool                inject_random = false;
 
     // Ritz vector x = V y and residual r = W y - theta x for column col of Z; |r|^2, |x|^2 go to SB_RITZ.
-    auto ritz_launch = [&](int col_in_H, int m_, T *xout) {
+    auto ritz_coefficients = [&](int col_in_H, int m_) {
         for(int i = 0; i < m_; ++i) {
             host[SB_Y + 2 * i]     = Z[i + static_cast<size_t>(m_) * col_in_H].real();
             host[SB_Y + 2 * i + 1] = Z[i + static_cast<size_t>(m_) * col_in_H].imag();
         }
+    };
+    auto ritz_launch = [&](int col_in_H, int m_, T *xout) {
+        ritz_coefficients(col_in_H, m_);
         ritz_residual<T>(n, m_, Vp, Wp, n, host + SB_Y, sm + SB_Y, w[col_in_H], xout, r, sm + SB_RITZ, scratch.as<double>(), s);
     };
     auto ritz_norm = [&]() { // |r| / |x| from the host copy of SB_RITZ
@@ -460,25 +470,34 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
         // (Not with correction solves: their FP32 matvecs would be lost on a pair that has converged.)
         const bool speculate = !use_inner && nev == 1 && m + 1 <= mmax && m < n && st.matvecs < p.max_matvecs;
         if(speculate) {
-            ritz_launch(ord[0], m, out);
             yprev.assign(m, cx(0.0, 0.0));
             for(int i = 0; i < m; ++i) yprev[i] = Z[i + static_cast<size_t>(m) * ord[0]];
             T *t = Vp + static_cast<int64_t>(m) * n;
-            const T *src = r;
-            if(inject_random) {
-                random_fill<T>(n, t, p.seed + 7919ull * (st.iters + 1), s);
-                src           = t;
-                inject_random = false;
-            } else if(p.precond != 0) {
-                apply_precond(w[ord[0]], out, t);
-                src = t;
+            bool done = false;
+            if(!inject_random && p.precond == 0) {
+                ritz_coefficients(ord[0], m);
+                done = expand_small<T>(n, m, Vp, Wp, n, host + SB_Y, w[ord[0]], out, r, nullptr, t, 0.5, sm + SB_RITZ, sm + SB_NRM, s);
+                static_assert(SB_RITZ == SB_NRM + 4, "expand_project writes both");
+                if(!done && expand_project<T>(n, m, Vp, Wp, n, host + SB_Y, sm + SB_Y, w[ord[0]], out, r, sm + SB_COL, sm + SB_NRM, scratch.as<double>(), s))
+                    done = expand_update<T>(n, m, Vp, n, sm + SB_COL, r, t, 0.5, sm + SB_H2, sm + SB_NRM, scratch.as<double>(), s);
             }
-            expand_from(src, t, m, sm + SB_NRM, sm + SB_NRM + 2);
+            if(!done) {
+                ritz_launch(ord[0], m, out);
+                const T *src = r;
+                if(inject_random) {
+                    random_fill<T>(n, t, p.seed + 7919ull * (st.iters + 1), s);
+                    src           = t;
+                    inject_random = false;
+                } else if(p.precond != 0) {
+                    apply_precond(w[ord[0]], out, t);
+                    src = t;
+                }
+                expand_from(src, t, m, sm + SB_NRM, sm + SB_NRM + 2);
+            }
             matvec(t, Wp + static_cast<int64_t>(m) * n, 1);
             st.matvecs += 1;
-            multidot<T>(n, m + 1, Vp, n, Wp + static_cast<int64_t>(m) * n, sm + SB_COL, scratch.as<double>(), s);
+            multidot_to_host<T>(n, m + 1, Vp, n, Wp + static_cast<int64_t>(m) * n, sm, host, SB_NRM, SB_RITZ + 2 - SB_NRM, scratch.as<double>(), s);
             if(refined) qr_append(m, p.shift);
-            DMRG_HIP_CHECK(hipMemcpyAsync(host, sm, (SB_RITZ + 2) * sizeof(double), hipMemcpyDeviceToHost, s));
             if(refined) qr_fetch();
             DMRG_HIP_CHECK(hipStreamSynchronize(s));
             rn[0]    = ritz_norm();
@@ -626,9 +645,8 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
         expand_from(src, t, m, sm + SB_NRM, sm + SB_NRM + 2);
         matvec(t, Wp + static_cast<int64_t>(m) * n, 1);
         st.matvecs += 1;
-        multidot<T>(n, m + 1, Vp, n, Wp + static_cast<int64_t>(m) * n, sm + SB_COL, scratch.as<double>(), s);
+        multidot_to_host<T>(n, m + 1, Vp, n, Wp + static_cast<int64_t>(m) * n, sm, host, SB_NRM, 4, scratch.as<double>(), s);
         if(refined) qr_append(m, p.shift);
-        DMRG_HIP_CHECK(hipMemcpyAsync(host, sm, (SB_NRM + 4) * sizeof(double), hipMemcpyDeviceToHost, s));
         if(refined) qr_fetch();
         DMRG_HIP_CHECK(hipStreamSynchronize(s));
         accept_expansion(m);

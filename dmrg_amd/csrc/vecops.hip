@@ -79,8 +79,17 @@ __device__ inline void publish(double *p, double v, bool device_scope) {
     else *p = v;
 }
 
-// partial: [row block][nv]; value v goes to out[v], or self_out[v & 1] for the column v / 2 == j_self (when given).
-__device__ inline void fold_in_last_block(const double *partial, int nv, double *out, int j_self, double *self_out, unsigned *counter) {
+// What a reduction's last workgroup also writes to pinned host memory: its sums to h_out, and n doubles of d to h.
+struct HostCopy {
+    double       *h_out = nullptr;
+    const double *d     = nullptr;
+    double       *h     = nullptr;
+    int           n     = 0; // at most VT_THREADS
+};
+
+// partial: [row block][nv]; value v goes to out[v], from column v / 2 == j_self on to self_out (when given).
+__device__ inline void fold_in_last_block(const double *partial, int nv, double *out, int j_self, double *self_out, unsigned *counter,
+                                          const HostCopy &hc = HostCopy{}) {
     __shared__ int last;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the partials of this wavefront are at device scope
     __syncthreads();
@@ -113,9 +122,11 @@ __device__ inline void fold_in_last_block(const double *partial, int nv, double 
     if(t < nv) {
         double acc = 0.0;
         for(int k = 0; k < per; ++k) acc += red[t + k * nv];
-        double *o = ((t >> 1) == j_self && self_out) ? self_out + (t & 1) : out + t;
+        double *o = ((t >> 1) >= j_self && self_out) ? self_out + (t - 2 * j_self) : out + t;
         *o        = acc;
+        if(hc.h_out) hc.h_out[t] = acc;
     }
+    if(t < hc.n) hc.h[t] = hc.d[t];
     if(t == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
@@ -175,7 +186,7 @@ struct DgksTest {
 template <typename T, int CH>
 __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m, int mc, const T *V, int64_t ldv, const T *x,
                                                                const int *skip, double *partial, unsigned *counter, double *out,
-                                                               int m_out, double *self_out, DgksTest dg) {
+                                                               int m_out, double *self_out, DgksTest dg, HostCopy hc) {
     if(dg.flag) {
         const bool run = dg.post[0] < dg.eta2 * dg.pre[0];
         if(blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) dg.flag[0] = run ? 1 : 0;
@@ -218,17 +229,17 @@ __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m,
         }
         __syncthreads();
     }
-    if(counter) fold_in_last_block(partial, 2 * mc, out, m_out, self_out, counter);
+    if(counter) fold_in_last_block(partial, 2 * mc, out, m_out, self_out, counter, hc);
 }
 
 static int md_grid(int64_t n) {
     return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(VEC_MAX_BLOCKS, (n + VT_THREADS * MD_PER_THREAD - 1) / (VT_THREADS * MD_PER_THREAD))));
 }
 
-// out[j] = sum_b partial[b][j] for j < m (column j == m_out goes to self_out instead, when given): one block
+// out[j] = sum_b partial[b][j] for j < m (columns from m_out on go to self_out instead, when given): one block
 // per column, each thread a fixed strided subset of the partials, then a fixed-order tree (deterministic).
 __global__ __launch_bounds__(VT_THREADS) void fold_columns(int nblk, int m, const double *partial, double *out, int m_out,
-                                                           double *self_out, const int *skip) {
+                                                           double *self_out, const int *skip, HostCopy hc) {
     if(skip && *skip == 0) return;
     __shared__ double red[2][VT_THREADS / 64];
     const int         j   = blockIdx.x;
@@ -239,15 +250,17 @@ __global__ __launch_bounds__(VT_THREADS) void fold_columns(int nblk, int m, cons
     }
     bsum<2>(acc, red);
     if(threadIdx.x == 0) {
-        double *o = (j == m_out && self_out) ? self_out : out + 2 * j;
+        double *o = (j >= m_out && self_out) ? self_out + 2 * (j - m_out) : out + 2 * j;
         o[0]      = acc[0];
         o[1]      = acc[1];
+        if(hc.h_out) hc.h_out[2 * j] = acc[0], hc.h_out[2 * j + 1] = acc[1];
     }
+    if(j == 0 && static_cast<int>(threadIdx.x) < hc.n) hc.h[threadIdx.x] = hc.d[threadIdx.x];
 }
 
 template <typename T>
 static void multidot_x_impl(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_out, double *d_self, const int *skip,
-                            const DgksTest &dg, double *scratch, hipStream_t s) {
+                            const DgksTest &dg, double *scratch, hipStream_t s, const HostCopy &hc = HostCopy{}) {
     const int mc = m + (d_self ? 1 : 0);
     if(mc <= 0) return;
     DMRG_REQUIRE(mc <= VEC_MAX_M, DMRG_ERR_ARG, "multidot: too many columns");
@@ -259,14 +272,14 @@ static void multidot_x_impl(int64_t n, int m, const T *V, int64_t ldv, const T *
         const bool in_last = want <= 2 * most && fused(static_cast<int64_t>(std::min(want, most)) * groups, 2 * mc);
         const int  rows    = in_last ? std::min(want, most) : std::min(want, 256);
         hipLaunchKernelGGL((multidot_partial<T, MD_CH_SHORT>), dim3(rows, groups), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch,
-                           in_last ? scratch_counter(scratch) : nullptr, d_out, d_self ? m : -1, d_self, dg);
+                           in_last ? scratch_counter(scratch) : nullptr, d_out, d_self ? m : -1, d_self, dg, hc);
         if(!in_last)
-            hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, rows, mc, scratch, d_out, d_self ? m : -1, d_self, fskip);
+            hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, rows, mc, scratch, d_out, d_self ? m : -1, d_self, fskip, hc);
     } else {
         const int g = md_grid(n);
         hipLaunchKernelGGL((multidot_partial<T, MD_CH>), dim3(g), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch, nullptr,
-                           nullptr, -1, nullptr, dg);
-        hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, g, mc, scratch, d_out, d_self ? m : -1, d_self, fskip);
+                           nullptr, -1, nullptr, dg, HostCopy{});
+        hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, g, mc, scratch, d_out, d_self ? m : -1, d_self, fskip, hc);
     }
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -274,6 +287,18 @@ static void multidot_x_impl(int64_t n, int m, const T *V, int64_t ldv, const T *
 template <typename T>
 void multidot(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_out, double *scratch, hipStream_t s) {
     multidot_x_impl<T>(n, m, V, ldv, x, d_out, nullptr, nullptr, DgksTest{}, scratch, s);
+}
+
+// The copies to the host ride on the fold of the reduction: a copy of its own is another launch, about 2 us, and its gap.
+template <typename T>
+void multidot_to_host(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_block, double *h_block, int extra, int n_extra,
+                      double *scratch, hipStream_t s) {
+    HostCopy hc;
+    hc.h_out = h_block;
+    hc.d     = d_block + extra;
+    hc.h     = h_block + extra;
+    hc.n     = n_extra;
+    multidot_x_impl<T>(n, m, V, ldv, x, d_block, nullptr, nullptr, DgksTest{}, scratch, s, hc);
 }
 
 template <typename T>
@@ -309,6 +334,41 @@ __device__ __forceinline__ void columns(int m, L &&load, F &&use) {
     }
 }
 
+// Row i of x = V y and r = W y - theta x.
+template <typename T>
+__device__ __forceinline__ void ritz_row(int64_t i, int m, const T *V, const T *W, int64_t ldv, const double *y, double theta, double &xr,
+                                         double &xi, double &rr, double &ri) {
+    double wr = 0, wi = 0;
+    struct VW {
+        T v, w;
+    };
+    xr = xi = 0;
+    columns<VW>(m, [&](int j) { return VW{V[i + j * ldv], W[i + j * ldv]}; },
+                [&](int j, const VW &e) {
+                    double vr, vi, ur, ui;
+                    ld(e.v, vr, vi);
+                    ld(e.w, ur, ui);
+                    const double yr = y[2 * j], yi = y[2 * j + 1];
+                    xr += vr * yr - vi * yi;
+                    xi += vr * yi + vi * yr;
+                    wr += ur * yr - ui * yi;
+                    wi += ur * yi + ui * yr;
+                });
+    rr = wr - theta * xr, ri = wi - theta * xi;
+}
+// Row i of V h.
+template <typename T>
+__device__ __forceinline__ void gemv_row(int64_t i, int m, const T *V, int64_t ldv, const double *h, double &ar, double &ai) {
+    ar = ai = 0;
+    columns<T>(m, [&](int j) { return V[i + j * ldv]; },
+               [&](int j, const T &v) {
+                   double vr, vi;
+                   ld(v, vr, vi);
+                   ar += vr * h[2 * j] - vi * h[2 * j + 1];
+                   ai += vr * h[2 * j + 1] + vi * h[2 * j];
+               });
+}
+
 template <typename T>
 __global__ __launch_bounds__(VT_THREADS) void gemv_update_kernel(int64_t n, int m, const T *V, int64_t ldv, const double *h,
                                                                  double alpha, double beta, T *x) {
@@ -316,14 +376,8 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_kernel(int64_t n, int 
     for(int j = threadIdx.x; j < 2 * m; j += VT_THREADS) hs[j] = h[j];
     __syncthreads();
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
-        double ar = 0, ai = 0;
-        columns<T>(m, [&](int j) { return V[i + j * ldv]; },
-                   [&](int j, const T &v) {
-                       double vr, vi;
-                       ld(v, vr, vi);
-                       ar += vr * hs[2 * j] - vi * hs[2 * j + 1];
-                       ai += vr * hs[2 * j + 1] + vi * hs[2 * j];
-                   });
+        double ar, ai;
+        gemv_row<T>(i, m, V, ldv, hs, ar, ai);
         double xr = 0, xi = 0;
         if(beta != 0.0) ld(x[i], xr, xi);
         x[i] = mk<T>(beta * xr + alpha * ar, beta * xi + alpha * ai);
@@ -343,14 +397,8 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_norm_kernel(int64_t n,
     __syncthreads();
     double acc[2] = {0.0, 0.0};
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
-        double ar = 0, ai = 0;
-        columns<T>(m, [&](int j) { return V[i + j * ldv]; },
-                   [&](int j, const T &v) {
-                       double vr, vi;
-                       ld(v, vr, vi);
-                       ar += vr * hs[2 * j] - vi * hs[2 * j + 1];
-                       ai += vr * hs[2 * j + 1] + vi * hs[2 * j];
-                   });
+        double ar, ai;
+        gemv_row<T>(i, m, V, ldv, hs, ar, ai);
         double xr = 0, xi = 0;
         if(beta != 0.0) ld(x[i], xr, xi);
         const T yv = mk<T>(beta * xr + alpha * ar, beta * xi + alpha * ai);
@@ -387,7 +435,7 @@ void gemv_update_norm(int64_t n, int m, const T *V, int64_t ldv, const double *d
     } else {
         hipLaunchKernelGGL(gemv_update_norm_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, alpha, beta, x, y, skip, scratch,
                            nullptr, nullptr);
-        hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_nrm2, -1, nullptr, skip);
+        hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_nrm2, -1, nullptr, skip, HostCopy{});
     }
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -412,22 +460,8 @@ __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, cons
     __syncthreads();
     double acc[2] = {0.0, 0.0};
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
-        double xr = 0, xi = 0, wr = 0, wi = 0;
-        struct VW {
-            T v, w;
-        };
-        columns<VW>(m, [&](int j) { return VW{V[i + j * ldv], W[i + j * ldv]}; },
-                    [&](int j, const VW &e) {
-                        double vr, vi, ur, ui;
-                        ld(e.v, vr, vi);
-                        ld(e.w, ur, ui);
-                        const double yr = ys[2 * j], yi = ys[2 * j + 1];
-                        xr += vr * yr - vi * yi;
-                        xi += vr * yi + vi * yr;
-                        wr += ur * yr - ui * yi;
-                        wi += ur * yi + ui * yr;
-                    });
-        const double rr = wr - theta * xr, ri = wi - theta * xi;
+        double xr, xi, rr, ri;
+        ritz_row<T>(i, m, V, W, ldv, ys, theta, xr, xi, rr, ri);
         x[i] = mk<T>(xr, xi);
         r[i] = mk<T>(rr, ri);
         acc[0] += rr * rr + ri * ri;
@@ -451,7 +485,7 @@ static void ritz_launch(int64_t n, int m, const T *V, const T *W, int64_t ld, co
                            scratch_counter(scratch), d_out);
     } else {
         hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch, nullptr, nullptr);
-        hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_out, -1, nullptr, nullptr);
+        hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_out, -1, nullptr, nullptr, HostCopy{});
     }
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -467,6 +501,326 @@ void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const d
         DMRG_HIP_CHECK(hipMemcpyAsync(d_y, h_y, 2 * static_cast<size_t>(m) * sizeof(double), hipMemcpyHostToDevice, s));
     }
     ritz_launch<T>(n, m, V, W, ld, d_y, c, theta, x, r, d_out, scratch, s);
+}
+
+// ------------------------------------------------------------------------------------------- expansion of a small basis
+// Ritz vector and residual, Gram-Schmidt with the DGKS test, and normalisation of a small problem, in one workgroup with the
+// vector in LDS. Bounded by latency: a pass over a basis in the caches takes 1 to 2 us, a launch of its own 4 us and 6 to 9
+// of the host's time, and the steps are six launches otherwise (n up to 512, up to 14 columns: 8.2 us against 19 in six, and
+// a sweep of L = 16 at chi = 32 takes 194 ms against 273).
+constexpr int     EX_THREADS = 1024;
+constexpr int     EX_WAVES   = EX_THREADS / 64;
+// One CU reads its caches at about 100 GB/s: up to here that costs less than the launches.
+constexpr int64_t EX_MAX_BYTES = 32768;
+
+template <typename T>
+struct ExpandArgs {
+    int64_t  n, ldv;
+    int      m;
+    const T *V, *W, *src; // W null: src is orthogonalised, else the residual
+    T       *x, *r, *t;
+    double   theta, eta2;
+    double  *ritz, *nrm;
+};
+
+// Sums over the workgroup, in every thread.
+template <int NV>
+__device__ inline void all_sum(double (&v)[NV], double (*red)[EX_WAVES]) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for(int i = 0; i < NV; ++i) v[i] = wsum(v[i]);
+    __syncthreads();
+    if(lane == 0)
+#pragma unroll
+        for(int i = 0; i < NV; ++i) red[i][wave] = v[i];
+    __syncthreads();
+#pragma unroll
+    for(int i = 0; i < NV; ++i) {
+        v[i] = 0;
+#pragma unroll
+        for(int w = 0; w < EX_WAVES; ++w) v[i] += red[i][w];
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(EX_THREADS) void expand_kernel(const ExpandArgs<T> g, const RitzCoef c) {
+    extern __shared__ __attribute__((aligned(16))) char expand_lds[];
+    T                *tv = reinterpret_cast<T *>(expand_lds);
+    __shared__ double hs[2 * RITZ_ARGS], part[2 * RITZ_ARGS][2], red[3][EX_WAVES];
+    const int         tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = static_cast<int>(g.n), m = g.m;
+    double            acc[3] = {0.0, 0.0, 0.0};
+    if(g.W) {
+        if(tid < 2 * m) hs[tid] = c.y[tid];
+        __syncthreads();
+        for(int i = tid; i < n; i += EX_THREADS) {
+            double xr, xi, rr, ri;
+            ritz_row<T>(i, m, g.V, g.W, g.ldv, hs, g.theta, xr, xi, rr, ri);
+            const T      rv = mk<T>(rr, ri);
+            g.x[i]          = mk<T>(xr, xi);
+            g.r[i]          = rv;
+            tv[i]           = rv;
+            double sr, si;
+            ld(rv, sr, si);
+            acc[0] += rr * rr + ri * ri;
+            acc[1] += xr * xr + xi * xi;
+            acc[2] += sr * sr + si * si;
+        }
+    } else {
+        for(int i = tid; i < n; i += EX_THREADS) {
+            const T v = g.src[i];
+            tv[i]     = v;
+            double sr, si;
+            ld(v, sr, si);
+            acc[2] += sr * sr + si * si;
+        }
+    }
+    all_sum<3>(acc, red);
+    if(g.W && tid == 0) g.ritz[0] = acc[0], g.ritz[1] = acc[1];
+    const double pre = acc[2];
+    double       post[1] = {pre};
+    // Projections: a wavefront per column and segment of rows, so that few columns also keep all wavefronts reading.
+    const int segs = m > 0 ? max(1, EX_WAVES / m) : 1, len = (n + segs - 1) / segs;
+    for(int pass = 0; m > 0 && pass < 2; ++pass) {
+        for(int task = wave; task < m * segs; task += EX_WAVES) {
+            const int j = task % m, i0 = task / m * len, i1 = min(n, i0 + len);
+            const T  *v = g.V + j * g.ldv;
+            double    ar = 0, ai = 0;
+#pragma unroll 8
+            for(int i = i0 + lane; i < i1; i += 64) {
+                double vr, vi, xr, xi;
+                ld(v[i], vr, vi);
+                ld(tv[i], xr, xi);
+                ar += vr * xr + vi * xi; // conj(v) x
+                ai += vr * xi - vi * xr;
+            }
+            ar = wsum(ar);
+            if constexpr(vtraits<T>::cx) ai = wsum(ai);
+            if(lane == 0) part[task][0] = ar, part[task][1] = ai;
+        }
+        __syncthreads();
+        if(tid < 2 * m) {
+            double h = 0;
+            for(int q = 0; q < segs; ++q) h += part[q * m + (tid >> 1)][tid & 1];
+            hs[tid] = h;
+        }
+        __syncthreads();
+        post[0] = 0;
+        for(int i = tid; i < n; i += EX_THREADS) {
+            double ar, ai;
+            gemv_row<T>(i, m, g.V, g.ldv, hs, ar, ai);
+            double xr, xi;
+            ld(tv[i], xr, xi);
+            const T y = mk<T>(xr - ar, xi - ai);
+            tv[i]     = y;
+            double yr, yi;
+            ld(y, yr, yi);
+            post[0] += yr * yr + yi * yi;
+        }
+        all_sum<1>(post, red);
+        if(!(post[0] < g.eta2 * pre)) break;
+    }
+    const double a = post[0] > 0.0 ? 1.0 / sqrt(post[0]) : 0.0; // a zero vector stays zero (breakdown tests see it)
+    for(int i = tid; i < n; i += EX_THREADS) {
+        double re, im;
+        ld(tv[i], re, im);
+        g.t[i] = mk<T>(a * re, a * im);
+    }
+    if(tid == 0) g.nrm[0] = pre, g.nrm[1] = 0.0, g.nrm[2] = post[0], g.nrm[3] = 0.0;
+}
+
+template <typename T>
+bool expand_small(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *h_y, double theta, T *x, T *r, const T *src, T *t,
+                  double eta2, double *d_ritz, double *d_nrm, hipStream_t s) {
+    if(n * static_cast<int64_t>(sizeof(T)) > EX_MAX_BYTES || m > RITZ_ARGS) return false;
+    RitzCoef c{};
+    if(W) std::copy(h_y, h_y + 2 * m, c.y);
+    const ExpandArgs<T> g{n, ldv, m, V, W, src, x, r, t, theta, eta2, d_ritz, d_nrm};
+    hipLaunchKernelGGL(expand_kernel<T>, dim3(1), dim3(EX_THREADS), static_cast<size_t>(n) * sizeof(T), s, g, c);
+    DMRG_HIP_CHECK(hipGetLastError());
+    return true;
+}
+
+// The same for problems of several workgroups, up to MD_SHORT rows: three launches (and a fold after the first two where one
+// workgroup per 256 rows is too many to fold in the last of them) instead of six (eleven). Each workgroup projects the rows
+// that it has just formed, so that the basis comes from its caches the second time; the second Gram-Schmidt pass's
+// projections are taken whether or not its test asks for them, and its norm from |t|^2 - |h|^2, h being rounding errors of
+// the first pass. Longer vectors come from HBM, where the extra projections cost more than the
+// launches. n = 8192, 14 columns: 22 us of kernels either way, but 5.4 ms a solve against 6.9; n = 122880: 13.0 ms against 14.5.
+
+// partial[blockIdx.x][2 j] = this workgroup's rows of conj(V[:, j]) x.
+template <typename T>
+__device__ __forceinline__ void project_rows(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *partial, int nv, bool device_scope,
+                                             double (*red)[VT_THREADS / 64]) {
+    constexpr int CH = MD_CH, NV = 2 * CH;
+    const int     lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for(int j0 = 0; j0 < m; j0 += CH) {
+        double acc[NV];
+#pragma unroll
+        for(int c = 0; c < NV; ++c) acc[c] = 0.0;
+        for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
+            double xr, xi;
+            ld(x[i], xr, xi);
+            T v[CH];
+#pragma unroll
+            for(int c = 0; c < CH; ++c) v[c] = V[i + min(j0 + c, m - 1) * ldv];
+#pragma unroll
+            for(int c = 0; c < CH; ++c) {
+                double vr, vi;
+                ld(v[c], vr, vi);
+                acc[2 * c] += vr * xr + vi * xi; // conj(v) x
+                acc[2 * c + 1] += vr * xi - vi * xr;
+            }
+        }
+        rs_step<NV / 2, 32, NV>(acc, lane);
+        __syncthreads();
+        if(rs_owner<NV>(lane)) red[rs_index<NV>(lane)][wave] = acc[0];
+        __syncthreads();
+        if(threadIdx.x < NV && j0 + static_cast<int>(threadIdx.x >> 1) < m) {
+            double t = 0;
+#pragma unroll
+            for(int w = 0; w < VT_THREADS / 64; ++w) t += red[threadIdx.x][w];
+            publish(partial + static_cast<int64_t>(blockIdx.x) * nv + 2 * j0 + threadIdx.x, t, device_scope);
+        }
+    }
+}
+
+// x, r as in ritz_kernel; columns: V^H r, then (|r|^2 as stored, 0), (0, 0), (|r|^2, |x|^2).
+template <typename T>
+__global__ __launch_bounds__(VT_THREADS) void ritz_project_kernel(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *y,
+                                                                  const RitzCoef c, double theta, T *x, T *r, double *partial,
+                                                                  unsigned *counter, double *out, double *tail) {
+    __shared__ double ys[2 * VEC_MAX_M];
+    __shared__ double red[2 * MD_CH][VT_THREADS / 64];
+    const int         nv = 2 * m + 6;
+    if(y) {
+        for(int j = threadIdx.x; j < 2 * m; j += VT_THREADS) ys[j] = y[j];
+    } else if(threadIdx.x < 2 * m) {
+        ys[threadIdx.x] = c.y[threadIdx.x]; // 2 m <= 2 RITZ_ARGS < VT_THREADS
+    }
+    __syncthreads();
+    double acc[3] = {0.0, 0.0, 0.0};
+    for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
+        double xr, xi, rr, ri;
+        ritz_row<T>(i, m, V, W, ldv, ys, theta, xr, xi, rr, ri);
+        const T rv = mk<T>(rr, ri);
+        x[i]       = mk<T>(xr, xi);
+        r[i]       = rv;
+        double sr, si;
+        ld(rv, sr, si);
+        acc[0] += sr * sr + si * si;
+        acc[1] += rr * rr + ri * ri;
+        acc[2] += xr * xr + xi * xi;
+    }
+    bsum<3>(acc, red);
+    if(threadIdx.x == 0) {
+        double *p = partial + static_cast<int64_t>(blockIdx.x) * nv + 2 * m;
+        const double v[6] = {acc[0], 0.0, 0.0, 0.0, acc[1], acc[2]};
+#pragma unroll
+        for(int k = 0; k < 6; ++k) publish(p + k, v[k], counter != nullptr);
+    }
+    project_rows<T>(n, m, V, ldv, r, partial, nv, counter != nullptr, red);
+    if(counter) fold_in_last_block(partial, nv, out, m, tail, counter);
+}
+
+// t = src - V h; columns: V^H t, then (|t|^2, 0).
+template <typename T>
+__global__ __launch_bounds__(VT_THREADS) void update_project_kernel(int64_t n, int m, const T *V, int64_t ldv, const double *h, const T *src,
+                                                                    T *t, double *partial, unsigned *counter, double *out) {
+    __shared__ double hs[2 * VEC_MAX_M];
+    __shared__ double red[2 * MD_CH][VT_THREADS / 64];
+    const int         nv = 2 * m + 2;
+    for(int j = threadIdx.x; j < 2 * m; j += VT_THREADS) hs[j] = h[j];
+    __syncthreads();
+    double acc[1] = {0.0};
+    for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
+        double ar, ai, xr, xi;
+        gemv_row<T>(i, m, V, ldv, hs, ar, ai);
+        ld(src[i], xr, xi);
+        const T y = mk<T>(xr - ar, xi - ai);
+        t[i]      = y;
+        double yr, yi;
+        ld(y, yr, yi);
+        acc[0] += yr * yr + yi * yi;
+    }
+    bsum<1>(acc, red);
+    if(threadIdx.x == 0) {
+        double *p = partial + static_cast<int64_t>(blockIdx.x) * nv + 2 * m;
+        publish(p, acc[0], counter != nullptr);
+        publish(p + 1, 0.0, counter != nullptr);
+    }
+    project_rows<T>(n, m, V, ldv, t, partial, nv, counter != nullptr, red);
+    if(counter) fold_in_last_block(partial, nv, out, -1, nullptr, counter);
+}
+
+// The second pass where |t|^2 (h2[2 m]) fell below eta2 |src|^2 (nrm[0]), and the normalisation; nrm[2] = |t|^2.
+template <typename T>
+__global__ __launch_bounds__(VT_THREADS) void expand_finish_kernel(int64_t n, int m, const T *V, int64_t ldv, const double *h2, double eta2, T *t,
+                                                                   double *nrm) {
+    __shared__ double hs[2 * VEC_MAX_M];
+    __shared__ double red[1][VT_THREADS / 64];
+    __shared__ double total;
+    double            post  = h2[2 * m];
+    const bool        again = m > 0 && post < eta2 * nrm[0];
+    if(again) { // the same in every workgroup
+        double acc[1] = {0.0};
+        for(int j = threadIdx.x; j < 2 * m; j += VT_THREADS) {
+            hs[j] = h2[j];
+            acc[0] += hs[j] * hs[j];
+        }
+        bsum<1>(acc, red);
+        if(threadIdx.x == 0) total = acc[0];
+        __syncthreads();
+        post = fmax(post - total, 0.0);
+    }
+    const double a = post > 0.0 ? 1.0 / sqrt(post) : 0.0; // a zero vector stays zero (breakdown tests see it)
+    for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
+        double ar = 0, ai = 0, xr, xi;
+        if(again) gemv_row<T>(i, m, V, ldv, hs, ar, ai);
+        ld(t[i], xr, xi);
+        t[i] = mk<T>(a * (xr - ar), a * (xi - ai));
+    }
+    if(blockIdx.x == 0 && threadIdx.x == 0) nrm[2] = post, nrm[3] = 0.0;
+}
+
+static bool expand_fits(int64_t n, int m) { return n <= MD_SHORT && m + 3 <= VEC_MAX_M; }
+// One row a thread, or two where that lets the last workgroup fold.
+static int expand_grid(int64_t n, int values) {
+    const int b = static_cast<int>(std::max<int64_t>(1, (n + VT_THREADS - 1) / VT_THREADS));
+    return b > FUSE_MAX_BLOCKS && b <= 2 * FUSE_MAX_BLOCKS && values <= FUSE_MAX_VALUES ? (b + 1) / 2 : b;
+}
+
+template <typename T>
+bool expand_project(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *h_y, double *d_y, double theta, T *x, T *r, double *d_out,
+                    double *d_tail, double *scratch, hipStream_t s) {
+    if(!expand_fits(n, m)) return false;
+    RitzCoef c{};
+    if(m <= RITZ_ARGS) {
+        std::copy(h_y, h_y + 2 * m, c.y);
+        d_y = nullptr;
+    } else {
+        DMRG_HIP_CHECK(hipMemcpyAsync(d_y, h_y, 2 * static_cast<size_t>(m) * sizeof(double), hipMemcpyHostToDevice, s));
+    }
+    const int  g  = expand_grid(n, 2 * m + 6);
+    const bool in = fused(g, 2 * m + 6);
+    hipLaunchKernelGGL(ritz_project_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ldv, d_y, c, theta, x, r, scratch,
+                       in ? scratch_counter(scratch) : nullptr, d_out, d_tail);
+    if(!in) hipLaunchKernelGGL(fold_columns, dim3(m + 3), dim3(VT_THREADS), 0, s, g, m + 3, scratch, d_out, m, d_tail, nullptr, HostCopy{});
+    DMRG_HIP_CHECK(hipGetLastError());
+    return true;
+}
+
+template <typename T>
+bool expand_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h, const T *src, T *t, double eta2, double *d_h2, double *d_nrm,
+                   double *scratch, hipStream_t s) {
+    if(!expand_fits(n, m)) return false;
+    const int  g  = expand_grid(n, 2 * m + 2);
+    const bool in = fused(g, 2 * m + 2);
+    hipLaunchKernelGGL(update_project_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, src, t, scratch,
+                       in ? scratch_counter(scratch) : nullptr, d_h2);
+    if(!in) hipLaunchKernelGGL(fold_columns, dim3(m + 1), dim3(VT_THREADS), 0, s, g, m + 1, scratch, d_h2, -1, nullptr, nullptr, HostCopy{});
+    hipLaunchKernelGGL(expand_finish_kernel<T>, dim3(ew_grid(n)), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h2, eta2, t, d_nrm);
+    DMRG_HIP_CHECK(hipGetLastError());
+    return true;
 }
 
 // ------------------------------------------------------------------------------------------- elementwise
@@ -675,7 +1029,7 @@ void cg_init(int64_t n, const T *x, const double *d_c, double sigma, T *r, T *p,
     const bool in_last = fused(g, 2);
     hipLaunchKernelGGL(cg_init_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, x, d_c, sigma, r, p, t, scratch,
                        in_last ? scratch_counter(scratch) : nullptr, d_rr);
-    if(!in_last) hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr);
+    if(!in_last) hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr, HostCopy{});
     hipLaunchKernelGGL(cg_start_kernel, dim3(1), dim3(1), 0, s, d_rr, state);
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -693,7 +1047,7 @@ void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t
     const bool in_last = fused(g, 2);
     hipLaunchKernelGGL(cg_update_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, x, p, q, d_dots, state, k, t, r, scratch,
                        in_last ? scratch_counter(scratch) : nullptr, d_rr);
-    if(!in_last) hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr);
+    if(!in_last) hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_rr, -1, nullptr, nullptr, HostCopy{});
     hipLaunchKernelGGL(cg_direction_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, r, d_dots, d_rr, state, k, rtol2, p);
     DMRG_HIP_CHECK(hipGetLastError());
 }
@@ -703,6 +1057,13 @@ void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t
     template void gemv_update<T>(int64_t, int, const T *, int64_t, const double *, double, double, T *, hipStream_t); \
     template void ritz_residual<T>(int64_t, int, const T *, const T *, int64_t, const double *, double *, double, T *,  \
                                    T *, double *, double *, hipStream_t);                                              \
+    template void multidot_to_host<T>(int64_t, int, const T *, int64_t, const T *, double *, double *, int, int, double *, hipStream_t);\
+    template bool expand_small<T>(int64_t, int, const T *, const T *, int64_t, const double *, double, T *, T *, const T *, T *, double,\
+                                  double *, double *, hipStream_t);                                                   \
+    template bool expand_project<T>(int64_t, int, const T *, const T *, int64_t, const double *, double *, double, T *, T *,\
+                                    double *, double *, double *, hipStream_t);                                       \
+    template bool expand_update<T>(int64_t, int, const T *, int64_t, const double *, const T *, T *, double, double *, double *,\
+                                   double *, hipStream_t);                                                            \
     template void scale_by_inv_norm<T>(int64_t, T *, const double *, hipStream_t);                                    \
     template void scale<T>(int64_t, T *, double, hipStream_t);                                                         \
     template void random_fill<T>(int64_t, T *, uint64_t, hipStream_t);                                               \

@@ -46,6 +46,11 @@ void vec_scratch_init(double *scratch, hipStream_t s);
 // out[j] = sum_i conj(V[i, j]) x[i], j < m (complex double, out on device, 2*m doubles).
 template <typename T>
 void multidot(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_out, double *scratch, hipStream_t s);
+// multidot to d_block, with 2 m doubles of the result, and then n_extra doubles of d_block from extra on, also at the same
+// places of h_block (pinned host memory; valid after a synchronisation).
+template <typename T>
+void multidot_to_host(int64_t n, int m, const T *V, int64_t ldv, const T *x, double *d_block, double *h_block, int extra, int n_extra,
+                      double *scratch, hipStream_t s);
 // out[j] = sum_i conj(V[i, j]) x[i] for j < m and, when d_self is given, d_self[0] = |x|^2 from the same pass.
 // skip (device int, optional): when *skip == 0 the kernels do nothing (outputs keep their values).
 template <typename T>
@@ -69,6 +74,22 @@ void gemv_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h, d
 template <typename T>
 void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *h_y, double *d_y, double theta, T *x, T *r,
                    double *d_out, double *scratch, hipStream_t s);
+// Small problems in one launch, false for others: with W, x = V y, r = W y - theta x and d_ritz as in ritz_residual (h_y on
+// the host), src = r; then t = src orthogonalised against V[:, 0:m] and normalised, a second pass taken where the first one
+// leaves less than eta2 of the squared norm; d_nrm[0] = |src|^2, d_nrm[2] = |t|^2 before the normalisation. src may be t.
+template <typename T>
+bool expand_small(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *h_y, double theta, T *x, T *r, const T *src, T *t,
+                  double eta2, double *d_ritz, double *d_nrm, hipStream_t s);
+// The same in steps for problems of up to 2^17 rows, false for others. expand_project: x, r as in ritz_residual and
+// d_out = V^H r; d_tail: |r|^2 (as stored), 0, 0, 0, |r|^2, |x|^2 (h_y, d_y as in ritz_residual). expand_update: t = src -
+// V d_h, with the second pass and the normalisation of expand_small; d_h2: room for 2 m + 2 doubles; d_nrm[0] = |src|^2 is
+// read, d_nrm[2] = |t|^2 written.
+template <typename T>
+bool expand_project(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *h_y, double *d_y, double theta, T *x, T *r, double *d_out,
+                    double *d_tail, double *scratch, hipStream_t s);
+template <typename T>
+bool expand_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h, const T *src, T *t, double eta2, double *d_h2, double *d_nrm,
+                   double *scratch, hipStream_t s);
 // x *= 1 / sqrt(d_nrm2[0]) (the squared norm read on the device).
 template <typename T>
 void scale_by_inv_norm(int64_t n, T *x, const double *d_nrm2, hipStream_t s);
