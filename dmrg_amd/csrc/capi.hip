@@ -164,7 +164,7 @@ void time_block_vectors(int64_t n, int m, int nrep, float ms[3], double bytes[3]
         ms[1]    = timed([&] { gemv_update<T>(n, m, V, n, d, -1.0, 1.0, y, s); });
         bytes[1] = static_cast<double>(m + 2) * n * es;
         // Ritz vector and residual x = V y, r = W y - theta x: reads 2m, writes 2
-        ms[2]    = timed([&] { ritz_residual<T>(n, m, V, W, n, h.data(), d, 0.5, x, r, d + 2 * VEC_MAX_M, scr.as<double>(), s); });
+        ms[2]    = timed([&] { ritz_residual<T>(n, m, V, W, n, h.data(), d, 0.5, x, r, d + 2 * VEC_MAX_M, nullptr, scr.as<double>(), s); });
         bytes[2] = static_cast<double>(2 * m + 2) * n * es;
     } catch(...) {
         if(e0) (void) hipEventDestroy(e0);

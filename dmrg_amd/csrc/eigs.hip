@@ -303,16 +303,32 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
         op->diagonal(diag.p, s);
     }
 
+    std::vector<cx> H(static_cast<size_t>(mmax) * mmax, cx(0.0, 0.0));
+    auto            Hat = [&](int i, int j) -> cx & { return H[i + static_cast<size_t>(mmax) * j]; };
+
     // ---- initial basis
-    int m = 0;
-    if(init && k0 > 0) {
+    int  m = 0;
+    bool projected = false; // W and H hold the initial basis already
+    auto accepted  = [&]() { return host[SB_NRM + 2] > 1e4 * eps_t * eps_t * host[SB_NRM] && host[SB_NRM] > 0; };
+    if(init && k0 == 1) { // one vector: its matvec does not wait for the test of its norm
+        DMRG_HIP_CHECK(hipMemcpyAsync(Vp, init, vbytes, hipMemcpyDeviceToDevice, s));
+        orthonormalize_into(Vp, 0, sm + SB_NRM, sm + SB_NRM + 2);
+        matvec(Vp, Wp, 1);
+        multidot_to_host<T>(n, 1, Vp, n, Wp, sm, host, SB_NRM, 4, scratch.as<double>(), s);
+        DMRG_HIP_CHECK(hipStreamSynchronize(s));
+        if(accepted()) {
+            m         = 1;
+            projected = true;
+            Hat(0, 0) = cx(host[SB_COL], host[SB_COL + 1]);
+        }
+    } else if(init && k0 > 0) {
         DMRG_HIP_CHECK(hipMemcpyAsync(Vp, init, vbytes * k0, hipMemcpyDeviceToDevice, s));
         for(int j = 0; j < k0; ++j) {
             if(j != m) DMRG_HIP_CHECK(hipMemcpyAsync(Vp + m * n, Vp + j * n, vbytes, hipMemcpyDeviceToDevice, s));
             orthonormalize_into(Vp + m * n, m, sm + SB_NRM, sm + SB_NRM + 2);
             DMRG_HIP_CHECK(hipMemcpyAsync(host + SB_NRM, sm + SB_NRM, 4 * sizeof(double), hipMemcpyDeviceToHost, s));
             DMRG_HIP_CHECK(hipStreamSynchronize(s));
-            if(host[SB_NRM + 2] > 1e4 * eps_t * eps_t * host[SB_NRM] && host[SB_NRM] > 0) ++m;
+            if(accepted()) ++m;
         }
     }
     if(m == 0) {
@@ -320,11 +336,9 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
         orthonormalize_into(Vp, 0, sm + SB_NRM, sm + SB_NRM + 2);
         m = 1;
     }
-    matvec(Vp, Wp, m);
+    if(!projected) matvec(Vp, Wp, m);
     st.matvecs += m;
-    std::vector<cx> H(static_cast<size_t>(mmax) * mmax, cx(0.0, 0.0));
-    auto            Hat = [&](int i, int j) -> cx & { return H[i + static_cast<size_t>(mmax) * j]; };
-    for(int j = 0; j < m; ++j) {
+    for(int j = 0; j < m && !projected; ++j) {
         multidot_to_host<T>(n, m, Vp, n, Wp + j * n, sm + SB_COL, host + SB_COL, 0, 0, scratch.as<double>(), s);
         DMRG_HIP_CHECK(hipStreamSynchronize(s));
         for(int i = 0; i < m; ++i) Hat(i, j) = cx(host[SB_COL + 2 * i], host[SB_COL + 2 * i + 1]);
@@ -354,14 +368,13 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
     };
     auto ritz_launch = [&](int col_in_H, int m_, T *xout) {
         ritz_coefficients(col_in_H, m_);
-        ritz_residual<T>(n, m_, Vp, Wp, n, host + SB_Y, sm + SB_Y, w[col_in_H], xout, r, sm + SB_RITZ, scratch.as<double>(), s);
+        ritz_residual<T>(n, m_, Vp, Wp, n, host + SB_Y, sm + SB_Y, w[col_in_H], xout, r, sm + SB_RITZ, host + SB_RITZ, scratch.as<double>(), s);
     };
     auto ritz_norm = [&]() { // |r| / |x| from the host copy of SB_RITZ
         return std::sqrt(std::max(0.0, host[SB_RITZ])) / std::sqrt(std::max(1e-300, host[SB_RITZ + 1]));
     };
     auto ritz = [&](int col_in_H, int m_, T *xout) -> double {
         ritz_launch(col_in_H, m_, xout);
-        DMRG_HIP_CHECK(hipMemcpyAsync(host + SB_RITZ, sm + SB_RITZ, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
         DMRG_HIP_CHECK(hipStreamSynchronize(s));
         return ritz_norm();
     };
@@ -463,8 +476,10 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
     };
 
     std::vector<double> rn(nev, 0.0);
+    int                 formed = 0; // pairs whose vectors and residual norms belong to the current basis
     while(true) {
         rayleigh_ritz();
+        formed = 0;
         // One wanted pair and no restart due: the residual check is deferred to the single synchronisation
         // of the iteration, and the expansion is computed meanwhile (discarded if the pair has converged).
         // (Not with correction solves: their FP32 matvecs would be lost on a pair that has converged.)
@@ -501,6 +516,7 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
             if(refined) qr_fetch();
             DMRG_HIP_CHECK(hipStreamSynchronize(s));
             rn[0]    = ritz_norm();
+            formed   = 1;
             st.nconv = converged(rn[0], w[ord[0]], 0) ? 1 : 0;
             if(st.nconv == 1) break; // converged: the expansion is dropped (m unchanged)
             if(rn[0] < 0.9 * best_r) {
@@ -518,7 +534,8 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
         // Residuals of the wanted pairs in order; stop at the first unconverged one (its r drives expansion).
         int pstar = -1;
         for(int q = 0; q < nev && q < m; ++q) {
-            rn[q] = ritz(ord[q], m, out + q * n);
+            rn[q]  = ritz(ord[q], m, out + q * n);
+            formed = q + 1;
             if(!converged(rn[q], w[ord[q]], q)) {
                 pstar = q;
                 break;
@@ -579,8 +596,10 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
             std::vector<cx> Q(static_cast<size_t>(m) * k);
             for(int j = 0; j < k; ++j)
                 for(int i = 0; i < m; ++i) Q[i + static_cast<size_t>(m) * j] = Qc[j][i];
-            transform_basis(Vp, m, Q, k);
-            transform_basis(Wp, m, Q, k);
+            if(!rotate_basis<T>(n, m, k, n, Vp, Wp, Q.data(), s)) {
+                transform_basis(Vp, m, Q, k);
+                transform_basis(Wp, m, Q, k);
+            }
             std::vector<cx> HQ(static_cast<size_t>(m) * k, cx(0.0, 0.0)), Hn(static_cast<size_t>(k) * k, cx(0.0, 0.0));
             for(int j = 0; j < k; ++j)
                 for(int l = 0; l < m; ++l)
@@ -617,7 +636,7 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
                     Rs[j + static_cast<size_t>(k) * j] = nr;
                     for(int l = 0; l < m; ++l) Qs[l + static_cast<size_t>(m) * j] = nr > 0 ? c[l] / nr : cx(0.0, 0.0);
                 }
-                transform_basis(Qr.as<T>(), m, Qs, k);
+                if(!rotate_basis<T>(n, m, k, n, Qr.as<T>(), nullptr, Qs.data(), s)) transform_basis(Qr.as<T>(), m, Qs, k);
                 std::fill(Rr.begin(), Rr.end(), cx(0.0, 0.0));
                 for(int j = 0; j < k; ++j)
                     for(int i = 0; i <= j; ++i) Rat(i, j) = Rs[i + static_cast<size_t>(k) * j];
@@ -653,9 +672,9 @@ EigsStats Davidson<T>::solve(const EigsParams &p, const T *init, int k0, T *out,
         ++st.iters;
     }
 
-    // ---- outputs: nkeep Ritz vectors (the first nconv were formed in the last pass already)
+    // ---- outputs: nkeep Ritz vectors, the first of them formed in the last pass already
     for(int q = 0; q < std::min(nkeep, m); ++q) {
-        const double rq = ritz(ord[q], m, out + q * n);
+        const double rq = q < formed ? rn[q] : ritz(ord[q], m, out + q * n);
         if(q < nev) {
             evals[q]  = w[ord[q]];
             rnorms[q] = rq;

@@ -449,7 +449,7 @@ struct RitzCoef {
 template <typename T>
 __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *y,
                                                           const RitzCoef c, double theta, T *x, T *r, double *partial, unsigned *counter,
-                                                          double *out) {
+                                                          double *out, HostCopy hc) {
     __shared__ double ys[2 * VEC_MAX_M];
     __shared__ double red[2][VT_THREADS / 64];
     if(y) {
@@ -472,27 +472,29 @@ __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, cons
         publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
         publish(partial + 2 * blockIdx.x + 1, acc[1], counter != nullptr);
     }
-    if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
+    if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter, hc);
 }
 
 template <typename T>
 static void ritz_launch(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *d_y, const RitzCoef &c, double theta, T *x, T *r,
-                        double *d_out, double *scratch, hipStream_t s) {
+                        double *d_out, double *h_out, double *scratch, hipStream_t s) {
+    HostCopy hc;
+    hc.h_out = h_out;
     DMRG_REQUIRE(m <= VEC_MAX_M, DMRG_ERR_ARG, "ritz: too many columns");
     const int g = grid_for(n);
     if(fused(g, 2)) {
         hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch,
-                           scratch_counter(scratch), d_out);
+                           scratch_counter(scratch), d_out, hc);
     } else {
-        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch, nullptr, nullptr);
-        hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_out, -1, nullptr, nullptr, HostCopy{});
+        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch, nullptr, nullptr, hc);
+        hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_out, -1, nullptr, nullptr, hc);
     }
     DMRG_HIP_CHECK(hipGetLastError());
 }
 
 template <typename T>
 void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *h_y, double *d_y, double theta, T *x, T *r,
-                   double *d_out, double *scratch, hipStream_t s) {
+                   double *d_out, double *h_out, double *scratch, hipStream_t s) {
     RitzCoef c{};
     if(m <= RITZ_ARGS) {
         std::copy(h_y, h_y + 2 * m, c.y);
@@ -500,7 +502,7 @@ void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const d
     } else {
         DMRG_HIP_CHECK(hipMemcpyAsync(d_y, h_y, 2 * static_cast<size_t>(m) * sizeof(double), hipMemcpyHostToDevice, s));
     }
-    ritz_launch<T>(n, m, V, W, ld, d_y, c, theta, x, r, d_out, scratch, s);
+    ritz_launch<T>(n, m, V, W, ld, d_y, c, theta, x, r, d_out, h_out, scratch, s);
 }
 
 // ------------------------------------------------------------------------------------------- expansion of a small basis
@@ -823,6 +825,57 @@ bool expand_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h,
     return true;
 }
 
+// ------------------------------------------------------------------------------------------- basis rotation
+// B[:, 0:k] <- B[:, 0:m] Q in place for up to two bases: a thread owns a row, reads its m values and writes k, so that a basis
+// is read and written once; Q comes with the launch. Bounded by the launch up to about 10^5 rows, by memory beyond. As a
+// GEMM with Q's upload, a copy back and a synchronisation per basis, a restart cost about 100 us in a sweep's small solves.
+constexpr int ROT_MAX_M = 24;  // a row's values in registers
+constexpr int ROT_ARGS  = 448; // doubles of Q (3.5 KiB of kernel arguments)
+struct RotationCoef {
+    double q[ROT_ARGS];
+};
+template <typename T>
+__global__ __launch_bounds__(VT_THREADS) void rotate_basis_kernel(int64_t n, int m, int k, int64_t ldv, T *B0, T *B1, const RotationCoef c) {
+    T            *B = blockIdx.y == 0 ? B0 : B1;
+    const int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x;
+    if(i >= n) return;
+    T v[ROT_MAX_M];
+#pragma unroll
+    for(int a = 0; a < ROT_MAX_M; ++a)
+        if(a < m) v[a] = B[i + a * ldv];
+    for(int j = 0; j < k; ++j) {
+        double re = 0, im = 0;
+#pragma unroll
+        for(int a = 0; a < ROT_MAX_M; ++a)
+            if(a < m) {
+                double vr, vi;
+                ld(v[a], vr, vi);
+                if constexpr(vtraits<T>::cx) {
+                    const double qr = c.q[2 * (j * m + a)], qi = c.q[2 * (j * m + a) + 1];
+                    re += vr * qr - vi * qi;
+                    im += vr * qi + vi * qr;
+                } else {
+                    re += vr * c.q[j * m + a];
+                }
+            }
+        B[i + j * ldv] = mk<T>(re, im);
+    }
+}
+
+template <typename T>
+bool rotate_basis(int64_t n, int m, int k, int64_t ldv, T *B0, T *B1, const std::complex<double> *Q, hipStream_t s) {
+    const int64_t blocks = (n + VT_THREADS - 1) / VT_THREADS;
+    if(m > ROT_MAX_M || k > m || m * k * (vtraits<T>::cx ? 2 : 1) > ROT_ARGS || blocks >= (int64_t(1) << 31)) return false;
+    RotationCoef c{};
+    for(int i = 0; i < m * k; ++i) {
+        if constexpr(vtraits<T>::cx) c.q[2 * i] = Q[i].real(), c.q[2 * i + 1] = Q[i].imag();
+        else c.q[i] = Q[i].real();
+    }
+    hipLaunchKernelGGL(rotate_basis_kernel<T>, dim3(static_cast<unsigned>(blocks), B1 ? 2 : 1), dim3(VT_THREADS), 0, s, n, m, k, ldv, B0, B1, c);
+    DMRG_HIP_CHECK(hipGetLastError());
+    return true;
+}
+
 // ------------------------------------------------------------------------------------------- elementwise
 template <typename T>
 __global__ void scale_inv_norm_kernel(int64_t n, T *x, const double *nrm2) {
@@ -1056,7 +1109,7 @@ void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t
     template void multidot<T>(int64_t, int, const T *, int64_t, const T *, double *, double *, hipStream_t);          \
     template void gemv_update<T>(int64_t, int, const T *, int64_t, const double *, double, double, T *, hipStream_t); \
     template void ritz_residual<T>(int64_t, int, const T *, const T *, int64_t, const double *, double *, double, T *,  \
-                                   T *, double *, double *, hipStream_t);                                              \
+                                   T *, double *, double *, double *, hipStream_t);                                    \
     template void multidot_to_host<T>(int64_t, int, const T *, int64_t, const T *, double *, double *, int, int, double *, hipStream_t);\
     template bool expand_small<T>(int64_t, int, const T *, const T *, int64_t, const double *, double, T *, T *, const T *, T *, double,\
                                   double *, double *, hipStream_t);                                                   \
@@ -1064,6 +1117,7 @@ void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t
                                     double *, double *, double *, hipStream_t);                                       \
     template bool expand_update<T>(int64_t, int, const T *, int64_t, const double *, const T *, T *, double, double *, double *,\
                                    double *, hipStream_t);                                                            \
+    template bool rotate_basis<T>(int64_t, int, int, int64_t, T *, T *, const std::complex<double> *, hipStream_t);   \
     template void scale_by_inv_norm<T>(int64_t, T *, const double *, hipStream_t);                                    \
     template void scale<T>(int64_t, T *, double, hipStream_t);                                                         \
     template void random_fill<T>(int64_t, T *, uint64_t, hipStream_t);                                               \

@@ -70,10 +70,11 @@ void multidot_dgks(int64_t n, int m, const T *V, int64_t ldv, const T *x, double
 template <typename T>
 void gemv_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h, double alpha, double beta, T *x, hipStream_t s);
 // x = V y, r = W y - theta x, d_out[0] = |r|^2, d_out[1] = |x|^2 (h_y: m complex doubles on the host, pinned; d_y: room for
-// them on the device, used when they are too many for the launch's arguments; h_y is then read by a queued copy).
+// them on the device, used when they are too many for the launch's arguments; h_y is then read by a queued copy). h_out
+// (pinned host memory, optional): the two norms there as well, valid after a synchronisation.
 template <typename T>
 void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const double *h_y, double *d_y, double theta, T *x, T *r,
-                   double *d_out, double *scratch, hipStream_t s);
+                   double *d_out, double *h_out, double *scratch, hipStream_t s);
 // Small problems in one launch, false for others: with W, x = V y, r = W y - theta x and d_ritz as in ritz_residual (h_y on
 // the host), src = r; then t = src orthogonalised against V[:, 0:m] and normalised, a second pass taken where the first one
 // leaves less than eta2 of the squared norm; d_nrm[0] = |src|^2, d_nrm[2] = |t|^2 before the normalisation. src may be t.
@@ -90,6 +91,10 @@ bool expand_project(int64_t n, int m, const T *V, const T *W, int64_t ldv, const
 template <typename T>
 bool expand_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h, const T *src, T *t, double eta2, double *d_h2, double *d_nrm,
                    double *scratch, hipStream_t s);
+// B[:, 0:k] <- B[:, 0:m] Q for B0 and, unless null, B1 (Q: m x k on the host, its real part for real T); false where m or Q
+// is too large for one launch's registers and arguments.
+template <typename T>
+bool rotate_basis(int64_t n, int m, int k, int64_t ldv, T *B0, T *B1, const std::complex<double> *Q, hipStream_t s);
 // x *= 1 / sqrt(d_nrm2[0]) (the squared norm read on the device).
 template <typename T>
 void scale_by_inv_norm(int64_t n, T *x, const double *d_nrm2, hipStream_t s);
