@@ -35,14 +35,17 @@ int zero_rows(const cx *K, double tol) {
 }
 
 template <typename T>
-void mixed_block_impl(MatVecOp &h1, MatVecOp &h2, const T *theta, int mode, T *mixed, MixedBlockResult &res, hipStream_t s) {
+void mixed_block_impl(MatVecOp &h1, MatVecOp &h2, const T *theta, int mode, T *mixed, MixedBlockResult &res, hipStream_t s,
+                      MixedBlockWorkspace &ws) {
     const int64_t n = h1.D.n();
-    DevBuf        Vb, HVb, dev, scr;
+    DevBuf       &Vb = ws.V, &HVb = ws.HV, &dev = ws.dev, &scr = ws.scr;
     Vb.reserve(3 * static_cast<size_t>(n) * sizeof(T));
     HVb.reserve(3 * static_cast<size_t>(n) * sizeof(T));
     dev.reserve(64 * sizeof(double));
-    scr.reserve(static_cast<size_t>(vec_scratch_doubles()) * sizeof(double));
-    vec_scratch_init(scr.as<double>(), s);
+    if(!scr.p) {
+        scr.reserve(static_cast<size_t>(vec_scratch_doubles()) * sizeof(double));
+        vec_scratch_init(scr.as<double>(), s);
+    }
     T      *V = Vb.as<T>(), *HV = HVb.as<T>();
     double *d = dev.as<double>(), *sc = scr.as<double>();
     auto    col = [&](T *B, int j) { return B + static_cast<int64_t>(j) * n; };
@@ -55,7 +58,7 @@ void mixed_block_impl(MatVecOp &h1, MatVecOp &h2, const T *theta, int mode, T *m
     // Modified Gram-Schmidt (env.cpp:74-93): a column of norm < eps stays as it is and later columns are not
     // projected against it.
     double nrm2[2];
-    for(int i = 0; i < 3; ++i) {
+    for(int i = gram_schmidt3<T>(n, V, std::numeric_limits<double>::epsilon(), s) ? 3 : 0; i < 3; ++i) {
         multidot_x<T>(n, 0, V, n, col(V, i), d, d + 2, nullptr, sc, s);
         DMRG_HIP_CHECK(hipMemcpyAsync(nrm2, d + 2, 2 * sizeof(double), hipMemcpyDeviceToHost, s));
         DMRG_HIP_CHECK(hipStreamSynchronize(s));
@@ -72,13 +75,15 @@ void mixed_block_impl(MatVecOp &h1, MatVecOp &h2, const T *theta, int mode, T *m
     cx K1[9], K2[9];
     for(int op = 0; op < 2; ++op) {
         (op == 0 ? h1 : h2).multax_device(V, n, HV, n, 3, s, false);
-        for(int j = 0; j < 3; ++j) multidot<T>(n, 3, V, n, col(HV, j), d + 8 + 6 * j, sc, s);
-        double host[18];
-        DMRG_HIP_CHECK(hipMemcpyAsync(host, d + 8, 18 * sizeof(double), hipMemcpyDeviceToHost, s));
-        DMRG_HIP_CHECK(hipStreamSynchronize(s));
+        for(int j = 0; j < 3; ++j) multidot<T>(n, 3, V, n, col(HV, j), d + 8 + 18 * op + 6 * j, sc, s);
+    }
+    double host[36];
+    DMRG_HIP_CHECK(hipMemcpyAsync(host, d + 8, 36 * sizeof(double), hipMemcpyDeviceToHost, s));
+    DMRG_HIP_CHECK(hipStreamSynchronize(s));
+    for(int op = 0; op < 2; ++op) {
         cx K[9];
         for(int j = 0; j < 3; ++j)
-            for(int i = 0; i < 3; ++i) K[i + 3 * j] = cx(host[6 * j + 2 * i], host[6 * j + 2 * i + 1]);
+            for(int i = 0; i < 3; ++i) K[i + 3 * j] = cx(host[18 * op + 6 * j + 2 * i], host[18 * op + 6 * j + 2 * i + 1]);
         lower_hermitian(K, op == 0 ? K1 : K2);
     }
     // K3 = K2 - K1 K1, then the mode's decoupling (env.cpp:166-176)
@@ -115,12 +120,7 @@ void mixed_block_impl(MatVecOp &h1, MatVecOp &h2, const T *theta, int mode, T *m
     for(int i = 1; i < 3; ++i)
         if(std::abs(Z[i + 3 * opt]) > std::abs(Z[kmax + 3 * opt])) kmax = i;
     const cx ph = std::abs(Z[kmax + 3 * opt]) > 0 ? Z[kmax + 3 * opt] / std::abs(Z[kmax + 3 * opt]) : cx(1.0, 0.0);
-    double   c[6];
-    for(int i = 0; i < 3; ++i) {
-        res.alpha[i] = (Z[i + 3 * opt] / ph).real();
-        c[2 * i]     = res.alpha[i];
-        c[2 * i + 1] = 0.0;
-    }
+    for(int i = 0; i < 3; ++i) res.alpha[i] = (Z[i + 3 * opt] / ph).real();
     res.opt_val = w[opt];
     res.opt_idx = opt;
     for(int i = 0; i < 9; ++i) {
@@ -128,21 +128,23 @@ void mixed_block_impl(MatVecOp &h1, MatVecOp &h2, const T *theta, int mode, T *m
         res.K2[2 * i] = K2[i].real(), res.K2[2 * i + 1] = K2[i].imag();
         res.K3[2 * i] = K3[i].real(), res.K3[2 * i + 1] = K3[i].imag();
     }
-    DMRG_HIP_CHECK(hipMemcpyAsync(d + 30, c, 6 * sizeof(double), hipMemcpyHostToDevice, s));
-    gemv_update<T>(n, 3, V, n, d + 30, 1.0, 0.0, mixed, s); // mixed = V col
-    DMRG_HIP_CHECK(hipStreamSynchronize(s));                  // the local buffers die at return
+    combine3<T>(n, V, res.alpha, mixed, s);
 }
 
 } // namespace
 
-void optimally_mixed_block(MatVecOp &h1, MatVecOp &h2, const void *theta, int mode, void *mixed, MixedBlockResult &res, hipStream_t s) {
+void optimally_mixed_block(MatVecOp &h1, MatVecOp &h2, const void *theta, int mode, void *mixed, MixedBlockResult &res, hipStream_t s,
+                           MixedBlockWorkspace *kept) {
     DMRG_REQUIRE(h1.dtype == h2.dtype, DMRG_ERR_ARG, "mixed block: both operators must have the same dtype");
     DMRG_REQUIRE(h1.D.d == h2.D.d && h1.D.chiL == h2.D.chiL && h1.D.chiR == h2.D.chiR, DMRG_ERR_DIMS,
                  "mixed block: operators act on different shapes");
-    if(h1.dtype == DMRG_FP64) mixed_block_impl<double>(h1, h2, static_cast<const double *>(theta), mode, static_cast<double *>(mixed), res, s);
+    MixedBlockWorkspace  local;
+    MixedBlockWorkspace &ws = kept ? *kept : local;
+    if(h1.dtype == DMRG_FP64) mixed_block_impl<double>(h1, h2, static_cast<const double *>(theta), mode, static_cast<double *>(mixed), res, s, ws);
     else if(h1.dtype == DMRG_CX64)
-        mixed_block_impl<cpx<double>>(h1, h2, static_cast<const cpx<double> *>(theta), mode, static_cast<cpx<double> *>(mixed), res, s);
+        mixed_block_impl<cpx<double>>(h1, h2, static_cast<const cpx<double> *>(theta), mode, static_cast<cpx<double> *>(mixed), res, s, ws);
     else throw Error(DMRG_ERR_ARG, "mixed block: FP64 or CX64 operators only");
+    if(!kept) DMRG_HIP_CHECK(hipStreamSynchronize(s)); // the local buffers die at return
 }
 
 } // namespace dmrg

@@ -88,6 +88,7 @@ struct Fdmrg {
     std::vector<int64_t>                      chi;           // chi[0..L]
     std::vector<DevBuf>                       EL, ER, EL2, ER2; // EL[i]: left of site i; ER[i]: right of site i
     DevBuf                                    theta, theta2, xbuf, ws, tmp, sdev, dense;
+    MixedBlockWorkspace                       mixed_ws;
     DeviceSvd                                 svd;
     std::unique_ptr<MatVecOp>                 hop, h2op;
     std::unique_ptr<Davidson<T>>              dav;
@@ -431,7 +432,7 @@ struct Fdmrg {
         xbuf.reserve(static_cast<size_t>(n) * es());
         MixedBlockResult mr;
         const auto       t0 = clock::now();
-        optimally_mixed_block(H1, H2, theta.p, cfg.expand_mode & 3, xbuf.p, mr, s);
+        optimally_mixed_block(H1, H2, theta.p, cfg.expand_mode & 3, xbuf.p, mr, s, &mixed_ws);
         t_expand += std::chrono::duration<double>(clock::now() - t0).count();
         ++res->expansions;
         split_two(i, !right, xbuf.as<T>());

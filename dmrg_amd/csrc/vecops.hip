@@ -876,6 +876,75 @@ bool rotate_basis(int64_t n, int m, int k, int64_t ldv, T *B0, T *B1, const std:
     return true;
 }
 
+// ------------------------------------------------------------------------------------------- Gram-Schmidt on three vectors
+// Modified Gram-Schmidt on the columns of V (n x 3) in one workgroup, a thread owning its rows throughout: a column of norm
+// below eps stays as it is and later ones are not projected against it. Column by column from the host, the norms cost three
+// synchronisations and twelve launches. Bounded by latency up to the limit (about 1 us per pass), by one CU's loads beyond.
+constexpr int64_t GS3_MAX_BYTES = 131072;
+template <typename T>
+__global__ __launch_bounds__(EX_THREADS) void gram_schmidt3_kernel(int n, T *V, double eps) {
+    __shared__ double red[4][EX_WAVES];
+    for(int i = 0; i < 3; ++i) {
+        T     *vi      = V + static_cast<int64_t>(i) * n;
+        double nrm2[1] = {0.0};
+        for(int k = threadIdx.x; k < n; k += EX_THREADS) {
+            double re, im;
+            ld(vi[k], re, im);
+            nrm2[0] += re * re + im * im;
+        }
+        all_sum<1>(nrm2, red);
+        const double rii = sqrt(nrm2[0]);
+        if(rii < eps) continue; // the same in every thread
+        const double a = 1.0 / rii;
+        double       h[4] = {0.0, 0.0, 0.0, 0.0};
+        for(int k = threadIdx.x; k < n; k += EX_THREADS) {
+            double re, im;
+            ld(vi[k], re, im);
+            const T q = mk<T>(a * re, a * im);
+            vi[k]     = q;
+            ld(q, re, im);
+            for(int j = i + 1; j < 3; ++j) {
+                double xr, xi;
+                ld(V[static_cast<int64_t>(j) * n + k], xr, xi);
+                h[2 * (j - i - 1)] += re * xr + im * xi;
+                h[2 * (j - i - 1) + 1] += re * xi - im * xr;
+            }
+        }
+        all_sum<4>(h, red);
+        for(int k = threadIdx.x; k < n; k += EX_THREADS) {
+            double re, im;
+            ld(vi[k], re, im);
+            for(int j = i + 1; j < 3; ++j) {
+                const double hr = h[2 * (j - i - 1)], hi = h[2 * (j - i - 1) + 1];
+                double       xr, xi;
+                ld(V[static_cast<int64_t>(j) * n + k], xr, xi);
+                V[static_cast<int64_t>(j) * n + k] = mk<T>(xr - (re * hr - im * hi), xi - (re * hi + im * hr));
+            }
+        }
+    }
+}
+template <typename T>
+bool gram_schmidt3(int64_t n, T *V, double eps, hipStream_t s) {
+    if(n * static_cast<int64_t>(sizeof(T)) > GS3_MAX_BYTES) return false;
+    hipLaunchKernelGGL(gram_schmidt3_kernel<T>, dim3(1), dim3(EX_THREADS), 0, s, static_cast<int>(n), V, eps);
+    DMRG_HIP_CHECK(hipGetLastError());
+    return true;
+}
+
+template <typename T>
+__global__ void combine3_kernel(int64_t n, const T *V, double c0, double c1, double c2, T *out) {
+    for(int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+        double a[3][2];
+        for(int j = 0; j < 3; ++j) ld(V[i + j * n], a[j][0], a[j][1]);
+        out[i] = mk<T>(c0 * a[0][0] + c1 * a[1][0] + c2 * a[2][0], c0 * a[0][1] + c1 * a[1][1] + c2 * a[2][1]);
+    }
+}
+template <typename T>
+void combine3(int64_t n, const T *V, const double *c, T *out, hipStream_t s) {
+    hipLaunchKernelGGL(combine3_kernel<T>, dim3(ew_grid(n)), dim3(VT_THREADS), 0, s, n, V, c[0], c[1], c[2], out);
+    DMRG_HIP_CHECK(hipGetLastError());
+}
+
 // ------------------------------------------------------------------------------------------- elementwise
 template <typename T>
 __global__ void scale_inv_norm_kernel(int64_t n, T *x, const double *nrm2) {
@@ -1118,6 +1187,8 @@ void cg_step(int64_t n, const T *x, T *p, const T *q, const double *d_dots, T *t
     template bool expand_update<T>(int64_t, int, const T *, int64_t, const double *, const T *, T *, double, double *, double *,\
                                    double *, hipStream_t);                                                            \
     template bool rotate_basis<T>(int64_t, int, int, int64_t, T *, T *, const std::complex<double> *, hipStream_t);   \
+    template bool gram_schmidt3<T>(int64_t, T *, double, hipStream_t);                                                \
+    template void combine3<T>(int64_t, const T *, const double *, T *, hipStream_t);                                  \
     template void scale_by_inv_norm<T>(int64_t, T *, const double *, hipStream_t);                                    \
     template void scale<T>(int64_t, T *, double, hipStream_t);                                                         \
     template void random_fill<T>(int64_t, T *, uint64_t, hipStream_t);                                               \

@@ -95,6 +95,13 @@ bool expand_update(int64_t n, int m, const T *V, int64_t ldv, const double *d_h,
 // is too large for one launch's registers and arguments.
 template <typename T>
 bool rotate_basis(int64_t n, int m, int k, int64_t ldv, T *B0, T *B1, const std::complex<double> *Q, hipStream_t s);
+// Modified Gram-Schmidt on the columns of V (n x 3); a column of norm below eps stays as it is and is not projected out of
+// later ones. False where n is too large for one workgroup.
+template <typename T>
+bool gram_schmidt3(int64_t n, T *V, double eps, hipStream_t s);
+// out = V c for three columns, c real on the host.
+template <typename T>
+void combine3(int64_t n, const T *V, const double *c, T *out, hipStream_t s);
 // x *= 1 / sqrt(d_nrm2[0]) (the squared norm read on the device).
 template <typename T>
 void scale_by_inv_norm(int64_t n, T *x, const double *d_nrm2, hipStream_t s);
