@@ -545,9 +545,9 @@ static pipe::Shape shape_of(TileCfg c, dmrg_dtype t) {
 // Microseconds that the pipelined kernel takes for g in shape s with ks K slices, with loads of W bytes per lane: a CU's
 // workgroups share its matrix cores, so r of them advance one stage in r stage times of MFMA work, but none of them faster
 // than its own chain of barrier, LDS read and MFMA (about 170 clocks beyond its MFMAs), and all of them together no faster
-// than their loads, about 17 clocks each. Within 15 % of the measured times of the matvec legs of chi 24 to 1024 (e.g.
-// FP64 402x165x825: 32x32 tiles 15.7 us, 3 slices 12.5, against 14.6 and 11.9 here; 328x5000x200 with 4-byte loads in
-// 32x32 tiles 28.1, with 16-byte loads in 64x64 tiles 21.7, against 26.6 and 19.5).
+// than their loads, about 17 clocks each. Real stages are too short for workgroups to hide that chain of one another (32x32
+// FP64: 0.165 us a stage with one workgroup on a CU, 0.33 with two; counted so, FP64 300x280 at D = 5 takes 39.1 us instead
+// of 41.2); complex ones hide it (counted alike, 173x211 would take 42.9 us instead of 41.5).
 static double pipe_cost_us(const GemmDesc &g, pipe::Shape s, int ks, int W) {
     const pipe::ShapeInfo i = pipe::shape_info(g.dtype, s);
     const bool   cplx = dtype_is_complex(g.dtype), sp = dtype_is_single(g.dtype);
@@ -556,7 +556,9 @@ static double pipe_cost_us(const GemmDesc &g, pipe::Shape s, int ks, int W) {
     const double mfma   = i.TM * i.TN * (i.BK / 4) * (cplx ? 3 : 1) * (sp ? 32.0 : 64.0);
     const double loads  = (i.BM + i.BN) * i.BK * static_cast<double>(dtype_size(g.dtype)) / (64.0 * W) * 17.0;
     const double tiles  = static_cast<double>((g.M + i.BM - 1) / i.BM) * ((g.N + i.BN - 1) / i.BN) * g.batch * ks;
-    auto         round  = [&](double r) { return stages * std::max({r * mfma * 1.04, r * loads, mfma + 170.0}); };
+    auto         round  = [&](double r) {
+        return stages * (cplx ? std::max({r * mfma * 1.04, r * loads, mfma + 170.0}) : r * std::max(mfma + 150.0, loads));
+    };
     const double per_cu = std::ceil(tiles / cus), full = std::floor(per_cu / i.resident), rest = per_cu - full * i.resident;
     double       us     = 3.0 + (full * (round(i.resident) + 1500.0) + (rest > 0 ? round(rest) : 0.0)) / clk;
     const double out    = static_cast<double>(g.M) * g.N * g.batch * static_cast<double>(dtype_size(g.dtype));
@@ -585,8 +587,16 @@ static std::vector<std::pair<double, LaunchPlan>> ranked_plans(const GemmDesc &g
 }
 
 static LaunchPlan heuristic_plan(const GemmDesc &g) {
-    // The streaming kernel where the columns dominate: below 8 columns per row the tiles' reuse of B is worth more.
-    if((g.M <= 16 || g.N >= 8 * g.M) && stream::takes(g)) return LaunchPlan{TileCfg::SMALLK, 1};
+    // The streaming kernel where the columns dominate: below 8 columns per row the tiles' reuse of B is worth more. Past 256
+    // fragments, laying A out in LDS takes 2 to 7 us, which real GEMMs win back from three 32x32 tiles per CU on and complex
+    // ones (four products against the tiles' three) hardly ever: K = M = 50, N = 960 complex 16.1 us, tiles 6.3; FP64 8.9
+    // against 6.0, at N = 32964 16 against 26.
+    if(stream::takes(g) && (g.M <= 16 || g.N >= 8 * g.M)) {
+        const int64_t fragments = static_cast<int64_t>((g.M + 15) / 16) * ((g.K + 3) / 4) * 64;
+        const int64_t tiles     = static_cast<int64_t>((g.M + 31) / 32) * ((g.N + 31) / 32) * g.batch;
+        if(g.M <= 16 || fragments <= 256 || (!dtype_is_complex(g.dtype) && tiles >= 3 * static_cast<int64_t>(device_cu_count())))
+            return LaunchPlan{TileCfg::SMALLK, 1};
+    }
     if(g.M <= 16) return LaunchPlan{TileCfg::T16x128, 1};
     return ranked_plans(g).front().second;
 }
