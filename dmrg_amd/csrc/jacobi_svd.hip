@@ -443,9 +443,16 @@ __global__ __launch_bounds__(512) void jacobi_resident(int m, int n, int tr, con
         if(lane == 0) nrm[j] = sqrt(a), perm[j] = j;
     }
     __syncthreads();
-    if(tid < n) { // descending, equal ones in their order
+    // Descending, equal ones in their order, NaN before all numbers: a total order, so that every rank is taken once and a
+    // column that is not a number stands in S.
+    if(tid < n) {
         int rank = 0;
-        for(int i = 0; i < n; ++i) rank += nrm[i] > nrm[tid] || (nrm[i] == nrm[tid] && i < tid) ? 1 : 0;
+        const double mine = nrm[tid];
+        for(int i = 0; i < n; ++i) {
+            const double other = nrm[i];
+            if(other != other) rank += mine == mine || i < tid ? 1 : 0;
+            else rank += other > mine || (other == mine && i < tid) ? 1 : 0;
+        }
         perm[rank] = tid;
         S[rank]    = nrm[tid];
     }
