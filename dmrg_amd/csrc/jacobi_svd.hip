@@ -28,28 +28,23 @@ struct jtraits<cpx<double>> {
     static constexpr bool cx = true;
 };
 
-// |gr + i gi| (gi = 0 for real T) without leaving the range: inner products of columns of norm 1e-130 are 1e-260.
+// |gr + i gi| (gi = 0 for real T), the inner product of two columns of squared norms al and be, where they are to be rotated,
+// else 0. A column whose squared norm is zero counts as a zero column, also where rounding has left something below 1e-162 in
+// it: linearly dependent columns shrink by eps a sweep. Norms of 1e130 or 1e-130 have products and squared products outside
+// the range; where al be is well inside, so are the others as far as they matter (|g|^2 <= al be), which one test of al be on
+// the serial chain of a round decides (tests of each root cost the block path 3 %).
 template <typename T>
-__device__ inline double magnitude(double gr, double gi) {
-    if constexpr(jtraits<T>::cx) {
-        double g = sqrt(gr * gr + gi * gi);
-        if(__builtin_expect(g < 1e-140, 0)) {
-            constexpr double up = 0x1p+500;
-            g                   = sqrt((gr * up) * (gr * up) + (gi * up) * (gi * up)) / up;
-        }
-        return g;
-    } else {
-        return fabs(gr);
+__device__ inline double coupling(double gr, double gi, double al, double be, double tol) {
+    const double p = al * be, g2 = jtraits<T>::cx ? gr * gr + gi * gi : gr * gr;
+    if(__builtin_expect(!(p > 1e-240 && p < 1e240), 0)) {
+        const double top = fmax(fabs(gr), fabs(gi)), f = top < 1.0 ? 0x1p+520 : 0x1p-520;
+        const double g = jtraits<T>::cx ? sqrt((gr * f) * (gr * f) + (gi * f) * (gi * f)) / f : fabs(gr);
+        const double b = sqrt(al) * sqrt(be);
+        return g > tol * b && b > 0.0 ? g : 0.0;
     }
+    return g2 > (tol * tol) * p ? (jtraits<T>::cx ? sqrt(g2) : fabs(gr)) : 0.0;
 }
 
-// Whether columns of squared norms al and be with inner product g are rotated. A column whose squared norm is zero counts as
-// a zero column, also where rounding has left something below 1e-162 in it: linearly dependent columns shrink by eps a sweep.
-__device__ inline bool rotates(double g, double al, double be, double tol) {
-    double b = sqrt(al * be);
-    if(__builtin_expect(b < 1e-140, 0)) b = sqrt(al) * sqrt(be);
-    return g > tol * b && b > 0.0;
-}
 // The smaller root of t^2 + 2 z t = 1, of z's sign.
 __device__ inline double tangent(double z) {
     if(fabs(z) > 1e150) return 0.5 / z; // z^2 leaves the range
@@ -116,8 +111,8 @@ __global__ __launch_bounds__(NT) void jacobi_round(int m, int n, int np, int r, 
 #pragma unroll
         for(int k = 0; k < NT / 64; ++k) al += red[0][k], be += red[1][k], gr += red[2][k], gi += red[3][k];
     }
-    const double g = magnitude<T>(gr, gi);
-    if(!rotates(g, al, be, tol)) return; // same decision in every thread of the workgroup
+    const double g = coupling<T>(gr, gi, al, be, tol);
+    if(g == 0.0) return; // same decision in every thread of the workgroup
     // Align the phase of column q so that the off-diagonal is |g|, then a real rotation zeroes it:
     // t = sign(z) / (|z| + sqrt(1 + z^2)), z = (be - al) / (2 |g|); w_p' = c w_p - s w_q^, w_q' = s w_p + c w_q^.
     const double z  = (be - al) / (2.0 * g);
@@ -246,8 +241,8 @@ __global__ __launch_bounds__(BJ_THREADS) void bj_eig(int n, int nbp, int r, int 
                 double       gr, gi;
                 if constexpr(jtraits<T>::cx) gr = gm.re, gi = gm.im;
                 else gr = gm, gi = 0.0;
-                const double g  = magnitude<T>(gr, gi);
-                const bool   on = rotates(g, al, be, tol);
+                const double g  = coupling<T>(gr, gi, al, be, tol);
+                const bool   on = g != 0.0;
                 ron[tid]        = on ? 1 : 0;
                 if(on) {
                     const double z = (be - al) / (2.0 * g);
@@ -389,8 +384,8 @@ __global__ __launch_bounds__(512) void jacobi_resident(int m, int n, int tr, con
                 }
                 al = row_sum(al), be = row_sum(be), gr = row_sum(gr);
                 if constexpr(cx) gi = row_sum(gi);
-                const double g = magnitude<T>(gr, gi);
-                if(rotates(g, al, be, tol)) {
+                const double g = coupling<T>(gr, gi, al, be, tol);
+                if(g != 0.0) {
                     // The rotation of jacobi_round: with d = be - al, h = sqrt(d^2 + (2 g)^2) and u = |d| + h the tangent is
                     // sign(d) 2 g / u. d and g are scaled to about 1 first, so that no square leaves the range.
                     const double d0 = be - al, e2 = fmax(fabs(d0), g);
@@ -552,8 +547,8 @@ __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T
                 be = group_sum<G>(be);
                 gr = group_sum<G>(gr);
                 if constexpr(jtraits<T>::cx) gi = group_sum<G>(gi);
-                const double g = magnitude<T>(gr, gi);
-                if(!live || !rotates(g, al, be, tol)) continue;
+                const double g = coupling<T>(gr, gi, al, be, tol);
+                if(!live || g == 0.0) continue;
                 const double z  = (be - al) / (2.0 * g);
                 const double t  = tangent(z);
                 const double c  = 1.0 / sqrt(1.0 + t * t), s = c * t;
