@@ -519,8 +519,11 @@ void ritz_residual(int64_t n, int m, const T *V, const T *W, int64_t ld, const d
 // a sweep of L = 16 at chi = 32 takes 194 ms against 273).
 constexpr int     EX_THREADS = 1024;
 constexpr int     EX_WAVES   = EX_THREADS / 64;
-// One CU reads its caches at about 100 GB/s: up to here that costs less than the launches.
-constexpr int64_t EX_MAX_BYTES = 32768;
+// The vector and, with the Ritz step, the basis elements up to which one CU's loads cost less than the launches. Iterations of
+// solves in one workgroup / in three launches, us: FP64 n = 2048 16.5 / 18.5 at 8 columns, 23.1 / 23.8 at 20, 33.5 / 33.2 at 28;
+// n = 4096 23.4 / 23.5 at 8, 28.1 / 25.3 at 12, 54.8 / 47.3 at 32; complex n = 2048 28.4 / 28.7 at 20, 32.4 / 32.4 at 24.
+constexpr int64_t EX_MAX_BYTES    = 32768;
+constexpr int64_t EX_MAX_ELEMENTS = 40960;
 
 template <typename T>
 struct ExpandArgs {
@@ -640,7 +643,7 @@ __global__ __launch_bounds__(EX_THREADS) void expand_kernel(const ExpandArgs<T> 
 template <typename T>
 bool expand_small(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *h_y, double theta, T *x, T *r, const T *src, T *t,
                   double eta2, double *d_ritz, double *d_nrm, hipStream_t s) {
-    if(n * static_cast<int64_t>(sizeof(T)) > EX_MAX_BYTES || m > RITZ_ARGS) return false;
+    if(n * static_cast<int64_t>(sizeof(T)) > EX_MAX_BYTES || m > RITZ_ARGS || (W && n * m > EX_MAX_ELEMENTS)) return false;
     RitzCoef c{};
     if(W) std::copy(h_y, h_y + 2 * m, c.y);
     const ExpandArgs<T> g{n, ldv, m, V, W, src, x, r, t, theta, eta2, d_ritz, d_nrm};
