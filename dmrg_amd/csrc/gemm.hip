@@ -575,8 +575,7 @@ static std::vector<std::pair<double, LaunchPlan>> ranked_plans(const GemmDesc &g
         const pipe::Shape s = shape_of(c, g.dtype);
         if((c == TileCfg::T128x64 && s != pipe::S128x64) || (c == TileCfg::T64x32 && s != pipe::S64x32)) continue;
         const int    bk = pipe::shape_info(g.dtype, s).BK;
-        pipe::Launch l;
-        const int    W = pipe::describe(g, pipe::shape_info(g.dtype, s), 1, l) ? l.W : 4;
+        const int    W = pipe::load_bytes(g, pipe::shape_info(g.dtype, s));
         for(int ks : {1, 2, 3, 4, 6, 8}) {
             if(ks > 1 && (g.K < 4 * bk * ks || !g.part || g.part_capacity < static_cast<int64_t>(g.M) * g.N * g.batch * ks)) continue;
             v.emplace_back(pipe_cost_us(g, s, ks, W), LaunchPlan{c, ks});
@@ -1167,13 +1166,14 @@ void gemm(const GemmDesc &gin, hipStream_t stream, TileCfg cfg, int ksplit) {
     const bool   large = macs >= static_cast<double>(g_tune_min_macs) || bytes * 16.0 >= static_cast<double>(g_tune_min_macs);
     const bool   tunable  = g_autotune && !g.accumulate && large;
     const bool   can_tune = tunable && cs == hipStreamCaptureStatusNone && !g_tls_no_tune;
-    const std::string key = tune_key(g);
-    LaunchPlan        p;
-    bool              found = false;
+    std::string  key;
+    LaunchPlan   p;
+    bool         found = false;
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         load_tune_cache_locked();
-        auto                        it = g_tuned.find(key);
+        if(can_tune || !g_tuned.empty()) key = tune_key(g);
+        auto it = g_tuned.find(key);
         if(it != g_tuned.end()) {
             p     = it->second;
             found = true;
@@ -1199,6 +1199,10 @@ void gemm(const GemmDesc &gin, hipStream_t stream, TileCfg cfg, int ksplit) {
         const bool        slices = p.ksplit <= 1 || (g.part && g.part_capacity >= static_cast<int64_t>(g.M) * g.N * g.batch * p.ksplit);
         if(shape != pipe::N_SHAPES && p.nsplit <= 0) e.pipelined = prepare_pipelined(oriented(g), shape, slices ? p.ksplit : 1, e.p);
         cache[ck] = e;
+        if(e.pipelined) {
+            run_pipelined(oriented(g), e.p, stream);
+            return;
+        }
     }
     launch_plan(g, p, stream);
 }

@@ -39,15 +39,24 @@ struct Walk {
     int64_t nin, nout, a_in, a_out, b_in, b_out;
     bool    ratio;
 };
-// 128-byte lines that the 64 units of a load touch: the order that touches fewer is taken.
+// 128-byte lines that the 64 units of a load touch, walking K (korder) or the non-K index first.
 int lines(const Idx2 &r, const Idx2 &k, bool korder, int ru, int ku, int kn) {
-    int64_t v[64];
-    for(int u = 0; u < 64; ++u) {
-        const int rl = korder ? u / kn : u % 16, kx = korder ? u % kn : u / 16;
-        v[u] = (idx_off(r, rl * ru) + idx_off(k, kx * ku)) / 128;
+    const int nk = korder ? kn : 4, nr = 64 / nk;
+    int64_t   slot[128], ro[64];
+    std::fill(slot, slot + 128, int64_t(-1));
+    for(int i = 0; i < nr; ++i) ro[i] = idx_off(r, i * ru);
+    int count = 0;
+    for(int j = 0; j < nk; ++j) {
+        const int64_t ko = idx_off(k, j * ku);
+        for(int i = 0; i < nr; ++i) {
+            const int64_t line = (ro[i] + ko) / 128;
+            uint32_t      h    = static_cast<uint32_t>(line ^ (line >> 7)) & 127;
+            while(slot[h] != -1 && slot[h] != line) h = (h + 1) & 127;
+            count += slot[h] == -1 ? 1 : 0;
+            slot[h] = line;
+        }
     }
-    std::sort(v, v + 64);
-    return static_cast<int>(std::unique(v, v + 64) - v);
+    return count;
 }
 
 // es: element size; maps r (extent R) and k in elements; in/out: the walk's strides of this operand.
@@ -72,14 +81,17 @@ bool operand(Operand &o, const void *p, int64_t batch, const Idx2 &r, const Idx2
     magic(o.r.c, o.rmul, o.rsh);
     magic(o.k.c, o.kmul, o.ksh);
     o.sep_r  = separable(o.r, static_cast<uint32_t>(RT));
-    const int kn = ro ? BK : BK / u;
-    o.korder = lines(o.r, o.k, true, ro ? u : 1, ro ? 1 : u, kn) <= lines(o.r, o.k, false, ro ? u : 1, ro ? 1 : u, kn);
     return span(o.r, o.sep_r ? std::min<int64_t>(R, RT) : R) + span(o.k, BK) + 16 < static_cast<int64_t>(0x7fffffff);
 }
 
-} // namespace
+// The order that touches fewer lines.
+void set_order(Operand &o, bool ro, int u, int BK) {
+    const int kn = ro ? BK : BK / u;
+    o.korder     = lines(o.r, o.k, true, ro ? u : 1, ro ? 1 : u, kn) <= lines(o.r, o.k, false, ro ? u : 1, ro ? 1 : u, kn);
+}
 
-bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bool k_units) {
+// All of a description but its operands' orders.
+bool describe_units(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bool k_units) {
     const int  es = static_cast<int>(dtype_size(g.dtype)), u = 16 / es;
     const Idx2 am = normal(g.am, g.M), ak = normal(g.ak, g.K), bk = normal(g.bk, g.K), bn = normal(g.bn, g.N);
     for(const Idx2 &x : {am, ak, bk, bn})
@@ -123,6 +135,21 @@ bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bo
     d.stages_per_slice = (d.stages + ksplit - 1) / ksplit;
     d.ksplit           = (d.stages + d.stages_per_slice - 1) / d.stages_per_slice;
     return true;
+}
+
+} // namespace
+
+bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bool k_units) {
+    if(!describe_units(g, s, ksplit, out, k_units)) return false;
+    const int u = 16 / static_cast<int>(dtype_size(g.dtype));
+    set_order(out.d.a, out.ar, u, s.BK);
+    set_order(out.d.b, out.br, u, s.BK);
+    return true;
+}
+
+int load_bytes(const GemmDesc &g, const ShapeInfo &s) {
+    Launch l;
+    return describe_units(g, s, 1, l, false) ? l.W : 4;
 }
 
 } // namespace pipe

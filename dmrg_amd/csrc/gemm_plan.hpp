@@ -43,6 +43,8 @@ struct Launch {
 // kernel does not take it (negative strides, K chunks that differ between the operands, operand tiles spanning 2 GiB).
 // k_units: units along K only, as grouped launches take them.
 bool describe(const GemmDesc &g, const ShapeInfo &s, int ksplit, Launch &out, bool k_units = false);
+// Bytes per lane and load that describe would give g (4 where it refuses), at a fraction of its time.
+int load_bytes(const GemmDesc &g, const ShapeInfo &s);
 // Launches on the grid of l.d.
 void launch_f64(const Launch &l, Shape s, dim3 grid, hipStream_t st);
 void launch_c128(const Launch &l, Shape s, dim3 grid, hipStream_t st);
