@@ -1077,8 +1077,9 @@ NoTuneScope::NoTuneScope() : prev_(g_tls_no_tune) { g_tls_no_tune = true; }
 NoTuneScope::~NoTuneScope() { g_tls_no_tune = prev_; }
 
 // Plans of GEMMs already met on this thread, by everything but their pointers: planning and describing a GEMM takes
-// about 10 us on the host, a launch about 3. An entry is good for one state of the tuner (g_plan_state); at most
-// PLAN_CACHE_MAX entries of about 700 bytes are kept, and given back when the thread ends.
+// about 3 us on the host, as much as a launch. An entry is good for one state of the tuner (g_plan_state); at most
+// PLAN_CACHE_MAX entries of about 700 bytes are kept, and given back when the thread ends. A full cache gives up one entry at
+// random: a stream that cycles through more shapes than it holds keeps hits in proportion (none if the oldest went, or all).
 constexpr size_t PLAN_CACHE_MAX = 4096;
 struct PlanKey {
     int64_t v[32];
@@ -1193,7 +1194,13 @@ void gemm(const GemmDesc &gin, hipStream_t stream, TileCfg cfg, int ksplit) {
     }
     // Kept unless a later call may time this GEMM and decide otherwise.
     if(found || can_tune || !tunable) {
-        if(cache.size() >= PLAN_CACHE_MAX) cache.clear();
+        if(cache.size() >= PLAN_CACHE_MAX && cache.find(ck) == cache.end()) {
+            static thread_local uint32_t draw = 1;
+            size_t                       b    = (draw = draw * 1664525u + 1013904223u) % cache.bucket_count();
+            while(cache.bucket_size(b) == 0) b = (b + 1) % cache.bucket_count();
+            const PlanKey gone = cache.begin(b)->first;
+            cache.erase(gone);
+        }
         PlanEntry        e{state, false, p, {}};
         const pipe::Shape shape = shape_of(p.cfg, g.dtype);
         const bool        slices = p.ksplit <= 1 || (g.part && g.part_capacity >= static_cast<int64_t>(g.M) * g.N * g.batch * p.ksplit);
