@@ -9,8 +9,8 @@
 //
 // The GEMMs of the contractions run in the pipelined kernels of gemm_pipe.hpp. The kernel here stages tiles through
 // registers (global -> registers -> LDS, double buffered, one barrier per K step; per-element 64-bit offsets where the
-// index maps are not separable). It serves outputs of at most 16 rows, the grouped launches, the block Jacobi steps and
-// the index maps that the pipelined kernels do not take. Each wave owns a (BM/WM) x (BN/WN) sub-tile of 16x16 blocks:
+// index maps are not separable). It serves outputs of at most 16 rows that the streaming kernel (gemm_stream.hip) does not
+// take, the block Jacobi steps, and single or grouped GEMMs whose index maps the pipelined kernels do not take. Each wave owns a (BM/WM) x (BN/WN) sub-tile of 16x16 blocks:
 //   FP64: v_mfma_f64_16x16x4_f64,  FP32: v_mfma_f32_16x16x4_f32.
 // Complex products use the 3-real-product (Gauss) form, 3 MFMAs per block per k-step:
 //   P1 = sum ar br, P2 = sum ai bi, P3 = sum (ar + ai)(br + bi);  re = P1 - P2, im = P3 - P1 - P2.

@@ -83,7 +83,6 @@ __device__ __forceinline__ const char *uni(const char *p) {
 }
 
 // RO: units run along the non-K index. W: bytes per lane and load (16; 4 where a unit is not contiguous in memory).
-// RO: units run along the non-K index. W: bytes per lane and load (16; 4 where a unit is not contiguous in memory).
 template <typename E, int RT, int BK, bool RO, int W, int NW>
 struct Loader {
     static constexpr int ES    = static_cast<int>(sizeof(E));

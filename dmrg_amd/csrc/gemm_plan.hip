@@ -2,33 +2,12 @@
 // the order in which a load's lanes walk memory.
 #include "gemm_plan.hpp"
 
-#include <algorithm>
-
 namespace dmrg {
 namespace pipe {
 namespace {
 
-constexpr uint32_t PLAIN = 0x7fffffffu;
-
-// The same map over an extent, with a chunk only where it is one.
-Idx2 normal(Idx2 x, int64_t ext) {
-    if(x.c == 1) x = Idx2{x.s1, 0, PLAIN};
-    if(ext <= static_cast<int64_t>(x.c) || x.s1 == x.s0 * static_cast<int64_t>(x.c)) x = Idx2{x.s0, 0, PLAIN};
-    return x;
-}
 bool is_plain(const Idx2 &x) { return x.c == PLAIN; }
 Idx2 scaled(Idx2 x, int64_t f) { return Idx2{x.s0 * f, x.s1 * f, x.c}; }
-// umulhi(i, mul) >> sh = i / c for i < 2^31.
-void magic(uint32_t c, uint32_t &mul, uint32_t &sh) {
-    uint32_t l = 0;
-    while((uint64_t(1) << l) < c) ++l;
-    mul = static_cast<uint32_t>(((uint64_t(1) << (31 + l)) + c - 1) / c);
-    sh  = l - 1;
-}
-int64_t span(const Idx2 &x, int64_t ext) {
-    if(ext <= 0) return 0;
-    return std::min<int64_t>(x.c - 1, ext - 1) * x.s0 + (ext - 1) / x.c * x.s1;
-}
 bool separable(const Idx2 &x, uint32_t ext) { return is_plain(x) || x.c % ext == 0 || ext % x.c == 0; }
 // Whether u consecutive indices are contiguous from every multiple of u on (element strides).
 bool unit_run(const Idx2 &x, int64_t ext, int u) { return u == 1 || (x.s0 == 1 && ext % u == 0 && (is_plain(x) || x.c % u == 0)); }

@@ -2,11 +2,35 @@
 #pragma once
 #include "gemm_pipe.hpp"
 
+#include <algorithm>
+
 namespace dmrg {
 namespace pipe {
 
-// Tile shapes per element type. Stages hold 8 to 16 KiB per operand tile, so that two workgroups (two wavefronts per
-// SIMD) fit a CU's 160 KiB of LDS; BK is at least two K positions of an MFMA fragment unit.
+constexpr uint32_t PLAIN = 0x7fffffffu;
+
+// The same map over an extent, with a chunk only where it is one.
+inline Idx2 normal(Idx2 x, int64_t ext) {
+    if(x.c == 1) x = Idx2{x.s1, 0, PLAIN};
+    if(ext <= static_cast<int64_t>(x.c) || x.s1 == x.s0 * static_cast<int64_t>(x.c)) x = Idx2{x.s0, 0, PLAIN};
+    return x;
+}
+// umulhi(i, mul) >> sh = i / c for i < 2^31 and c > 1 (Granlund and Montgomery, Division by invariant integers using
+// multiplication, 1994).
+inline void magic(uint32_t c, uint32_t &mul, uint32_t &sh) {
+    uint32_t l = 0;
+    while((uint64_t(1) << l) < c) ++l;
+    mul = static_cast<uint32_t>(((uint64_t(1) << (31 + l)) + c - 1) / c);
+    sh  = l - 1;
+}
+// The largest offset of a map with non-negative strides over an extent.
+inline int64_t span(const Idx2 &x, int64_t ext) {
+    if(ext <= 0) return 0;
+    return std::min<int64_t>(x.c - 1, ext - 1) * x.s0 + (ext - 1) / x.c * x.s1;
+}
+
+// Tile shapes per element type. Stages hold 4 KiB (32 rows) to 16 KiB per operand tile, so that two workgroups (two
+// wavefronts per SIMD) or more fit a CU's 160 KiB of LDS; BK is at least two K positions of an MFMA fragment unit.
 enum Shape { S128x64 = 0, S64x64 = 1, S64x32 = 2, S32x32 = 3, N_SHAPES = 4 };
 struct ShapeInfo {
     int BM, BN, BK, NS, TM, TN, resident; // resident: workgroups a CU holds; BM = 0: no such shape for the type

@@ -11,14 +11,14 @@
 // chi = 512, D = 5 (10x10 on 262144 columns) complex FP64 21.3 -> 16.9 (4.97 TB/s, the rate of a large copy), FP32 18.2 -> 11.8;
 // 173x211 complex 9.0 -> 5.9; D = 8, 8 vectors of 120x88 real 12.5 -> 7.4; chi = 24, D = 3 real 5.8 -> 3.4; D = 25 (50x50 on 32964
 // columns) real 25.2 -> 16.2.
-#include "gemm_pipe.hpp"
+#include "gemm_plan.hpp"
 #include "gemm_stream.hpp"
-
-#include <algorithm>
 
 namespace dmrg {
 namespace stream {
-constexpr uint32_t PLAIN = 0x7fffffffu;
+using pipe::magic;
+using pipe::normal;
+using pipe::span;
 
 // MFMA steps over K, at least two (the divisions by multiplication below have no divisor 1).
 __host__ __device__ inline int ksteps(int K) { return K <= 8 ? 2 : (K + 3) / 4; }
@@ -149,19 +149,6 @@ __global__ __launch_bounds__(256) void grouped_kernel(const Desc *descs, const i
     const Desc g = descs[i];
     body<R, CPLX, KST>(g, blockIdx.x - start[i], 0, lds);
 }
-
-Idx2 normal(Idx2 x, int64_t ext) {
-    if(x.c == 1) x = Idx2{x.s1, 0, PLAIN};
-    if(ext <= static_cast<int64_t>(x.c) || x.s1 == x.s0 * static_cast<int64_t>(x.c)) x = Idx2{x.s0, 0, PLAIN};
-    return x;
-}
-void magic(uint32_t c, uint32_t &mul, uint32_t &sh) {
-    uint32_t l = 0;
-    while((uint64_t(1) << l) < c) ++l;
-    mul = static_cast<uint32_t>(((uint64_t(1) << (31 + l)) + c - 1) / c);
-    sh  = l - 1;
-}
-int64_t span(const Idx2 &x, int64_t ext) { return std::min<int64_t>(x.c - 1, ext - 1) * x.s0 + (ext - 1) / x.c * x.s1; }
 
 template <typename R, bool CPLX>
 void run(const Desc &d, dim3 grid, size_t lds, hipStream_t s) {

@@ -5,8 +5,8 @@
 //
 // Each sweep runs the n(n-1)/2 pairs in n-1 rounds of disjoint pairs (circle method). When W and V fit in
 // LDS, one workgroup runs every sweep with both matrices resident and a barrier between rounds (up to 128 x 64 the whole
-// SVD is that one launch). Mid-size problems launch one kernel per round with one workgroup (1 to 4 wavefronts, by column length) per pair; large
-// ones pair blocks of 16 columns instead (block one-sided Jacobi, three launches per round of block pairs). The
+// SVD is that one launch). Others of up to 32 columns launch one kernel per round with one workgroup (1 to 4 wavefronts, by
+// column length) per pair; larger ones pair blocks of 16 columns instead (block one-sided Jacobi, three launches per round of block pairs). The
 // only host round trip per sweep reads whether any rotation was applied.
 #include "svd.hpp"
 
@@ -482,24 +482,17 @@ void launch_resident(int m, int n, int tr, const T *A, double tol, int max_sweep
     DMRG_HIP_CHECK(hipGetLastError());
 }
 
-template <int G>
-__device__ inline double group_sum(double v) {
-#pragma unroll
-    for(int off = G / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, G);
-    return v;
-}
-
 // Whole Jacobi iteration in one workgroup with W (m x n) and V (n x n) resident in LDS, for small problems
-// where a kernel launch per round would dominate. A group of G lanes handles one pair; the groups take the
+// where a kernel launch per round would dominate. A wavefront handles one pair; the wavefronts take the
 // pairs of a round in turn, a barrier separates the rounds, and the sweeps stop after a sweep that applied no
 // rotation (at most max_sweeps; the number of sweeps run goes to sweeps_out).
-template <typename T, int G>
+template <typename T>
 __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T *V, double tol, int max_sweeps, int *sweeps_out) {
     extern __shared__ unsigned char lds_raw[];
     T            *Ws = reinterpret_cast<T *>(lds_raw);
     T            *Vs = Ws + static_cast<int64_t>(m) * n;
     __shared__ int rotated;
-    const int     tid = threadIdx.x, lane = tid % G, grp = tid / G, ngrp = blockDim.x / G;
+    const int     tid = threadIdx.x, lane = tid & 63, grp = tid >> 6, ngrp = blockDim.x / 64;
     for(int t = tid; t < m * n; t += blockDim.x) Ws[t] = W[t];
     for(int t = tid; t < n * n; t += blockDim.x) {
         const bool d = (t % n) == (t / n);
@@ -511,7 +504,7 @@ __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T
         if(tid == 0) rotated = 0;
         __syncthreads();
         for(int r = 0; r < np - 1; ++r) {
-            // every group runs the same trip count so that the shuffles see whole groups
+            // every wavefront runs the same trip count
             for(int i0 = 0; i0 < np / 2; i0 += ngrp) {
                 const int i = i0 + grp;
                 int       p = 0, q = 0;
@@ -528,7 +521,7 @@ __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T
                 T     *wp = Ws + p * m, *wq = Ws + q * m;
                 double al = 0, be = 0, gr = 0, gi = 0;
                 if(live) {
-                    for(int k = lane; k < m; k += G) {
+                    for(int k = lane; k < m; k += 64) {
                         if constexpr(jtraits<T>::cx) {
                             const T x = wp[k], y = wq[k];
                             al += x.re * x.re + x.im * x.im;
@@ -543,10 +536,10 @@ __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T
                         }
                     }
                 }
-                al = group_sum<G>(al);
-                be = group_sum<G>(be);
-                gr = group_sum<G>(gr);
-                if constexpr(jtraits<T>::cx) gi = group_sum<G>(gi);
+                al = wave_sum(al);
+                be = wave_sum(be);
+                gr = wave_sum(gr);
+                if constexpr(jtraits<T>::cx) gi = wave_sum(gi);
                 const double g = coupling<T>(gr, gi, al, be, tol);
                 if(!live || g == 0.0) continue;
                 const double z  = (be - al) / (2.0 * g);
@@ -555,7 +548,7 @@ __global__ __launch_bounds__(1024) void jacobi_lds(int m, int n, int np, T *W, T
                 const double er = gr / g, ei = -gi / g;
                 if(lane == 0) rotated = 1;
                 auto rot = [&](T *x, T *y, int len) {
-                    for(int k = lane; k < len; k += G) {
+                    for(int k = lane; k < len; k += 64) {
                         if constexpr(jtraits<T>::cx) {
                             const T      xv = x[k], yv = y[k];
                             const double yr = yv.re * er - yv.im * ei, yi = yv.re * ei + yv.im * er;
@@ -717,9 +710,9 @@ void DeviceSvd::jacobi(int m, int n, const T *A, std::vector<double> &S) {
     if(resident) {
         int *dsweeps = reinterpret_cast<int *>(flag + 1);
         // n <= 32: at most 16 pairs a round, one wavefront each
-        DMRG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&jacobi_lds<T, 64>), hipFuncAttributeMaxDynamicSharedMemorySize,
+        DMRG_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&jacobi_lds<T>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                            static_cast<int>(JACOBI_LDS_BYTES)));
-        hipLaunchKernelGGL((jacobi_lds<T, 64>), dim3(1), dim3(1024), lds, s, mm, nn, np, W, V, tol, 60, dsweeps);
+        hipLaunchKernelGGL((jacobi_lds<T>), dim3(1), dim3(1024), lds, s, mm, nn, np, W, V, tol, 60, dsweeps);
         DMRG_HIP_CHECK(hipGetLastError());
         int hs = 0;
         DMRG_HIP_CHECK(hipMemcpyAsync(&hs, dsweeps, sizeof(int), hipMemcpyDeviceToHost, s));
