@@ -59,13 +59,15 @@ static int grid_for(int64_t n) {
 // A reduction over few workgroups folds its partial sums in its last workgroup instead of a second launch: every
 // workgroup stores its partials at device scope (past the XCD's own L2), waits for them and counts itself in; the one that
 // counts last reads all partials past the non-coherent caches and sums them in workgroup order (deterministic), then resets
-// the counter for the next use. The order: partials are atomic stores, the barrier puts them before thread 0's count, the
-// count releases at device scope and the last one acquires, so that every partial is visible to its workgroup. On the chip,
-// each wavefront waits for its own stores before the barrier (stores to memory count in vmcnt, and one past the L2 counts down
-// when it has arrived); the release then adds one L2 write-back per workgroup. Measured: nothing, solve at chi = 64
-// 5.37-5.46 ms with the release, 5.39 without; a fence in every thread instead 5.76 against 5.27.
+// the counter for the next use.
+// The order of partials and count follows from this chip's rules, not from the language: an atomic store at device scope
+// (sc1) counts in vmcnt until it has arrived past the L2; every wavefront waits for vmcnt 0 before the barrier in front of
+// its workgroup's count, and the count and the loads of the partials are at device scope too. These are the instructions of a
+// device-scope release and acquire without the write-back and the invalidation of the L2, which concern plain stores and
+// loads; nothing plain passes between the workgroups of one launch. With both (an acquire-release count), a solve at chi = 64
+// takes 5.41 ms instead of 5.28, with a fence in every thread 5.76.
 #if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
-#error "the folds' waits are written for gfx950"
+#error "the folds' order is written for gfx950"
 #endif
 // Up to 128 workgroups: every one of them counts itself in at one address, which takes about 10 ns each (n = 122880: 480
 // workgroups, update and norm 6.9 us, against 3.3 + 2.6 for the update and a fold of its own).
@@ -101,7 +103,7 @@ __device__ inline void fold_in_last_block(const double *partial, int nv, double 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the partials of this wavefront are at device scope
     __syncthreads();
     if(threadIdx.x == 0)
-        last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x * gridDim.y - 1 ? 1 : 0;
+        last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x * gridDim.y - 1 ? 1 : 0;
     __syncthreads();
     if(!last) return;
     // Thread t sums value t % nv over the row blocks b = t / nv, t / nv + per, ...; then thread v adds the per

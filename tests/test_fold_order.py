@@ -1,6 +1,7 @@
-"""The reductions that their last workgroup folds: each workgroup's count, an atomic at device scope, releases the partial sums
-that the workgroup stored and acquires the others', and each wavefront waits for its stores before the barrier in front of
-it. Read from the compiled kernels, because a missing order shows in no test that runs them."""
+"""The reductions that their last workgroup folds rest on an order that the chip gives and the language does not: partial sums
+are stored and loaded at device scope (sc1), and every wavefront waits for its stores (vmcnt 0) before the barrier in front of
+its workgroup's count. Read from the compiled kernels, because a missing wait shows in no test that runs them; other chips
+are refused."""
 import re
 import shutil
 import subprocess
@@ -19,21 +20,25 @@ def device_compile(arch, *args):
     return subprocess.run([B.HIPCC, *flags, f"--offload-arch={arch}", "--cuda-device-only", *args, str(SRC)], capture_output=True, text=True)
 
 
-def test_counts_release_and_acquire(tmp_path):
+def test_partials_are_at_device_scope_before_the_count(tmp_path):
     out = tmp_path / "vecops.s"
     r = device_compile("gfx950", "-S", "-o", str(out))
     assert r.returncode == 0, r.stderr
     ops = [line.split(";")[0].split() for line in out.read_text().splitlines()]
-    ops = [o for o in ops if o and re.match(r"(global_atomic_add|buffer_wbl2|buffer_inv|s_waitcnt|s_barrier|s_endpgm)\b", o[0])]
+    ops = [o for o in ops if o and re.match(r"(global_|flat_|s_waitcnt|s_barrier|s_endpgm)", o[0])]
     counts = [i for i, o in enumerate(ops) if o[0].startswith("global_atomic_add")]
     assert counts
     for i in counts:
-        assert ops[i - 2][0] == "buffer_wbl2" and ops[i - 1][0] == "s_waitcnt" and "vmcnt(0)" in " ".join(ops[i - 1])
-        assert ops[i + 1][0] == "s_waitcnt" and "vmcnt(0)" in " ".join(ops[i + 1]) and ops[i + 2][0] == "buffer_inv"
-        barrier = max(j for j in range(i) if ops[j][0] == "s_barrier")
-        assert any(ops[j][0] == "s_waitcnt" and "vmcnt(0)" in " ".join(ops[j]) for j in range(barrier - 2, barrier))
+        start = max((j for j in range(i) if ops[j][0] == "s_endpgm"), default=0)  # of this kernel
+        barrier = max(j for j in range(start, i) if ops[j][0] == "s_barrier")
+        assert not any(o[0].startswith("global_store") for o in ops[barrier:i])
+        stores = [j for j in range(start, barrier) if ops[j][0].startswith("global_store") and ops[j][-1] == "sc1"]
+        assert stores
+        assert any(o[0] == "s_waitcnt" and "vmcnt(0)" in " ".join(o) for o in ops[max(stores) + 1:barrier])
+        end = next(j for j in range(i, len(ops)) if ops[j][0] == "s_endpgm")
+        assert any(o[0] == "global_load_dwordx2" and o[-1] == "sc1" for o in ops[i:end])
 
 
 def test_other_targets_are_refused():
     r = device_compile("gfx942", "-fsyntax-only")
-    assert r.returncode != 0 and "written for gfx950" in r.stderr
+    assert r.returncode != 0 and "order is written for gfx950" in r.stderr
