@@ -657,8 +657,10 @@ bool expand_small(int64_t n, int m, const T *V, const T *W, int64_t ldv, const d
 // The same for problems of several workgroups, up to MD_SHORT rows: three launches (and a fold after the first two where one
 // workgroup per 256 rows is too many to fold in the last of them) instead of six (eleven). Each workgroup projects the rows
 // that it has just formed, so that the basis comes from its caches the second time; the second Gram-Schmidt pass's
-// projections are taken whether or not its test asks for them, and its norm from |t|^2 - |h|^2, h being rounding errors of
-// the first pass. Longer vectors come from HBM, where the extra projections cost more than the
+// projections are taken whether or not its test asks for them, and its norm from |t|^2 - |h|^2. That is no difference of close
+// numbers: h holds the rounding errors of the first pass, a few eps |src| with the solver's bases (orthonormal to 4e-15 after
+// 3000 steps with restarts in 64 bits, 5e-8 in 32), and a t below 100 eps |src| is dropped as a breakdown; down to that line
+// the stored vector's norm is 1 to 2.2e-16 (in 32 bits to 2e-9, as with the norm taken from the vector). Longer vectors come from HBM, where the extra projections cost more than the
 // launches. n = 8192, 14 columns: 22 us of kernels either way, but 5.4 ms a solve against 6.9; n = 122880: 13.0 ms against 14.5.
 
 // partial[blockIdx.x][2 j] = this workgroup's rows of conj(V[:, j]) x.
@@ -784,7 +786,8 @@ __global__ __launch_bounds__(VT_THREADS) void expand_finish_kernel(int64_t n, in
         bsum<1>(acc, red);
         if(threadIdx.x == 0) total = acc[0];
         __syncthreads();
-        post = fmax(post - total, 0.0);
+        post -= total;
+        if(post < 0.0) post = 0.0; // NaN stays NaN
     }
     const double a = post > 0.0 ? 1.0 / sqrt(post) : 0.0; // a zero vector stays zero (breakdown tests see it)
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
