@@ -192,7 +192,7 @@ struct DgksTest {
 
 // Columns j < m are V[:, j]; column m (when with_self) is x itself, so x^H x comes out of the same pass. Workgroup
 // (b, g) takes the rows of b and the columns [CH g, CH (g + 1)) and then every CH gridDim.y-th group.
-template <typename T, int CH>
+template <typename T, int CH, bool FOLD>
 __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m, int mc, const T *V, int64_t ldv, const T *x,
                                                                const int *skip, double *partial, unsigned *counter, double *out,
                                                                int m_out, double *self_out, DgksTest dg, HostCopy hc) {
@@ -206,7 +206,8 @@ __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m,
     constexpr int     NV = 2 * CH;
     __shared__ double red[NV][VT_THREADS / 64];
     const int         lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for(int j0 = blockIdx.y * CH; j0 < mc; j0 += CH * static_cast<int>(gridDim.y)) {
+    constexpr bool    SPLIT = CH == MD_CH_SHORT; // long vectors: one workgroup takes all columns of its rows
+    for(int j0 = SPLIT ? blockIdx.y * CH : 0; j0 < mc; j0 += SPLIT ? CH * static_cast<int>(gridDim.y) : CH) {
         double acc[NV];
 #pragma unroll
         for(int c = 0; c < NV; ++c) acc[c] = 0.0;
@@ -233,12 +234,12 @@ __global__ __launch_bounds__(VT_THREADS) void multidot_partial(int64_t n, int m,
                 double t = 0;
 #pragma unroll
                 for(int w = 0; w < VT_THREADS / 64; ++w) t += red[threadIdx.x][w];
-                publish(partial + 2 * (static_cast<int64_t>(blockIdx.x) * mc + j0 + c) + (threadIdx.x & 1), t, counter != nullptr);
+                publish(partial + 2 * (static_cast<int64_t>(blockIdx.x) * mc + j0 + c) + (threadIdx.x & 1), t, FOLD);
             }
         }
         __syncthreads();
     }
-    if(counter) fold_in_last_block(partial, 2 * mc, out, m_out, self_out, counter, hc);
+    if constexpr(FOLD) fold_in_last_block(partial, 2 * mc, out, m_out, self_out, counter, hc);
 }
 
 static int md_grid(int64_t n) {
@@ -280,13 +281,17 @@ static void multidot_x_impl(int64_t n, int m, const T *V, int64_t ldv, const T *
         const int want   = static_cast<int>(std::max<int64_t>(1, (n + VT_THREADS - 1) / VT_THREADS));
         const bool in_last = want <= 2 * most && fused(static_cast<int64_t>(std::min(want, most)) * groups, 2 * mc);
         const int  rows    = in_last ? std::min(want, most) : std::min(want, 256);
-        hipLaunchKernelGGL((multidot_partial<T, MD_CH_SHORT>), dim3(rows, groups), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch,
-                           in_last ? scratch_counter(scratch) : nullptr, d_out, d_self ? m : -1, d_self, dg, hc);
-        if(!in_last)
+        if(in_last) {
+            hipLaunchKernelGGL((multidot_partial<T, MD_CH_SHORT, true>), dim3(rows, groups), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch,
+                               scratch_counter(scratch), d_out, d_self ? m : -1, d_self, dg, hc);
+        } else {
+            hipLaunchKernelGGL((multidot_partial<T, MD_CH_SHORT, false>), dim3(rows, groups), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch,
+                               nullptr, nullptr, -1, nullptr, dg, HostCopy{});
             hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, rows, mc, scratch, d_out, d_self ? m : -1, d_self, fskip, hc);
+        }
     } else {
         const int g = md_grid(n);
-        hipLaunchKernelGGL((multidot_partial<T, MD_CH>), dim3(g), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch, nullptr,
+        hipLaunchKernelGGL((multidot_partial<T, MD_CH, false>), dim3(g), dim3(VT_THREADS), 0, s, n, m, mc, V, ldv, x, skip, scratch, nullptr,
                            nullptr, -1, nullptr, dg, HostCopy{});
         hipLaunchKernelGGL(fold_columns, dim3(mc), dim3(VT_THREADS), 0, s, g, mc, scratch, d_out, d_self ? m : -1, d_self, fskip, hc);
     }
@@ -328,23 +333,30 @@ void multidot_dgks(int64_t n, int m, const T *V, int64_t ldv, const T *x, double
 }
 
 // ------------------------------------------------------------------------------------------- gemv
-// use(j, load(j)) for j < m in order, with eight loads in flight: one at a time, a row of a basis of 13 waits for 13
-// memory latencies (n = 8192: update 8 -> 4.0 us, Ritz vector and residual 10 -> 6.8 us).
-template <typename T, typename L, typename F>
-__device__ __forceinline__ void columns(int m, L &&load, F &&use) {
-    constexpr int UN = 8;
-    for(int j0 = 0; j0 < m; j0 += UN) {
-        T v[UN];
+// use(j, load(j)) for j < m in order, in groups of UN loads in flight, then of half as many, and so on. Where two bases are
+// read, or one that other CUs have just written, a row waits for its columns' latencies one after another otherwise (a solve of
+// four pairs at n = 8192 34.2 -> 33.5 ms, Ritz vector and residual of n = 32768, 13 columns 7.8 -> 7.65 us); a plain update and
+// long vectors, bound by bandwidth, are faster one by one with all wavefronts resident (complex n = 524288: update of 8
+// columns 14.0 us against 14.6, Ritz vector and residual of 8 27.9 against 28.7, FP64 n = 2097152 of 13 91.6 against 106).
+template <typename T, int UN, typename L, typename F>
+__device__ __forceinline__ void columns(int m, L &&load, F &&use, int j0 = 0) {
+    if constexpr(UN == 1) {
+        for(int j = j0; j < m; ++j) use(j, load(j));
+    } else {
+        for(; j0 + UN <= m; j0 += UN) {
+            T v[UN];
 #pragma unroll
-        for(int u = 0; u < UN; ++u) v[u] = load(min(j0 + u, m - 1));
+            for(int u = 0; u < UN; ++u) v[u] = load(j0 + u);
 #pragma unroll
-        for(int u = 0; u < UN; ++u)
-            if(j0 + u < m) use(j0 + u, v[u]);
+            for(int u = 0; u < UN; ++u) use(j0 + u, v[u]);
+        }
+        columns<T, UN / 2>(m, load, use, j0);
     }
 }
+constexpr int COL_UN = 8;
 
 // Row i of x = V y and r = W y - theta x.
-template <typename T>
+template <typename T, int UN = COL_UN>
 __device__ __forceinline__ void ritz_row(int64_t i, int m, const T *V, const T *W, int64_t ldv, const double *y, double theta, double &xr,
                                          double &xi, double &rr, double &ri) {
     double wr = 0, wi = 0;
@@ -352,24 +364,28 @@ __device__ __forceinline__ void ritz_row(int64_t i, int m, const T *V, const T *
         T v, w;
     };
     xr = xi = 0;
-    columns<VW>(m, [&](int j) { return VW{V[i + j * ldv], W[i + j * ldv]}; },
-                [&](int j, const VW &e) {
-                    double vr, vi, ur, ui;
-                    ld(e.v, vr, vi);
-                    ld(e.w, ur, ui);
-                    const double yr = y[2 * j], yi = y[2 * j + 1];
-                    xr += vr * yr - vi * yi;
-                    xi += vr * yi + vi * yr;
-                    wr += ur * yr - ui * yi;
-                    wi += ur * yi + ui * yr;
-                });
+    auto add = [&](int j, const T &v, const T &w) {
+        double vr, vi, ur, ui;
+        ld(v, vr, vi);
+        ld(w, ur, ui);
+        const double yr = y[2 * j], yi = y[2 * j + 1];
+        xr += vr * yr - vi * yi;
+        xi += vr * yi + vi * yr;
+        wr += ur * yr - ui * yi;
+        wi += ur * yi + ui * yr;
+    };
+    if constexpr(UN == 1) {
+        for(int j = 0; j < m; ++j) add(j, V[i + j * ldv], W[i + j * ldv]);
+    } else {
+        columns<VW, UN>(m, [&](int j) { return VW{V[i + j * ldv], W[i + j * ldv]}; }, [&](int j, const VW &e) { add(j, e.v, e.w); });
+    }
     rr = wr - theta * xr, ri = wi - theta * xi;
 }
 // Row i of V h.
-template <typename T>
+template <typename T, int UN = COL_UN>
 __device__ __forceinline__ void gemv_row(int64_t i, int m, const T *V, int64_t ldv, const double *h, double &ar, double &ai) {
     ar = ai = 0;
-    columns<T>(m, [&](int j) { return V[i + j * ldv]; },
+    columns<T, UN>(m, [&](int j) { return V[i + j * ldv]; },
                [&](int j, const T &v) {
                    double vr, vi;
                    ld(v, vr, vi);
@@ -386,7 +402,7 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_kernel(int64_t n, int 
     __syncthreads();
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
         double ar, ai;
-        gemv_row<T>(i, m, V, ldv, hs, ar, ai);
+        gemv_row<T, 1>(i, m, V, ldv, hs, ar, ai);
         double xr = 0, xi = 0;
         if(beta != 0.0) ld(x[i], xr, xi);
         x[i] = mk<T>(beta * xr + alpha * ar, beta * xi + alpha * ai);
@@ -394,7 +410,7 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_kernel(int64_t n, int 
 }
 
 // y = beta x + alpha V h (x may alias y) and per-block partials of |y|^2.
-template <typename T>
+template <typename T, bool FOLD>
 __global__ __launch_bounds__(VT_THREADS) void gemv_update_norm_kernel(int64_t n, int m, const T *V, int64_t ldv, const double *h,
                                                                       double alpha, double beta, const T *x, T *y,
                                                                       const int *skip, double *partial, unsigned *counter,
@@ -407,7 +423,7 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_norm_kernel(int64_t n,
     double acc[2] = {0.0, 0.0};
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
         double ar, ai;
-        gemv_row<T>(i, m, V, ldv, hs, ar, ai);
+        gemv_row<T, 1>(i, m, V, ldv, hs, ar, ai);
         double xr = 0, xi = 0;
         if(beta != 0.0) ld(x[i], xr, xi);
         const T yv = mk<T>(beta * xr + alpha * ar, beta * xi + alpha * ai);
@@ -418,10 +434,10 @@ __global__ __launch_bounds__(VT_THREADS) void gemv_update_norm_kernel(int64_t n,
     }
     bsum<2>(acc, red);
     if(threadIdx.x == 0) {
-        publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
-        publish(partial + 2 * blockIdx.x + 1, 0.0, counter != nullptr);
+        publish(partial + 2 * blockIdx.x, acc[0], FOLD);
+        publish(partial + 2 * blockIdx.x + 1, 0.0, FOLD);
     }
-    if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
+    if constexpr(FOLD) fold_in_last_block(partial, 2, out, -1, nullptr, counter);
 }
 
 static int ew_grid(int64_t n) { return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(8192, (n + VT_THREADS - 1) / VT_THREADS))); }
@@ -439,10 +455,10 @@ void gemv_update_norm(int64_t n, int m, const T *V, int64_t ldv, const double *d
     DMRG_REQUIRE(m <= VEC_MAX_M, DMRG_ERR_ARG, "gemv: too many columns");
     const int g = grid_for(n);
     if(fused(g, 2)) {
-        hipLaunchKernelGGL(gemv_update_norm_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, alpha, beta, x, y, skip, scratch,
+        hipLaunchKernelGGL((gemv_update_norm_kernel<T, true>), dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, alpha, beta, x, y, skip, scratch,
                            scratch_counter(scratch), d_nrm2);
     } else {
-        hipLaunchKernelGGL(gemv_update_norm_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, alpha, beta, x, y, skip, scratch,
+        hipLaunchKernelGGL((gemv_update_norm_kernel<T, false>), dim3(g), dim3(VT_THREADS), 0, s, n, m, V, ldv, d_h, alpha, beta, x, y, skip, scratch,
                            nullptr, nullptr);
         hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_nrm2, -1, nullptr, skip, HostCopy{});
     }
@@ -450,13 +466,14 @@ void gemv_update_norm(int64_t n, int m, const T *V, int64_t ldv, const double *d
 }
 
 // ------------------------------------------------------------------------------------------- Ritz vector + residual
-// The coefficients come with the launch (up to RITZ_ARGS of them) or from device memory (y).
+// The coefficients come with the launch (up to RITZ_ARGS of them) or from device memory (y). With one column at a time, the
+// compiler is held to eight wavefronts a SIMD: left alone it unrolls into 86 registers and five.
 constexpr int RITZ_ARGS = 32;
 struct RitzCoef {
     double y[2 * RITZ_ARGS];
 };
-template <typename T>
-__global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *y,
+template <typename T, int UN, bool FOLD>
+__global__ __launch_bounds__(VT_THREADS, UN == 1 ? 8 : 4) void ritz_kernel(int64_t n, int m, const T *V, const T *W, int64_t ldv, const double *y,
                                                           const RitzCoef c, double theta, T *x, T *r, double *partial, unsigned *counter,
                                                           double *out, HostCopy hc) {
     __shared__ double ys[2 * VEC_MAX_M];
@@ -470,7 +487,7 @@ __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, cons
     double acc[2] = {0.0, 0.0};
     for(int64_t i = blockIdx.x * static_cast<int64_t>(VT_THREADS) + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * VT_THREADS) {
         double xr, xi, rr, ri;
-        ritz_row<T>(i, m, V, W, ldv, ys, theta, xr, xi, rr, ri);
+        ritz_row<T, UN>(i, m, V, W, ldv, ys, theta, xr, xi, rr, ri);
         x[i] = mk<T>(xr, xi);
         r[i] = mk<T>(rr, ri);
         acc[0] += rr * rr + ri * ri;
@@ -478,10 +495,10 @@ __global__ __launch_bounds__(VT_THREADS) void ritz_kernel(int64_t n, int m, cons
     }
     bsum<2>(acc, red);
     if(threadIdx.x == 0) {
-        publish(partial + 2 * blockIdx.x, acc[0], counter != nullptr);
-        publish(partial + 2 * blockIdx.x + 1, acc[1], counter != nullptr);
+        publish(partial + 2 * blockIdx.x, acc[0], FOLD);
+        publish(partial + 2 * blockIdx.x + 1, acc[1], FOLD);
     }
-    if(counter) fold_in_last_block(partial, 2, out, -1, nullptr, counter, hc);
+    if constexpr(FOLD) fold_in_last_block(partial, 2, out, -1, nullptr, counter, hc);
 }
 
 template <typename T>
@@ -492,10 +509,11 @@ static void ritz_launch(int64_t n, int m, const T *V, const T *W, int64_t ld, co
     DMRG_REQUIRE(m <= VEC_MAX_M, DMRG_ERR_ARG, "ritz: too many columns");
     const int g = grid_for(n);
     if(fused(g, 2)) {
-        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch,
+        hipLaunchKernelGGL((ritz_kernel<T, COL_UN, true>), dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch,
                            scratch_counter(scratch), d_out, hc);
     } else {
-        hipLaunchKernelGGL(ritz_kernel<T>, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch, nullptr, nullptr, hc);
+        const auto kernel = n <= MD_SHORT ? ritz_kernel<T, COL_UN, false> : ritz_kernel<T, 1, false>;
+        hipLaunchKernelGGL(kernel, dim3(g), dim3(VT_THREADS), 0, s, n, m, V, W, ld, d_y, c, theta, x, r, scratch, nullptr, nullptr, HostCopy{});
         hipLaunchKernelGGL(fold_columns, dim3(1), dim3(VT_THREADS), 0, s, g, 1, scratch, d_out, -1, nullptr, nullptr, hc);
     }
     DMRG_HIP_CHECK(hipGetLastError());
