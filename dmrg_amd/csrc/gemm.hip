@@ -547,7 +547,9 @@ static pipe::Shape shape_of(TileCfg c, dmrg_dtype t) {
 // than its own chain of barrier, LDS read and MFMA (about 170 clocks beyond its MFMAs), and all of them together no faster
 // than their loads, about 17 clocks each. Real stages are too short for workgroups to hide that chain of one another (32x32
 // FP64: 0.165 us a stage with one workgroup on a CU, 0.33 with two; counted so, FP64 300x280 at D = 5 takes 39.1 us instead
-// of 41.2); complex ones hide it (counted alike, 173x211 would take 42.9 us instead of 41.5).
+// of 41.2); complex ones hide it (counted alike, 173x211 would take 42.9 us instead of 41.5). Over 360 legs 1 and 3 of random
+// operators (bonds 12 to 840, d 2 and 4, D 3 to 8; 78 to 104 of each type) the cheapest plan takes 2.8 % longer than the best
+// of 13 forced ones in the geometric mean (2.1 % complex FP64, 3.9 % complex FP32), 94 % are within 10 %, the worst 24 %.
 static double pipe_cost_us(const GemmDesc &g, pipe::Shape s, int ks, int W) {
     const pipe::ShapeInfo i = pipe::shape_info(g.dtype, s);
     const bool   cplx = dtype_is_complex(g.dtype), sp = dtype_is_single(g.dtype);
@@ -589,7 +591,9 @@ static LaunchPlan heuristic_plan(const GemmDesc &g) {
     // The streaming kernel where the columns dominate: below 8 columns per row the tiles' reuse of B is worth more. Past 256
     // fragments, laying A out in LDS takes 2 to 7 us, which real GEMMs win back from three 32x32 tiles per CU on and complex
     // ones (four products against the tiles' three) hardly ever: K = M = 50, N = 960 complex 16.1 us, tiles 6.3; FP64 8.9
-    // against 6.0, at N = 32964 16 against 26.
+    // against 6.0, at N = 32964 16 against 26. Over K = M of 10 to 64 and 576 to 65536 columns (70 sizes of each type) the
+    // choice takes 0.1 % longer than the best of streaming, 32x32 and 64x64 tiles in the geometric mean, 96 % are within
+    // 10 %, the worst 18 % (FP32, K = M = 64; complex FP32, K = M = 18).
     if(stream::takes(g) && (g.M <= 16 || g.N >= 8 * g.M)) {
         const int64_t fragments = static_cast<int64_t>((g.M + 15) / 16) * ((g.K + 3) / 4) * 64;
         const int64_t tiles     = static_cast<int64_t>((g.M + 31) / 32) * ((g.N + 31) / 32) * g.batch;

@@ -8,18 +8,19 @@
 // loop over K has none but the complex sums: loads take no address arithmetic (a uniform base moves from stage to stage),
 // no masks (only the last stage of a K chunk is masked) and no register copies on the way to LDS, and conjugation is a sign
 // in those sums and the epilogue. Loads and LDS reads are spread between the MFMAs one by one: issued together, all
-// wavefronts wait for the same queue with their matrix cores idle (chi = 512 leg 3: 146 us together, 124 us spread).
+// wavefronts wait for the same queue with their matrix cores idle (chi = 512 leg 3 of an earlier form: 146 us together, 124 us spread).
 //
 // The unit of all traffic is 16 bytes: U = 16 / sizeof(element) elements that are consecutive along the operand's
 // non-K index (R orientation) or along K (K orientation). A stage holds an operand tile as blocks of 16 units of the
 // non-K index; a block is stored k-major or r-major, whichever lets the 64 lanes of a load walk memory in order (the
 // choice only changes addresses). An MFMA fragment is one ds_read_b128 per lane; a 16-lane group always covers 256
-// contiguous or XOR-spread bytes, so reads are free of bank conflicts in both orders (SQ_LDS_BANK_CONFLICT is 0).
+// contiguous or XOR-spread bytes, so reads are free of bank conflicts in both orders.
 //
 // Measured (MI355X, microseconds, register-staged kernels -> here): complex FP64 chi = 512, D = 5 leg 1 (1024x2560x512)
-// 153 -> 141, leg 3 (1024x512x2560) 148 -> 124; d = 4, D = 8 leg 3 (2048x512x4096) 448 -> 364 (94 TFLOP/s, of 98 that the
-// three-product form reaches at the measured MFMA rate); real FP64 2048x1024x5120 380 -> 301 (71 TFLOP/s); complex FP32
-// leg 1 92 -> 77, leg 3 80 -> 70; real FP32 640x301x1505 47 -> 15.
+// 153 -> 123, leg 3 (1024x512x2560) 148 -> 118, complex FP32 leg 1 92 -> 68, leg 3 80 -> 65 (kernel traces of 200 matvecs;
+// the first twenty launches after an idle spell take 15 to 20 % longer); complex 4096x4096x4096 97 TFLOP/s, of 98 that the
+// three-product form reaches at the measured MFMA rate; real FP64 2048x1024x5120 380 -> 301 (71 TFLOP/s); real FP32
+// 640x301x1505 47 -> 15. No LDS bank conflict is counted on these legs.
 #pragma once
 #include "common.hpp"
 

@@ -8,7 +8,8 @@
 // accuracy in single precision and vector instructions.
 //
 // Measured (MI355X, us; before: 16x128 or 64x64 tiles, or one column per thread): 
-// chi = 512, D = 5 (10x10 on 262144 columns) complex FP64 21.3 -> 16.9 (4.97 TB/s, the rate of a large copy), FP32 18.2 -> 11.8;
+// chi = 512, D = 5 (10x10 on 262144 columns) complex FP64 21.3 -> 16.9, FP32 18.2 -> 11.8 (among 200 matvecs in a row 16.0,
+// 5.2 TB/s, the rate of a large copy, and 11.0);
 // 173x211 complex 9.0 -> 5.9; D = 8, 8 vectors of 120x88 real 12.5 -> 7.4; chi = 24, D = 3 real 5.8 -> 3.4; D = 25 (50x50 on 32964
 // columns) real 25.2 -> 16.2.
 #include "gemm_plan.hpp"

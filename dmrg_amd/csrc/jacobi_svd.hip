@@ -325,8 +325,8 @@ __device__ inline double row_sum(double v) {
 // rotation; n <= 64 makes at most 32 pairs, so that every row has one pair a round and a barrier ends the round. A round is
 // one serial chain (LDS read, three sums, the rotation's angle, LDS write, barrier), which is what bounds it: hence the
 // sums without LDS and an angle of two dependent roots instead of five roots and quotients. Whole SVDs of a graded
-// spectrum: FP64 64x64 1.49 ms against 5.0 in rounds of block pairs with three launches each, complex 2.55 against 6.1;
-// FP64 32x32 0.30 ms against 1.19 with sums through LDS and the rest in launches of its own.
+// spectrum: FP64 64x64 1.39 ms against 5.4 in rounds of block pairs with three launches each, complex 2.65 against 7.0;
+// FP64 32x32 0.31 ms against 1.20 with sums through LDS and the rest in launches of its own.
 template <typename T, int E, int EV>
 __global__ __launch_bounds__(512) void jacobi_resident(int m, int n, int tr, const T *A, double tol, int max_sweeps, T *U, T *Vt, double *S) {
     constexpr bool cx = jtraits<T>::cx;
